@@ -21,6 +21,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "dstm.h"
 #include "fft_lds.h"
 #include "tune.h"
 #include "vpmx_ctx.h"
@@ -1302,6 +1303,8 @@ void free_fft_plans(Ctx *c) {
     c->sinr_cache.clear();
     for (auto &kv : c->sinl_cache) (void)hipFree(kv.second);
     c->sinl_cache.clear();
+    for (auto &kv : c->sinf_cache) (void)hipFree(kv.second);
+    c->sinf_cache.clear();
 }
 
 // Eigenvalues 4 sin^2(pi k / (2(m+1))) / h^2 of the 1-D Dirichlet second difference,
@@ -2484,11 +2487,17 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     if (form == SOLVE_CTX) form = c->precision == 1 ? SOLVE_FP32 : SOLVE_FP64;
     const bool wave32 = wave_class(ax[0], true) && wave_class(ax[1], true) && wave_class(ax[2], true);
     const bool wave64 = wave_class(ax[0], false) && wave_class(ax[1], false) && wave_class(ax[2], false);
-    const bool inv64 = form == SOLVE_INV64 && wave32 && wave64 && c->dst_kernel == 4;
-    const bool f32 = (form == SOLVE_FP32 && wave32) || inv64;
+    // small grids in every form: FP64 products, whole planes per work-group (three launches)
+    const bool planes = c->dst_kernel == 4 && dstm_plane_fits(c, m);
+    const bool inv64 = !planes && form == SOLVE_INV64 && wave32 && wave64 && c->dst_kernel == 4;
+    const bool f32 = !planes && ((form == SOLVE_FP32 && wave32) || inv64);
+    // a pass whose lines are short enough: products with the sine matrix (k_dstm.hip)
+    auto mm = [&](int d, bool in32) { return c->dst_kernel == 4 && dstm_line_fits(m[d], in32); };
     if (inv64) reuse = 0;  // (the fine solves' reuse keeps FP32 arrays)
+    // the kept transforms are worth their corrections (six launches) on large grids only
+    if ((int64_t)wn[0] * wn[1] * wn[2] < SPECTRAL_MIN_NODES) reuse = 0;
     // one-wave kernels on every axis: rows of the work array padded to 128 bytes
-    const bool wave_all = f32 || (c->dst_kernel == 4 && wave_class(ax[0], false) && wave_class(ax[1], false) &&
+    const bool wave_all = f32 || planes || (c->dst_kernel == 4 && wave_class(ax[0], false) && wave_class(ax[1], false) &&
                                   wave_class(ax[2], false));
     if (wave_all) {
         const int q = f32 ? 32 : 16;
@@ -2500,7 +2509,12 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     a.w = a.wo = w;
     const int key[6] = {m[0], m[1], m[2], a.px, ncomp, f32 ? 1 : 0};
     const size_t wbytes = (f32 ? sizeof(float) : sizeof(double)) * (size_t)a.wcs * ncomp;
-    if (reuse == 2 && bc && std::equal(key, key + 6, c->save_key)) {
+    const DmSolve ds{{m[0], m[1], m[2]}, a.px, a.wcs, ncomp, f32};
+    const bool timed = a.my == c->dst_timed_m;
+    if (planes) {
+        VPMX_TRY(dstm_plane_fwd(c, ds, rhs, bc, a.ih2, w));
+        c->save_key[5] = -1;
+    } else if (reuse == 2 && bc && std::equal(key, key + 6, c->save_key)) {
         // the kept x/y forward transforms of the RHS (still in the work array), less those of
         // the folded Dirichlet terms
         VPMX_TRY(fold_correct(c, a, ncomp, f32, *bc));
@@ -2508,10 +2522,12 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     } else {
         // x forward (with boundary folding)
         a.nlines = (int64_t)m[1] * m[2];
-        VPMX_TRY(run_pass<DST_XF>(c, a, ncomp, ax[0], f32));
+        if (mm(0, f32)) VPMX_TRY(dstm_x_fwd(c, ds, rhs, bc, a.ih2, w));
+        else VPMX_TRY(run_pass<DST_XF>(c, a, ncomp, ax[0], f32));
         // y forward
         a.nlines = (int64_t)a.px * m[2];
-        VPMX_TRY(run_pass<DST_Y>(c, a, ncomp, ax[1], f32));
+        if (mm(1, f32)) VPMX_TRY(dstm_y(c, ds, w, timed));
+        else VPMX_TRY(run_pass<DST_Y>(c, a, ncomp, ax[1], f32));
         c->save_key[5] = -1;
         // keep them: the rest of this solve runs in a second array (one-wave kernels only; the
         // correction pass takes a row per work-group)
@@ -2527,7 +2543,7 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     // faces' sums
     a.nlines = (int64_t)a.px * m[1];
     FaceBufs fb{};
-    const bool zspec = face_nd && !inv64 && (f32 || (c->dst_kernel == 4 && wave_class(ax[2], false)));
+    const bool zspec = face_nd && !inv64 && (f32 || mm(2, false) || (c->dst_kernel == 4 && wave_class(ax[2], false)));
     if (face_nd) {
         VPMX_TRY(face_bufs(c, m[0], m[1], m[2], ncomp, &fb));
         if (zspec) {
@@ -2539,8 +2555,12 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
         // FP32 forward transforms and diagonal; the inverse passes in FP64
         double *w64 = (double *)ensure(c, c->dst_work64, sizeof(double) * (size_t)a.wcs * ncomp, &st);
         if (st) return st;
-        VPMX_TRY(launch_zmix(c, a, ncomp, ax[2], w64));
+        if (mm(2, false)) VPMX_TRY(dstm_z(c, ds, a.w, w64, false, a.lam, a.norm, nullptr, nullptr, timed));
+        else VPMX_TRY(launch_zmix(c, a, ncomp, ax[2], w64));
         a.w = a.wo = w64;
+    } else if (mm(2, f32)) {
+        VPMX_TRY(dstm_z(c, ds, a.w, a.wo, f32, a.lam, a.norm, a.zsum, a.zw, timed));
+        a.w = a.wo;
     } else {
         VPMX_TRY(run_pass<DST_Z>(c, a, ncomp, ax[2], f32));
         a.w = a.wo;
@@ -2555,12 +2575,19 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
         return partial_values(c, a, ncomp, f32, *part, out);
     }
     const bool fi = f32 && !inv64;
-    // y inverse
+    // y inverse, x inverse -> output interior
     a.nlines = (int64_t)a.px * m[2];
-    VPMX_TRY(run_pass<DST_Y>(c, a, ncomp, ax[1], fi));
-    // x inverse -> output interior
-    a.nlines = (int64_t)m[1] * m[2];
-    VPMX_TRY(run_pass<DST_XI>(c, a, ncomp, ax[0], fi));
+    if (planes) {
+        VPMX_TRY(dstm_plane_inv(c, ds, a.w, out));
+    } else {
+        DmSolve di = ds;
+        di.f32 = fi;
+        if (mm(1, fi)) VPMX_TRY(dstm_y(c, di, a.w, timed));
+        else VPMX_TRY(run_pass<DST_Y>(c, a, ncomp, ax[1], fi));
+        a.nlines = (int64_t)m[1] * m[2];
+        if (mm(0, fi)) VPMX_TRY(dstm_x_inv(c, di, a.w, out));
+        else VPMX_TRY(run_pass<DST_XI>(c, a, ncomp, ax[0], fi));
+    }
     if (!bc) VPMX_TRY(zero_faces(c, wn, out, ncomp));
     return VPMX_OK;
 }

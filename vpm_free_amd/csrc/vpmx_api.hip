@@ -99,7 +99,6 @@ static void collect_times(Ctx *, const bool *) {}
 // SOL(faces) += boundary sums (ibctyp 2 point sources, 3 panels; tree form with levmax
 // levels when levmax >= 0, pmlib.f90:69 ibctyp/itree/levmax), then the Dirichlet solve of
 // the whole grid.
-constexpr int64_t FACE_SPECTRAL_MIN = 96 * 96 * 96;  // grid nodes from which the spectral derivatives pay
 static int pmesh_inf(Ctx *c, const Grid &g, GView rhs, GView sol, DBuf &s0buf, bool fine, int levmax, int ibctyp,
                      const SolvePartial *part = nullptr) {
     int st = VPMX_OK;
@@ -119,7 +118,7 @@ static int pmesh_inf(Ctx *c, const Grid &g, GView rhs, GView sol, DBuf &s0buf, b
     int64_t nb = 0;
     // SOL_0 is read only through its normal derivatives at the faces: on large grids they come
     // straight from its spectrum (no inverse y and x passes), else from the solved field
-    const bool spectral = c->face_derivs == 1 || (c->face_derivs < 0 && G >= FACE_SPECTRAL_MIN && n[0] <= 322);
+    const bool spectral = c->face_derivs == 1 || (c->face_derivs < 0 && G >= SPECTRAL_MIN_NODES && n[0] <= 322);
     if (spectral) {
         double *fd = normal_derivs_table(c, 3, n, &st);
         if (st) return st;
@@ -195,7 +194,7 @@ static int yaps_single(Ctx *c, bool *used) {
                          part.ys[1] <= nb[1] - 1 && part.zs[1] <= nb[2] - 1 && part.xs[0] < part.xs[1] &&
                          part.ys[0] < part.ys[1] && part.zs[0] < part.zs[1] && part.xs[1] == nb[0] + 1 - part.xs[0] &&
                          part.ys[1] == nb[1] + 1 - part.ys[0] && nb[0] <= 322 && P.ncoarse >= 1;
-    const bool use_part = part_ok && (c->fine_partial == 1 || (c->fine_partial < 0 && B >= FACE_SPECTRAL_MIN));
+    const bool use_part = part_ok && (c->fine_partial == 1 || (c->fine_partial < 0 && B >= SPECTRAL_MIN_NODES));
     VPMX_TRY(pmesh_inf(c, gb, rv, sv, c->sol0, true, tree ? G.ilevmax : -1, P.ibctyp, use_part ? &part : nullptr));
     mark(c, ST_FINE, 1);
     used[ST_FINE] = used[ST_BOUNDS] = true;

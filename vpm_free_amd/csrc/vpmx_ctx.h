@@ -112,6 +112,7 @@ struct Ctx : vpmx_ctx {
     std::map<std::pair<int, double>, void *> fdw_cache;  // normal-derivative weights per (m, h)
     std::map<std::pair<int, int>, void *> sinr_cache;  // sin(pi p k / (m+1)), k = 1..m, per (m, p)
     std::map<std::pair<int, int>, void *> sinl_cache;  // rows p = a s, a = 1..m/s, of the DST-I matrix, per (m, s)
+    std::map<int, void *> sinf_cache;  // operand fragments of the folded DST-I matrix, per m
     DBuf scan_tmp, red_tmp, rm_flag, rm_pos, rm_x, rm_q, rm_grid;
     DBuf tile_flag, tile_pos, tile_list;  // interpolation: cell tiles holding particles
     // projection without zeros for empty tiles: tile_flag maps the node tiles of a view of
