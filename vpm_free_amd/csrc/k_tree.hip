@@ -14,10 +14,12 @@
 // entry e is a (level, cell) node, its children follow it, and skip[e] is the first entry
 // after its subtree.  The reference's recursion visits the children of a refined cell in
 // link order, depth first — exactly this preorder — so walking the list with "refine:
-// e+1, accept: skip[e]" takes the reference's terms in the reference's order.  A wave owns
-// an 8x8 patch of target nodes and walks the list with a wave-uniform cursor (every entry
-// load is a broadcast): a lane that accepts a node waits until the cursor has passed that
-// node's subtree while lanes that refine descend.
+// e+1, accept: skip[e]" takes the reference's terms.  A wave owns a patch of target nodes and
+// walks trees with a wave-uniform cursor (every entry load is a broadcast): a lane that
+// accepts a node waits until the cursor has passed that node's subtree while lanes that refine
+// descend.  The trees are shared out over the launch (part p the trees p, p + parts, ...) and
+// the parts' sums added in their order: one wave per patch over the whole list is some 6000
+// entries one after another with two or three waves on a CU, all latency.
 //
 // The refinement test r < 10 sqrt(DS) decides which terms are taken, so r, the centroids
 // and DS are formed with the reference's operation order and no contraction: for
@@ -26,6 +28,7 @@
 #include <hip/hip_ext.h>
 
 #include <array>
+#include <cmath>
 #include <map>
 
 #include "bnodes.h"
@@ -45,7 +48,7 @@ struct TreeLink {
     int32_t nch;
 };
 
-// Target patches: wave w of the evaluation covers tile w; the tiles of face q are
+// Target patches: work-group w of the evaluation covers tile w; the tiles of face q are
 // [off[q], off[q+1]), nu[q] tiles along the face's inner target axis.
 struct TreeTiles {
     int off[7];
@@ -58,8 +61,10 @@ struct TreePlan {
     TreeTiles tiles{};
     int4 *desc = nullptr;     // per entry: base, pitch, level, kind
     int *skip = nullptr;      // per entry
-    double4 *pos = nullptr;   // per entry: centroid, refinement parameter (k_tree_entries)
-    double4 *val = nullptr;   // per entry: DS, source per component
+    double4 *line = nullptr;  // per entry: centroid, refinement parameter; sources (k_tree_entries)
+    double2 *aux = nullptr;   // per entry: DS, refinement radius
+    int nroot = 0;
+    int *root = nullptr;      // first entry of each tree, and the end of the list
 };
 
 using PlanKey = std::array<int, 4>;
@@ -157,7 +162,7 @@ int build_links(Ctx *c, const int n[3], int levmax, std::vector<std::vector<Tree
 
 // Preorder of the forest rooted at every cell of level levmax.
 int flatten(Ctx *c, const std::vector<std::vector<TreeLink>> &lv, int levmax, std::vector<int4> &desc,
-            std::vector<int> &skip) {
+            std::vector<int> &skip, std::vector<int> &root) {
     struct Frame {
         int lev, idx, next;
         size_t pos;
@@ -165,6 +170,7 @@ int flatten(Ctx *c, const std::vector<std::vector<TreeLink>> &lv, int levmax, st
     std::vector<Frame> st;
     for (int r = 0; r < (int)lv[levmax].size(); r++) {
         st.push_back({levmax, r, 0, desc.size()});
+        root.push_back((int)desc.size());
         const TreeLink &t0 = lv[levmax][r];
         desc.push_back(make_int4(t0.base, t0.pitch, levmax, t0.kind));
         skip.push_back(0);
@@ -187,31 +193,38 @@ int flatten(Ctx *c, const std::vector<std::vector<TreeLink>> &lv, int levmax, st
             st.pop_back();
         }
     }
+    root.push_back((int)desc.size());
     return VPMX_OK;
 }
 
 // Entry aggregates from the level-0 cells (build_level_nbound_3d's sums, same order:
 // rows of the group outer, cells of a row inner; area-weighted source).  pos.w encodes the
 // refinement test of the traversal:
-//   point sources (tree_calc_3d):   refine iff r < pos.w  — 10 sqrt(DS) above level 0, -1 at
-//                                   level 0 (never), +inf at dummies (always);
+//   point sources (tree_calc_3d):   refine iff r < w, w = 10 sqrt(DS) above level 0, 0 at
+//                                   level 0 (never), 1e150 at dummies (always); one 64-byte line
+//                                   per entry: pos with w^2 (1 - 1e-14) for w, val the products
+//                                   source * DS with the skip index in the bits of w; aux (DS, w);
 //   panels (tree_calc_3d_s):        refine iff r / pos.w < 10 — sqrt(DS) above level 0, NaN at
 //                                   level 0 (never), -1 at dummies of kind -1 (always), 0 at
 //                                   dummies of kind -2 (never: the reference takes them as
 //                                   cells of zero area, r / 0 = inf).
 // Dummies sit at the origin with zero area and source, as the reference's zeroed level
 // arrays leave them.
-__global__ void k_tree_entries(int64_t nent, const int4 *__restrict__ desc, int64_t nb, const double *__restrict__ cxyz,
-                               const double *__restrict__ sig, const double *__restrict__ ds, double4 *__restrict__ pos,
-                               double4 *__restrict__ val, int panels) {
+__global__ void k_tree_entries(int64_t nent, const int4 *__restrict__ desc, const int *__restrict__ skip, int64_t nb,
+                               const double *__restrict__ cxyz, const double *__restrict__ sig,
+                               const double *__restrict__ ds, double4 *__restrict__ line, double2 *__restrict__ aux,
+                               int panels) {
 #pragma clang fp contract(off)
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= nent) return;
     const int4 d = desc[e];
+    const double sk = __longlong_as_double(skip[e]);
+    double4 *pos = line + 2 * e, *val = line + 2 * e + 1;
     if (d.w < 0) {
-        const double w = panels ? (d.w == -1 ? -1.0 : 0.0) : __builtin_inf();
-        pos[e] = make_double4(0.0, 0.0, 0.0, w);
-        val[e] = make_double4(0.0, 0.0, 0.0, 0.0);
+        const double w = panels ? (d.w == -1 ? -1.0 : 0.0) : 1e300;
+        *pos = make_double4(0.0, 0.0, 0.0, w);
+        *val = make_double4(0.0, 0.0, 0.0, panels ? 0.0 : sk);
+        aux[e] = make_double2(0.0, 1e150);
         return;
     }
     const int s = 1 << d.z;
@@ -230,82 +243,136 @@ __global__ void k_tree_entries(int64_t nent, const int4 *__restrict__ desc, int6
         }
     }
     const double fl = (double)(s * s);
-    double w;
-    if (panels) w = d.z > 0 ? sqrt(sc) : __builtin_nan("");
-    else w = d.z > 0 ? 10.0 * sqrt(sc) : -1.0;
-    pos[e] = make_double4(xc / fl, yc / fl, zc / fl, w);
-    val[e] = make_double4(sc, q0 / sc, q1 / sc, q2 / sc);
+    if (panels) {
+        *pos = make_double4(xc / fl, yc / fl, zc / fl, d.z > 0 ? sqrt(sc) : __builtin_nan(""));
+        *val = make_double4(sc, q0 / sc, q1 / sc, q2 / sc);
+        return;
+    }
+    const double w = d.z > 0 ? 10.0 * sqrt(sc) : 0.0, w2 = w * w;
+    *pos = make_double4(xc / fl, yc / fl, zc / fl, w2 * (1.0 - 1e-14));
+    *val = make_double4(q0 / sc * sc, q1 / sc * sc, q2 / sc * sc, sk);
+    aux[e] = make_double2(sc, w);
 }
 
-constexpr int TR_WAVES = 4;
+constexpr int TR_WAVES = 8, TR_PARTS = 16;
 
-// One wave per 8x8 patch of target nodes.  SOL(target) += SOURCE / (4 pi).
-__global__ void __launch_bounds__(64 * TR_WAVES)
-    k_tree_eval(Grid g, TreeTiles tt, int nent, const double4 *__restrict__ pos, const double4 *__restrict__ val,
-                const int *__restrict__ skip, GView sol) {
-#pragma clang fp contract(off)
-    const int lane = threadIdx.x & 63;
-    const int w = blockIdx.x * TR_WAVES + (threadIdx.x >> 6);
-    if (w >= tt.off[6]) return;  // whole waves
-    int q = 0;
-    while (w >= tt.off[q + 1]) q++;
+// The target node (1-based) t of lane `lane` of patch w (TR_T x 8 by 8 nodes, target t in its
+// t-th 8 columns); face q, false past the face's edge.
+constexpr int TR_T = 2;
+__device__ __forceinline__ bool tree_target(const Grid &g, const TreeTiles &tt, int w, int lane, int t, int *q, int *i,
+                                            int *j, int *k) {
+    int f = 0;
+    while (w >= tt.off[f + 1]) f++;
+    *q = f;
     const int NX = g.n[0], NY = g.n[1], NZ = g.n[2];
-    const int tl = w - tt.off[q];
-    const int u = (tl % tt.nu[q]) * 8 + (lane & 7);
-    const int v = (tl / tt.nu[q]) * 8 + (lane >> 3);
-    const int hi = q & 1;
-    int i, j, k;
-    bool ok;
-    if (q < 2) {  // X faces: all (j, k)
-        i = hi ? NX : 1; j = u + 1; k = v + 1;
-        ok = u < NY && v < NZ;
-    } else if (q < 4) {  // Y faces: i = 2..NX-1, all k
-        j = hi ? NY : 1; i = u + 2; k = v + 1;
-        ok = u < NX - 2 && v < NZ;
-    } else {  // Z faces: i = 2..NX-1, j = 2..NY-1
-        k = hi ? NZ : 1; i = u + 2; j = v + 2;
-        ok = u < NX - 2 && v < NY - 2;
+    const int tl = w - tt.off[f];
+    const int u = (tl % tt.nu[f]) * 8 * TR_T + 8 * t + (lane & 7);
+    const int v = (tl / tt.nu[f]) * 8 + (lane >> 3);
+    const int hi = f & 1;
+    if (f < 2) {  // X faces: all (j, k)
+        *i = hi ? NX : 1; *j = u + 1; *k = v + 1;
+        return u < NY && v < NZ;
     }
-    const double X = g.x0[0] + (double)(i - 1) * g.h[0];
-    const double Y = g.x0[1] + (double)(j - 1) * g.h[1];
-    const double Z = g.x0[2] + (double)(k - 1) * g.h[2];
-    const double lg2 = 2.0 * log((sqrt(2.0) - 1) / (sqrt(2.0) + 1));
-    double S0 = 0.0, S1 = 0.0, S2 = 0.0;
-    int until = ok ? 0 : 0x7fffffff;  // the lane takes no term before entry `until`
-    int e = 0;
-    while (e < nent) {
-        const double4 p = pos[e];
-        const double4 a = val[e];
-        const int sk = skip[e];
-        bool refine = false;
-        if (e >= until) {
-            const double XR = p.x - X, YR = p.y - Y, ZR = p.z - Z;
-            const double r = sqrt(XR * XR + YR * YR + ZR * ZR);
-            if (r < p.w) {
-                refine = true;
-            } else {
-                if (r > 1e-05) {
-                    const double wdr = a.x / r;
-                    S0 = S0 - a.y * wdr;
-                    S1 = S1 - a.z * wdr;
-                    S2 = S2 - a.w * wdr;
-                } else {  // self term of a cell whose centroid is the node
-                    const double f = sqrt(a.x) * lg2;
-                    S0 = S0 + a.y * f;
-                    S1 = S1 + a.z * f;
-                    S2 = S2 + a.w * f;
+    if (f < 4) {  // Y faces: i = 2..NX-1, all k
+        *j = hi ? NY : 1; *i = u + 2; *k = v + 1;
+        return u < NX - 2 && v < NZ;
+    }
+    // Z faces: i = 2..NX-1, j = 2..NY-1
+    *k = hi ? NZ : 1; *i = u + 2; *j = v + 2;
+    return u < NX - 2 && v < NY - 2;
+}
+
+// SOL(target) += SOURCE / (4 pi).  The test r < w needs r itself only where r^2 and w^2 agree to
+// 1e-14; elsewhere the squares decide, and the accepted term's 1/r comes from the reciprocal
+// square root and one third-order step.  What bounds the walk is the scalar loads of the entries:
+// one 64-byte line per entry, the next one in list order fetched ahead (the list ends with one
+// line of padding), TR_T targets per lane to each line, and the eight waves of a work-group on
+// neighbouring patches of the same trees, so that they find each other's lines in the scalar
+// cache (a 129 x 129 x 41 block: 0.87 ms with the waves of a work-group on different trees).
+__global__ void __launch_bounds__(64 * TR_WAVES)
+    k_tree_eval(Grid g, TreeTiles tt, int nroot, const int *__restrict__ root, const double4 *__restrict__ line,
+                const double2 *__restrict__ aux, double *__restrict__ part) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tile = blockIdx.x * TR_WAVES + wave;
+    if (tile >= tt.off[6]) return;
+    double X[TR_T], Y[TR_T], Z[TR_T], S[TR_T][3];
+    int until[TR_T];  // target t takes no term before entry until[t]
+#pragma unroll
+    for (int t = 0; t < TR_T; t++) {
+        int q, i, j, k;
+        until[t] = tree_target(g, tt, tile, lane, t, &q, &i, &j, &k) ? 0 : 0x7fffffff;
+        X[t] = g.x0[0] + (double)(i - 1) * g.h[0];
+        Y[t] = g.x0[1] + (double)(j - 1) * g.h[1];
+        Z[t] = g.x0[2] + (double)(k - 1) * g.h[2];
+        S[t][0] = S[t][1] = S[t][2] = 0.0;
+    }
+    for (int r0 = blockIdx.y; r0 < nroot; r0 += TR_PARTS) {
+        int e = root[r0];
+        const int end = root[r0 + 1];
+        double4 p = line[2 * e], v = line[2 * e + 1];
+        while (e < end) {
+            const double4 p1 = line[2 * e + 2], v1 = line[2 * e + 3];
+            const int sk = (int)__double_as_longlong(v.w);
+            bool refine = false;
+#pragma unroll
+            for (int t = 0; t < TR_T; t++) {
+                const double XR = p.x - X[t], YR = p.y - Y[t], ZR = p.z - Z[t];
+                const double r2 = XR * XR + YR * YR + ZR * ZR;
+                const bool live = e >= until[t];
+                bool down = r2 < p.w;
+                const bool close = live && ((!down && r2 <= p.w * (1.0 + 2.1e-14)) || r2 <= 1.1e-10);
+                double y = __builtin_amdgcn_rsq(r2);
+                const double er = fma(-r2 * y, y, 1.0);
+                y = fma(y * er, fma(0.375, er, 0.5), y);
+                if (__any(close)) {  // (whole wave: the square roots stay out of the common path)
+                    const double r = sqrt(r2);
+                    const double2 x = aux[e];
+                    if (!down) down = r < x.y;
+                    if (!down && !(r > 1e-05))  // self term of a cell whose centroid is the node
+                        y = -sqrt(x.x) * (2.0 * log((sqrt(2.0) - 1) / (sqrt(2.0) + 1))) / x.x;
                 }
-                until = sk;
+                if (live && !down) {
+                    S[t][0] = fma(-v.x, y, S[t][0]);
+                    S[t][1] = fma(-v.y, y, S[t][1]);
+                    S[t][2] = fma(-v.z, y, S[t][2]);
+                    until[t] = sk;
+                }
+                refine = refine || (live && down);
             }
+            const int next = __builtin_amdgcn_readfirstlane(__any(refine) ? e + 1 : sk);
+            if (next == e + 1) {
+                p = p1;
+                v = v1;
+            } else {
+                p = line[2 * next];
+                v = line[2 * next + 1];
+            }
+            e = next;
         }
-        e = __builtin_amdgcn_readfirstlane(__any(refine) ? e + 1 : sk);
     }
-    if (!ok) return;
-    const double PI4 = 4.0 * (4.0 * atan(1.0));
+    const int64_t nt = (int64_t)tt.off[6] * 64 * TR_T;
+#pragma unroll
+    for (int t = 0; t < TR_T; t++)
+        for (int c = 0; c < 3; c++)
+            part[((int64_t)blockIdx.y * 3 + c) * nt + ((int64_t)tile * TR_T + t) * 64 + lane] = S[t][c];
+}
+
+// SOL(target) += (the parts' sums, in order) / div.
+__global__ void __launch_bounds__(256) k_tree_sum(Grid g, TreeTiles tt, int parts, const double *__restrict__ part,
+                                                  double div, GView sol) {
+#pragma clang fp contract(off)
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x, nt = (int64_t)tt.off[6] * 64 * TR_T;
+    if (e >= nt) return;
+    const int lane = (int)(e & 63), t = (int)(e >> 6) % TR_T;
+    int q, i, j, k;
+    if (!tree_target(g, tt, (int)(e / (64 * TR_T)), lane, t, &q, &i, &j, &k)) return;
     const int64_t o = sol.at(i - 1, j - 1, k - 1);
-    sol.p[o] = sol.p[o] + S0 / PI4;
-    sol.p[sol.cs + o] = sol.p[sol.cs + o] + S1 / PI4;
-    sol.p[2 * sol.cs + o] = sol.p[2 * sol.cs + o] + S2 / PI4;
+    for (int c = 0; c < 3; c++) {
+        double s = 0.0;
+        for (int p = 0; p < parts; p++) s += part[((int64_t)p * 3 + c) * nt + e];
+        sol.p[c * sol.cs + o] = sol.p[c * sol.cs + o] + s / div;
+    }
 }
 
 // tree_calc_3d_s (pmbound.f90:1346-1481) under calc_boundinf_3d_lev_s (:1255-1345):
@@ -314,81 +381,69 @@ __global__ void __launch_bounds__(64 * TR_WAVES)
 // the cell's area) times the source of the FIRST top-level cell, as the reference passes
 // nv = 1 at the top.  SOL += SOURCE.
 __global__ void __launch_bounds__(64 * TR_WAVES)
-    k_tree_eval_s(Grid g, TreeTiles tt, int nent, int levmax, const int4 *__restrict__ desc,
-                  const double4 *__restrict__ pos, const double4 *__restrict__ val, const int *__restrict__ skip,
-                  GView sol) {
+    k_tree_eval_s(Grid g, TreeTiles tt, int nroot, const int *__restrict__ root, int levmax,
+                  const int4 *__restrict__ desc, const double4 *__restrict__ line, const int *__restrict__ skip,
+                  double *__restrict__ part) {
 #pragma clang fp contract(off)
-    const int lane = threadIdx.x & 63;
-    const int w = blockIdx.x * TR_WAVES + (threadIdx.x >> 6);
-    if (w >= tt.off[6]) return;
-    int q = 0;
-    while (w >= tt.off[q + 1]) q++;
-    const int NX = g.n[0], NY = g.n[1], NZ = g.n[2];
-    const int tl = w - tt.off[q];
-    const int u = (tl % tt.nu[q]) * 8 + (lane & 7);
-    const int v = (tl / tt.nu[q]) * 8 + (lane >> 3);
-    const int hi = q & 1;
-    int i, j, k, iplane;
-    bool ok;
-    if (q < 2) {
-        i = hi ? NX : 1; j = u + 1; k = v + 1; iplane = hi ? -2 : 2;
-        ok = u < NY && v < NZ;
-    } else if (q < 4) {
-        j = hi ? NY : 1; i = u + 2; k = v + 1; iplane = hi ? -1 : 1;
-        ok = u < NX - 2 && v < NZ;
-    } else {
-        k = hi ? NZ : 1; i = u + 2; j = v + 2; iplane = hi ? -3 : 3;
-        ok = u < NX - 2 && v < NY - 2;
-    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tile = blockIdx.x * TR_WAVES + wave;
+    if (tile >= tt.off[6]) return;
+    int q, i, j, k;
+    const bool ok = tree_target(g, tt, tile, lane, blockIdx.z, &q, &i, &j, &k);
+    const int iplane = (q & 1 ? -1 : 1) * (q < 2 ? 2 : (q < 4 ? 1 : 3));
     const PanelFrame fr = panel_frame(iplane, g.h);
     const double XO[3] = {g.x0[0] + (double)(i - 1) * g.h[0], g.x0[1] + (double)(j - 1) * g.h[1],
                           g.x0[2] + (double)(k - 1) * g.h[2]};
     const double PI4 = 4.0 * (4.0 * atan(1.0));
-    const double4 first = val[0];  // the first top-level cell
+    const double4 first = line[1];  // the first top-level cell
     double S0 = 0.0, S1 = 0.0, S2 = 0.0;
     int until = ok ? 0 : 0x7fffffff;
-    int e = 0;
-    while (e < nent) {
-        const double4 p = pos[e];
-        const double4 a = val[e];
-        const int lev = desc[e].z;
-        const int sk = skip[e];
-        bool refine = false;
-        if (e >= until) {
-            const double d[3] = {XO[0] - p.x, XO[1] - p.y, XO[2] - p.z};
-            const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-            if (r / p.w < 10) {
-                refine = true;
-            } else {
-                if (lev != levmax) {
-                    const double PR = PI4 * r;
-                    S0 = S0 - a.y * a.x / PR;
-                    S1 = S1 - a.z * a.x / PR;
-                    S2 = S2 - a.w * a.x / PR;
+    for (int t = blockIdx.y; t < nroot; t += TR_PARTS) {
+        int e = root[t];
+        const int end = root[t + 1];
+        while (e < end) {
+            const double4 p = line[2 * e];
+            const double4 a = line[2 * e + 1];
+            const int lev = desc[e].z;
+            const int sk = skip[e];
+            bool refine = false;
+            if (e >= until) {
+                const double d[3] = {XO[0] - p.x, XO[1] - p.y, XO[2] - p.z};
+                const double r = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+                if (r / p.w < 10) {
+                    refine = true;
                 } else {
-                    const double FIS = fsour_a4(fr, d, a.x, PI4);
-                    S0 = S0 + first.y * FIS;
-                    S1 = S1 + first.z * FIS;
-                    S2 = S2 + first.w * FIS;
+                    if (lev != levmax) {
+                        const double PR = PI4 * r;
+                        S0 = S0 - a.y * a.x / PR;
+                        S1 = S1 - a.z * a.x / PR;
+                        S2 = S2 - a.w * a.x / PR;
+                    } else {
+                        const double FIS = fsour_a4(fr, d, a.x, PI4);
+                        S0 = S0 + first.y * FIS;
+                        S1 = S1 + first.z * FIS;
+                        S2 = S2 + first.w * FIS;
+                    }
+                    until = sk;
                 }
-                until = sk;
             }
+            e = __builtin_amdgcn_readfirstlane(__any(refine) ? e + 1 : sk);
         }
-        e = __builtin_amdgcn_readfirstlane(__any(refine) ? e + 1 : sk);
     }
-    if (!ok) return;
-    const int64_t o = sol.at(i - 1, j - 1, k - 1);
-    sol.p[o] = sol.p[o] + S0;
-    sol.p[sol.cs + o] = sol.p[sol.cs + o] + S1;
-    sol.p[2 * sol.cs + o] = sol.p[2 * sol.cs + o] + S2;
+    const int64_t nt = (int64_t)tt.off[6] * 64 * TR_T;
+    double *o = part + (int64_t)blockIdx.y * 3 * nt + ((int64_t)tile * TR_T + blockIdx.z) * 64 + lane;
+    o[0] = S0;
+    o[nt] = S1;
+    o[2 * nt] = S2;
 }
 
 void free_plan(TreePlan *p) {
     if (!p) return;
     (void)hipFree(p->desc);
     (void)hipFree(p->skip);
-    (void)hipFree(p->pos);
-    (void)hipFree(p->val);
+    (void)hipFree(p->line);
+    (void)hipFree(p->root);
+    (void)hipFree(p->aux);
     delete p;
 }
 
@@ -406,26 +461,31 @@ int get_plan(Ctx *c, const Grid &g, int levmax, int64_t nb, TreePlan **out) {
     VPMX_TRY(build_links(c, g.n, levmax, lv));
     if ((int64_t)lv[0].size() != nb) return fail(c, VPMX_ERR_STATE, "tree: level-0 cells differ from the face sources");
     std::vector<int4> desc;
-    std::vector<int> skip;
+    std::vector<int> skip, root;
     desc.reserve((size_t)(nb * 4 / 3 + 64));
     skip.reserve(desc.capacity());
-    VPMX_TRY(flatten(c, lv, levmax, desc, skip));
+    VPMX_TRY(flatten(c, lv, levmax, desc, skip, root));
     TreePlan *p = new TreePlan();
     p->nb = nb;
     p->nent = (int64_t)desc.size();
+    p->nroot = (int)root.size() - 1;
     const int NX = g.n[0], NY = g.n[1], NZ = g.n[2];
     const int U[6] = {NY, NY, NX - 2, NX - 2, NX - 2, NX - 2};
     const int V[6] = {NZ, NZ, NZ, NZ, NY - 2, NY - 2};
     p->tiles.off[0] = 0;
     for (int q = 0; q < 6; q++) {
-        p->tiles.nu[q] = (U[q] + 7) / 8;
+        p->tiles.nu[q] = (U[q] + 8 * TR_T - 1) / (8 * TR_T);
         p->tiles.off[q + 1] = p->tiles.off[q] + p->tiles.nu[q] * ((V[q] + 7) / 8);
     }
-    const size_t ne = (size_t)p->nent;
+    skip.push_back(p->nent);  // one entry of padding: the walks load ahead
+    desc.push_back(make_int4(-1, 0, 0, -1));
+    const size_t ne = (size_t)p->nent + 1;
     hipError_t e = hipMalloc((void **)&p->desc, sizeof(int4) * ne);
     if (e == hipSuccess) e = hipMalloc((void **)&p->skip, sizeof(int) * ne);
-    if (e == hipSuccess) e = hipMalloc((void **)&p->pos, sizeof(double4) * ne);
-    if (e == hipSuccess) e = hipMalloc((void **)&p->val, sizeof(double4) * ne);
+    if (e == hipSuccess) e = hipMalloc((void **)&p->line, sizeof(double4) * 2 * ne);
+    if (e == hipSuccess) e = hipMalloc((void **)&p->aux, sizeof(double2) * ne);
+    if (e == hipSuccess) e = hipMalloc((void **)&p->root, sizeof(int) * root.size());
+    if (e == hipSuccess) e = hipMemcpy(p->root, root.data(), sizeof(int) * root.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->desc, desc.data(), sizeof(int4) * ne, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->skip, skip.data(), sizeof(int) * ne, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -445,22 +505,28 @@ int boundary_sums_tree(Ctx *c, const Grid &g, int64_t nb, const double *sig, con
     TreePlan *p = nullptr;
     VPMX_TRY(get_plan(c, g, levmax, nb, &p));
     hipLaunchKernelGGL(k_tree_entries, dim3((unsigned)((p->nent + 255) / 256)), dim3(256), 0, c->stream, p->nent,
-                       p->desc, nb, cxyz, sig, ds, p->pos, p->val, panels ? 1 : 0);
+                       p->desc, p->skip, nb, cxyz, sig, ds, p->line, p->aux, panels ? 1 : 0);
     VPMX_HIP(c, hipGetLastError());
-    const unsigned blocks = (unsigned)((p->tiles.off[6] + TR_WAVES - 1) / TR_WAVES);
-    if (panels) {
-        hipLaunchKernelGGL(k_tree_eval_s, dim3(blocks), dim3(64 * TR_WAVES), 0, c->stream, g, p->tiles, (int)p->nent,
-                           levmax, p->desc, p->pos, p->val, p->skip, sol);
-        VPMX_HIP(c, hipGetLastError());
-        return VPMX_OK;
-    }
+    const int ntile = p->tiles.off[6];
+    const int64_t nt = (int64_t)ntile * 64 * TR_T;
+    int st = VPMX_OK;
+    double *part = (double *)ensure(c, c->tree_part, sizeof(double) * 3 * TR_PARTS * (size_t)nt, &st);
+    if (st) return st;
+    const unsigned blocks = (unsigned)((ntile + TR_WAVES - 1) / TR_WAVES);
     hipEvent_t e0, e1;
-    if (fine && kernel_events(c, K_BOUNDSUM, &e0, &e1))
-        hipExtLaunchKernelGGL(k_tree_eval, dim3(blocks), dim3(64 * TR_WAVES), 0, c->stream, e0, e1, 0, g, p->tiles,
-                              (int)p->nent, p->pos, p->val, p->skip, sol);
+    if (panels)
+        hipLaunchKernelGGL(k_tree_eval_s, dim3(blocks, TR_PARTS, TR_T), dim3(64 * TR_WAVES), 0, c->stream, g, p->tiles,
+                           p->nroot, p->root, levmax, p->desc, p->line, p->skip, part);
+    else if (fine && kernel_events(c, K_BOUNDSUM, &e0, &e1))
+        hipExtLaunchKernelGGL(k_tree_eval, dim3(blocks, TR_PARTS), dim3(64 * TR_WAVES), 0, c->stream, e0, e1, 0, g,
+                              p->tiles, p->nroot, p->root, p->line, p->aux, part);
     else
-        hipLaunchKernelGGL(k_tree_eval, dim3(blocks), dim3(64 * TR_WAVES), 0, c->stream, g, p->tiles, (int)p->nent,
-                           p->pos, p->val, p->skip, sol);
+        hipLaunchKernelGGL(k_tree_eval, dim3(blocks, TR_PARTS), dim3(64 * TR_WAVES), 0, c->stream, g, p->tiles, p->nroot,
+                           p->root, p->line, p->aux, part);
+    VPMX_HIP(c, hipGetLastError());
+    const double PI4 = 4.0 * (4.0 * std::atan(1.0));
+    hipLaunchKernelGGL(k_tree_sum, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, c->stream, g, p->tiles, TR_PARTS,
+                       part, panels ? 1.0 : PI4, sol);
     VPMX_HIP(c, hipGetLastError());
     return VPMX_OK;
 }

@@ -90,6 +90,7 @@ struct Ctx : vpmx_ctx {
     int bs_mode = 2;  // boundary sums (option boundsum): 2 spectral (default), 0 lattice tables, 1 direct LDS source tiles
     void *bsx[2] = {nullptr, nullptr};  // spectral boundary-sum plans: fine block, coarse grid
     void *tree = nullptr;  // tree boundary-sum plans per (grid, levels)
+    DBuf tree_part;        // the tree walk's partial sums
     int num_cu = 256;       // compute units of the device
     int64_t max_lds = 65536;  // LDS bytes a work-group may hold (device attribute)
     bool dst_reuse = true;  // second fine solve from the first one's forward transforms (option dst_reuse)
