@@ -583,18 +583,16 @@ int point_sums(Ctx *c, const Grid &g, int64_t ns, const double *cxyz, const doub
     int64_t nt = 2 * ((int64_t)NY * NZ + (int64_t)(NX - 2) * NZ + (int64_t)(NX - 2) * (NY - 2));
     if (fine && c->bs_mode == 2) {
         mark(c, ST_BOUNDS, 0);
-        hipEvent_t e0, e1;
-        const bool timed = kernel_events(c, K_BOUNDSUM, &e0, &e1);
-        if (timed) VPMX_HIP(c, hipEventRecord(e0, c->stream));
+        mark(c, ST_COUNT + K_BOUNDSUM, 0, true);
         const int st = boundary_sums_spectral(c, g, ns, a, sol, 0);
         if (st == VPMX_OK) {
-            if (timed) VPMX_HIP(c, hipEventRecord(e1, c->stream));
-            mark(c, ST_BOUNDS, 1);
+            mark(c, ST_COUNT + K_BOUNDSUM, 1);
+            mark(c, ST_BOUNDS, 1, true);
             c->last_pairs += (double)nt * (double)ns;
             return VPMX_OK;
         }
         if (st != VPMX_ERR_UNSUP) return st;
-        if (timed) c->kev_pending[K_BOUNDSUM] -= 1;  // nothing ran: drop the interval
+        unmark(c, ST_COUNT + K_BOUNDSUM);  // nothing ran: drop the interval
         mark(c, ST_BOUNDS, 1);  // faces too long for the in-LDS transforms: lattice kernel
     } else if (c->bs_mode == 2) {  // the coarse grid: its own plan
         const int st = boundary_sums_spectral(c, g, ns, a, sol, 1);

@@ -642,8 +642,7 @@ int p2m_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
         if (!ensure(c, c->tile_pos, sizeof(int) * (size_t)(tiles0 + 1), &st)) return st;
         if (!ensure(c, c->tile_list, sizeof(int) * (size_t)tiles0, &st)) return st;
         if (keep_zeros && !ensure(c, c->zt_prev, sizeof(int) * (size_t)tiles0, &st)) return st;
-        const bool timed_all = kclass >= 0 && kernel_events(c, kclass, &e0, &e1);
-        if (timed_all) VPMX_HIP(c, hipEventRecord(e0, c->stream));
+        if (kclass >= 0) mark(c, ST_COUNT + kclass, 0);
         if (n > 0) {
             const dim3 gs((unsigned)((n + 255) / 256));
             if (f32)
@@ -698,7 +697,7 @@ int p2m_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
                         &out, &vx, &vy, &vz, &w0, &w1, &w2, (void *)&lst, (void *)&nl};
         VPMX_HIP(c, hipLaunchKernel(fn, dim3((unsigned)tiles), dim3(256), args, 0, c->stream));
         VPMX_HIP(c, hipGetLastError());
-        if (timed_all) VPMX_HIP(c, hipEventRecord(e1, c->stream));
+        if (kclass >= 0) mark(c, ST_COUNT + kclass, 1);
         return VPMX_OK;
     }
     if (ncomp == 3 && kclass >= 0 && kernel_events(c, kclass, &e0, &e1)) {
@@ -919,8 +918,7 @@ int m2p_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
         int *list = (int *)ensure(c, c->tile_list, sizeof(int) * (size_t)tiles, &st); if (st) return st;
         const unsigned gt = (unsigned)((tiles + 255) / 256);
         // timed as a whole (tile list and the tiles)
-        const bool timed = kernel_events(c, K_M2P, &e0, &e1);
-        if (timed) VPMX_HIP(c, hipEventRecord(e0, c->stream));
+        mark(c, ST_COUNT + K_M2P, 0, true);  // (the interpolation stage starts here)
         hipLaunchKernelGGL(k_m2p_outside, grid, dim3(256), 0, c->stream, keys, n, c->dn, up, gp);
         hipLaunchKernelGGL(k_zero_int, dim3(gt), dim3(256), 0, c->stream, flag, (int64_t)tiles);
         hipLaunchKernelGGL(k_m2p_flag_particles, grid, dim3(256), 0, c->stream, keys, n, c->dn, s.cn[0], s.cn[1], ntx,
@@ -948,7 +946,7 @@ int m2p_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
         const unsigned wg = (unsigned)(ch.per_cu * c->num_cu);
         VPMX_HIP(c, hipLaunchKernel(fn, dim3(wg), dim3(256), args, 0, c->stream));
         VPMX_HIP(c, hipGetLastError());
-        if (timed) VPMX_HIP(c, hipEventRecord(e1, c->stream));
+        mark(c, ST_COUNT + K_M2P, 1);
         return VPMX_OK;
     }
     if (itypeb == 2)

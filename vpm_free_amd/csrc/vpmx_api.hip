@@ -171,7 +171,7 @@ static int yaps_single(Ctx *c, bool *used) {
     GView rv = view(rhs_bl, nb), sv = view(sol_bl, nb);
     Grid gb = make_grid(G.nnbl, &G.xbound_bl[0], G.dpm);
     // 1. fine infinite-domain solve over the whole block
-    mark(c, ST_FINE, 0);
+    mark(c, ST_FINE, 0, true);
     // the boundary sums accumulate on the faces; the second solve writes every interior node
     VPMX_TRY(zero_faces(c, nb, sv));
     c->dst_timed_m = gb.n[1] - 2;  // the block's y lines are the timed sine-transform passes
@@ -199,7 +199,7 @@ static int yaps_single(Ctx *c, bool *used) {
     mark(c, ST_FINE, 1);
     used[ST_FINE] = used[ST_BOUNDS] = true;
     // 2. coarse correction
-    mark(c, ST_COARSE, 0);
+    mark(c, ST_COARSE, 0, true);
     const int cn[3] = {G.nn_coarse[0], G.nn_coarse[1], G.nn_coarse[2]};
     int64_t GC = (int64_t)cn[0] * cn[1] * cn[2];
     double *samp = (double *)ensure(c, c->samp, sizeof(double) * 3 * (size_t)GC, &st); if (st) return st;
@@ -235,7 +235,7 @@ static int yaps_single(Ctx *c, bool *used) {
     mark(c, ST_COARSE, 1);
     used[ST_COARSE] = true;
     // 3. TSC correction of the inner-box faces
-    mark(c, ST_BC, 0);
+    mark(c, ST_BC, 0, true);
     InterpArgs ia;
     for (int d = 0; d < 6; d++) ia.nbl[d] = G.nnbl_bl[d];
     for (int d = 0; d < 3; d++) {
@@ -251,7 +251,7 @@ static int yaps_single(Ctx *c, bool *used) {
     mark(c, ST_BC, 1);
     used[ST_BC] = true;
     // 4. final solve on the inner box
-    mark(c, ST_FINAL, 0);
+    mark(c, ST_FINAL, 0, true);
     const int32_t *w = G.nnbl_bl;
     int wn[3] = {w[3] - w[0] + 1, w[4] - w[1] + 1, w[5] - w[2] + 1};
     double h[3];
@@ -307,7 +307,7 @@ static int yaps_multi(Ctx *c, bool *used) {
     mark(c, ST_FINE, 1);
     used[ST_FINE] = used[ST_BOUNDS] = true;
     // 2. samples of every block, coarse RHS, coarse solve
-    mark(c, ST_COARSE, 0);
+    mark(c, ST_COARSE, 0, true);
     const int cn[3] = {G.nn_coarse[0], G.nn_coarse[1], G.nn_coarse[2]};
     const int64_t GC = (int64_t)cn[0] * cn[1] * cn[2];
     double *samp = (double *)ensure(c, c->samp, sizeof(double) * 3 * (size_t)GC * NB, &st); if (st) return st;
@@ -378,7 +378,7 @@ static int yaps_multi(Ctx *c, bool *used) {
     mark(c, ST_COARSE, 1);
     used[ST_COARSE] = true;
     // 3. interp_stencil on every block's inner-box faces
-    mark(c, ST_BC, 0);
+    mark(c, ST_BC, 0, true);
     MbArgs a;
     for (int d = 0; d < 3; d++) {
         a.h[d] = G.dpm[d];
@@ -397,7 +397,7 @@ static int yaps_multi(Ctx *c, bool *used) {
     mark(c, ST_BC, 1);
     used[ST_BC] = true;
     // 4. inner-box solves
-    mark(c, ST_FINAL, 0);
+    mark(c, ST_FINAL, 0, true);
     for (int b = 0; b < NB; b++) {
         const int32_t *w = &G.nnbl_bl[6 * b];
         int wn[3] = {w[3] - w[0] + 1, w[4] - w[1] + 1, w[5] - w[2] + 1};
@@ -503,7 +503,7 @@ static int run_vpm(Ctx *c, int whattodo, const double *xp, const double *qp, dou
                                    view(rhs_bl + boff[b], block_n(G, b))));
         }
     }
-    mark(c, ST_PROJ, 1);
+    mark(c, ST_PROJ, 1, !multi && P.interf_iproj == 4);  // (the timed projection path has just ended)
     used[ST_PROJ] = true;
     if (whattodo == 4 || whattodo == 5) {
         // no Poisson solve (vpm.f90:316-373): mode 4 stretching from the velocity grids of the
@@ -513,15 +513,15 @@ static int run_vpm(Ctx *c, int whattodo, const double *xp, const double *qp, dou
         double *str = (double *)ensure(c, c->str, sizeof(double) * 3 * (size_t)GG, &st); if (st) return st;
         if (fresh || whattodo == 5) VPMX_TRY(fill(c, vel, 3 * GG, 0.0));  // velvr*_pm = 0
         GView rg = global_rhs(c);
-        mark(c, ST_FD, 0);
+        mark(c, ST_FD, 0, whattodo == 4);
         if (whattodo == 4) VPMX_TRY(stretch_kernel(c, gn, G.dpm, rg, view(vel, gn), view(str, gn)));
         else VPMX_TRY(diffuse_kernel(c, gn, G.dpm, ni, rg, view(str, gn)));
         mark(c, ST_FD, 1);
         used[ST_FD] = true;
-        mark(c, ST_BACK, 0);
+        mark(c, ST_BACK, 0, true);
         VPMX_TRY(m2p_gather(c, gg, c->sort, xp, qp, c->neqpm + 1, P.interf_iproj, view(vel, gn), view(str, gn), up, gp,
                             n, whattodo == 5 ? 2 : 1));
-        mark(c, ST_BACK, 1);
+        mark(c, ST_BACK, 1, whattodo == 4);
         used[ST_BACK] = true;
         c->have_grids = true;
         collect_times(c, used);
@@ -547,16 +547,16 @@ static int run_vpm(Ctx *c, int whattodo, const double *xp, const double *qp, dou
     double *str = (double *)ensure(c, c->str, sizeof(double) * 3 * (size_t)GG, &st); if (st) return st;
     GView psi = global_psi(c);
     GView rg = global_rhs(c);
-    mark(c, ST_FD, 0);
+    mark(c, ST_FD, 0, !multi);
     if (whattodo == 2) VPMX_TRY(curl_stretch_kernel(c, gn, G.dpm, psi, rg, view(vel, gn), view(str, gn)));
     else VPMX_TRY(curl_kernel(c, gn, G.dpm, psi, view(vel, gn)));
     mark(c, ST_FD, 1);
     used[ST_FD] = true;
     if (whattodo == 2) {
-        mark(c, ST_BACK, 0);
+        mark(c, ST_BACK, 0, true);
         VPMX_TRY(m2p_gather(c, gg, c->sort, xp, qp, c->neqpm + 1, P.interf_iproj, view(vel, gn), view(str, gn), up, gp,
                             n));
-        mark(c, ST_BACK, 1);
+        mark(c, ST_BACK, 1, true);  // (with the timed interpolation path)
         used[ST_BACK] = true;
     }
     collect_times(c, used);
@@ -1171,10 +1171,7 @@ void vpmx_destroy(vpmx_ctx *p) {
         for (hipEvent_t e : c->kev0[k]) (void)hipEventDestroy(e);
         for (hipEvent_t e : c->kev1[k]) (void)hipEventDestroy(e);
     }
-    for (int k = 0; k < ST_COUNT; k++) {
-        for (hipEvent_t e : c->sev0[k]) (void)hipEventDestroy(e);
-        for (hipEvent_t e : c->sev1[k]) (void)hipEventDestroy(e);
-    }
+    for (hipEvent_t e : c->bev) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(c->stream);
     delete c;
 }

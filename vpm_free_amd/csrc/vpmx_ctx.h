@@ -147,8 +147,14 @@ struct Ctx : vpmx_ctx {
     // the outermost API call ends (TimingScope), so no stage drains the stream
     bool timing = true;
     int timing_depth = 0;
-    std::vector<hipEvent_t> sev0[ST_COUNT], sev1[ST_COUNT];
-    int sev_used[ST_COUNT] = {};
+    // interval boundaries of this call: events in queue order, and the intervals between them
+    // (kind: a Stage, or ST_COUNT + a KClass whose whole path is timed)
+    struct Span {
+        int kind, a, b;
+    };
+    std::vector<hipEvent_t> bev;
+    int bev_used = 0;
+    std::vector<Span> spans;
     double stage_ms[ST_COUNT] = {};
     double last_pairs = 0.0;
     std::vector<hipEvent_t> kev0[K_COUNT], kev1[K_COUNT];
@@ -162,8 +168,6 @@ struct Ctx : vpmx_ctx {
 
 void free_fft_plans(Ctx *c);
 double wall_ms();
-// Stage timing: drain the stream at both ends so the interval covers exactly the stage's
-// kernels (enqueueing is asynchronous).
 // Add the durations of the recorded dispatches of every class (the stream is drained).
 inline void resolve_kernel_times(Ctx *c) {
     for (int k = 0; k < K_COUNT; k++) {
@@ -177,26 +181,39 @@ inline void resolve_kernel_times(Ctx *c) {
         c->kev_pending[k] = 0;
     }
 }
-// Stage timing: an event on the stream at the stage's start and end (a stage may run several
-// times in one call; each run gets its own pair).
-inline void mark(Ctx *c, int stage, int end) {
+// Timing events carry no system-scope release: they are only read back after the stream has been
+// drained, and a release at every boundary of a small call costs more than its kernels (33^3 ring:
+// 690 us a call with them, 645 without, 575 with no events at all).
+inline hipError_t timing_event(hipEvent_t *e) { return hipEventCreateWithFlags(e, hipEventDisableSystemFence); }
+// The index of a boundary event: a new one at this point of the stream, or -- same: nothing has
+// been queued since the last one -- the last one again.
+inline int boundary(Ctx *c, bool same) {
+    if (same && c->bev_used > 0) return c->bev_used - 1;
+    if (c->bev_used == (int)c->bev.size()) {
+        hipEvent_t e;
+        if (timing_event(&e) != hipSuccess) return -1;
+        c->bev.push_back(e);
+    }
+    if (hipEventRecord(c->bev[c->bev_used], c->stream) != hipSuccess) return -1;
+    return c->bev_used++;
+}
+// Start (end = 0) and end of an interval of `kind`; same: see boundary().
+inline void mark(Ctx *c, int kind, int end, bool same = false) {
     if (!c->timing || !c->kev_ok || c->timing_depth == 0 || c->nodrain) return;
     if (!end) {
-        const int i = c->sev_used[stage];
-        if (i == (int)c->sev0[stage].size()) {
-            hipEvent_t a, b;
-            if (hipEventCreate(&a) != hipSuccess) return;
-            if (hipEventCreate(&b) != hipSuccess) {
-                (void)hipEventDestroy(a);
-                return;
-            }
-            c->sev0[stage].push_back(a);
-            c->sev1[stage].push_back(b);
-        }
-        if (hipEventRecord(c->sev0[stage][i], c->stream) == hipSuccess) c->sev_used[stage] = i + 1;
-    } else if (c->sev_used[stage] > 0) {
-        (void)hipEventRecord(c->sev1[stage][c->sev_used[stage] - 1], c->stream);
+        const int i = boundary(c, same);
+        if (i >= 0) c->spans.push_back({kind, i, -1});
+        return;
     }
+    for (int q = (int)c->spans.size() - 1; q >= 0; q--)
+        if (c->spans[q].kind == kind && c->spans[q].b < 0) {
+            c->spans[q].b = boundary(c, same);
+            return;
+        }
+}
+// Takes back the open interval of `kind` (its path turned out not to run).
+inline void unmark(Ctx *c, int kind) {
+    if (!c->spans.empty() && c->spans.back().kind == kind && c->spans.back().b < 0) c->spans.pop_back();
 }
 // The outermost API call that runs stages: zero the stage times at its start, drain the
 // stream at its end and add up the recorded intervals (and the timed kernels).
@@ -204,23 +221,27 @@ struct TimingScope {
     Ctx *c;
     explicit TimingScope(Ctx *cc) : c(cc) {
         if (c->timing_depth++ == 0) {
-            for (int s = 0; s < ST_COUNT; s++) {
-                c->stage_ms[s] = 0.0;
-                c->sev_used[s] = 0;
-            }
+            for (int s = 0; s < ST_COUNT; s++) c->stage_ms[s] = 0.0;
+            c->bev_used = 0;
+            c->spans.clear();
         }
     }
     ~TimingScope() {
         if (--c->timing_depth != 0) return;
         if (c->nodrain) return;  // (nothing was recorded; a drain is not allowed under capture)
         (void)hipStreamSynchronize(c->stream);
-        for (int s = 0; s < ST_COUNT; s++) {
-            for (int i = 0; i < c->sev_used[s]; i++) {
-                float ms = 0.f;
-                if (hipEventElapsedTime(&ms, c->sev0[s][i], c->sev1[s][i]) == hipSuccess) c->stage_ms[s] += ms;
+        for (const Ctx::Span &p : c->spans) {
+            float ms = 0.f;
+            if (p.b < 0 || hipEventElapsedTime(&ms, c->bev[p.a], c->bev[p.b]) != hipSuccess) continue;
+            if (p.kind < ST_COUNT) {
+                c->stage_ms[p.kind] += ms;
+            } else {
+                c->k_ms[p.kind - ST_COUNT] += ms;
+                c->k_launches[p.kind - ST_COUNT] += 1;
             }
-            c->sev_used[s] = 0;
         }
+        c->bev_used = 0;
+        c->spans.clear();
         resolve_kernel_times(c);
     }
 };
@@ -231,8 +252,8 @@ inline bool kernel_events(Ctx *c, int k, hipEvent_t *e0, hipEvent_t *e1) {
     if (i >= 64) return false;  // more than 64 undrained dispatches: leave the rest untimed
     if (i == (int)c->kev0[k].size()) {
         hipEvent_t a, b;
-        if (hipEventCreate(&a) != hipSuccess) return false;
-        if (hipEventCreate(&b) != hipSuccess) {
+        if (timing_event(&a) != hipSuccess) return false;
+        if (timing_event(&b) != hipSuccess) {
             (void)hipEventDestroy(a);
             return false;
         }
