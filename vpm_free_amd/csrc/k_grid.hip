@@ -100,19 +100,22 @@ int stretch_kernel(Ctx *c, const int n[3], const double h[3], GView rhs, GView v
 }
 
 // curl and stretching in one pass (calc_velocity_serial_3d, vpm_gcalc.f90:1-132): a work-group
-// owns a TX x TY column tile (256 threads) and marches through CS_KC planes of z, keeping the
+// owns a TX x TY column tile (256 threads) and marches through kc planes of z, keeping the
 // velocity of three planes (with a one-node halo in x and y) in LDS; each plane's velocity is
 // formed once per tile (halo nodes by the neighbouring tiles too) with k_curl's expressions,
 // and the stretching term reads its velocity neighbours from LDS with k_stretch's expressions
 // -- the same values bit for bit, without writing the velocity grid and reading it back.  The
-// tile shape is a tuner choice (the halo's share against the x extent of the rows).
-constexpr int CS_KC = 32;
+// tile shape is a tuner choice (the halo's share against the x extent of the rows).  kc is 32
+// where that gives every CU two work-groups, and is halved down to 4 until it does: each plane
+// is one dependent step of some 2 us (a 41^3 grid in one chunk: 75 us on 11 work-groups), and
+// the three planes formed twice per chunk cost little there.
+constexpr int CS_KC = 32, CS_KC_MIN = 4;
 // Tiles go out XCD by XCD in contiguous slices of each round of R work-groups (xcd_slice; R
 // about the work-groups resident at once), so the tiles that share halo columns, and the
 // planes each of them reads three times, meet in one L2.
 template <int TX, int TY>
 __global__ void __launch_bounds__(256) k_curl_stretch(int nx, int ny, int nz, double ix2, double iy2, double iz2,
-                                                       GView psi, GView rhs, GView vel, GView out, int R) {
+                                                       GView psi, GView rhs, GView vel, GView out, int R, int kc) {
 #pragma clang fp contract(off)
     static_assert(TX * TY == 256, "one thread per column of the tile");
     constexpr int CS_HX = TX + 2, CS_HY = TY + 2;
@@ -120,7 +123,7 @@ __global__ void __launch_bounds__(256) k_curl_stretch(int nx, int ny, int nz, do
     const int64_t gx = gridDim.x, gy = gridDim.y;
     const int64_t lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
     const int64_t slot = xcd_slice(lin, gx * gy * gridDim.z, R);
-    const int i0 = (int)(slot % gx) * TX, j0 = (int)((slot / gx) % gy) * TY, kb = (int)(slot / (gx * gy)) * CS_KC;
+    const int i0 = (int)(slot % gx) * TX, j0 = (int)((slot / gx) % gy) * TY, kb = (int)(slot / (gx * gy)) * kc;
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
     const double *p0 = psi.p, *p1 = psi.p + psi.cs, *p2 = psi.p + 2 * psi.cs;
     auto fill = [&](int kk) {  // velocity of plane kk on the tile and its halo
@@ -145,7 +148,7 @@ __global__ void __launch_bounds__(256) k_curl_stretch(int nx, int ny, int nz, do
     };
     fill(kb - 1);
     fill(kb);
-    const int kend = kb + CS_KC < nz ? kb + CS_KC : nz;
+    const int kend = kb + kc < nz ? kb + kc : nz;
     const int i = i0 + tx, j = j0 + ty;
     for (int k = kb; k < kend; k++) {
         fill(k + 1);
@@ -184,7 +187,7 @@ __global__ void __launch_bounds__(256) k_curl_stretch(int nx, int ny, int nz, do
 // and their operands are k_curl's and k_stretch's, so the values are the same bit for bit.
 template <int TX, int TY>
 __global__ void __launch_bounds__(256) k_curl_stretch_w(int nx, int ny, int nz, double ix2, double iy2, double iz2,
-                                                         GView psi, GView rhs, GView vel, GView out, int R) {
+                                                         GView psi, GView rhs, GView vel, GView out, int R, int kc) {
 #pragma clang fp contract(off)
     static_assert(TX * TY == 256, "one thread per column of the tile");
     constexpr int CS_HX = TX + 2, CS_HY = TY + 2, RX = TX + 4, RY = TY + 4;
@@ -194,7 +197,7 @@ __global__ void __launch_bounds__(256) k_curl_stretch_w(int nx, int ny, int nz, 
     const int64_t gx = gridDim.x, gy = gridDim.y;
     const int64_t lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
     const int64_t slot = xcd_slice(lin, gx * gy * gridDim.z, R);
-    const int i0 = (int)(slot % gx) * TX, j0 = (int)((slot / gx) % gy) * TY, kb = (int)(slot / (gx * gy)) * CS_KC;
+    const int i0 = (int)(slot % gx) * TX, j0 = (int)((slot / gx) % gy) * TY, kb = (int)(slot / (gx * gy)) * kc;
     const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX;
     const double *p0 = psi.p, *p1 = psi.p + psi.cs, *p2 = psi.p + 2 * psi.cs;
     // the thread's region columns: (hx, hy) <-> node (i0 - 2 + hx, j0 - 2 + hy)
@@ -218,7 +221,7 @@ __global__ void __launch_bounds__(256) k_curl_stretch_w(int nx, int ny, int nz, 
         w0[s][2] = ld(p0, s, kb - 1);
         w1[s][2] = ld(p1, s, kb - 1);
     }
-    const int kend = kb + CS_KC < nz ? kb + CS_KC : nz;
+    const int kend = kb + kc < nz ? kb + kc : nz;
     const int i = i0 + tx, j = j0 + ty;
     const bool tin = i < nx && j < ny;
     const bool sint = i >= 2 && i <= nx - 3 && j >= 2 && j <= ny - 3;
@@ -313,10 +316,13 @@ int curl_stretch_kernel(Ctx *c, const int n[3], const double h[3], GView psi, GV
     int nx = n[0], ny = n[1], nz = n[2];
     int R = c->num_cu * 4 / 8 * 8;  // about the work-groups resident at once (4 per CU)
     if (R < 8) R = 8;
-    void *args[] = {&nx, &ny, &nz, &ix2, &iy2, &iz2, &psi, &rhs, &vel, &out, &R};
+    int kc = CS_KC;
+    const int64_t cols = (int64_t)((n[0] + 31) / 32) * ((n[1] + 7) / 8);
+    while (kc > CS_KC_MIN && cols * ((n[2] + kc - 1) / kc) < 2 * (int64_t)c->num_cu) kc /= 2;
+    void *args[] = {&nx, &ny, &nz, &ix2, &iy2, &iz2, &psi, &rhs, &vel, &out, &R, &kc};
     auto grid_of = [&](int fi) {
         return dim3((unsigned)((n[0] + shp[fi][0] - 1) / shp[fi][0]), (unsigned)((n[1] + shp[fi][1] - 1) / shp[fi][1]),
-                    (unsigned)((n[2] + CS_KC - 1) / CS_KC));
+                    (unsigned)((n[2] + kc - 1) / kc));
     };
     // trials write the real outputs: every variant writes the same values to every node
     auto trial = [&](int fi, int) -> int {
@@ -429,6 +435,12 @@ __device__ __forceinline__ double tsc(double x) {
     return 0.5 * ((a + 1.5) * (a + 1.5)) - 1.5 * ((a + 0.5) * (a + 0.5));
 }
 
+// The weights of coarse nodes n-1, n, n+1 (1-based) at x, along one axis.
+__device__ __forceinline__ void tsc3(double x, double xc, double hc, int n, double w[3]) {
+#pragma clang fp contract(off)
+    for (int d = 0; d < 3; d++) w[d] = tsc((x - xc - (double)(n - 2 + d) * hc) / hc);
+}
+
 // interp_stencil for every node of the six faces of the inner box, in face order.
 __global__ void __launch_bounds__(256) k_face_interp(int ncomp, InterpArgs a, int64_t nface, GView csol, GView samp,
                                                       GView sol) {
@@ -464,23 +476,27 @@ __global__ void __launch_bounds__(256) k_face_interp(int ncomp, InterpArgs a, in
     int64_t o = sol.at(i - 1, j - 1, k - 1);
     double acc[3];
     for (int q = 0; q < ncomp; q++) acc[q] = sol.p[q * sol.cs + o];
-    for (int kc = kn - 1; kc <= kn + 1; kc++)
-        for (int jc = jn - 1; jc <= jn + 1; jc++)
-            for (int ic = in - 1; ic <= in + 1; ic++) {
-                double xc = (X0 - a.xc[0] - (double)(ic - 1) * a.hc[0]) / a.hc[0];
-                double yc = (X1 - a.xc[1] - (double)(jc - 1) * a.hc[1]) / a.hc[1];
-                double zc = (X2 - a.xc[2] - (double)(kc - 1) * a.hc[2]) / a.hc[2];
-                double fw = tsc(xc) * tsc(yc) * tsc(zc);
-                bool ok = ic >= 1 && ic <= a.cn[0] && jc >= 1 && jc <= a.cn[1] && kc >= 1 && kc <= a.cn[2];
-                int64_t oc = ok ? csol.at(ic - 1, jc - 1, kc - 1) : 0;
+    double wx[3], wy[3], wz[3];
+    tsc3(X0, a.xc[0], a.hc[0], in, wx);
+    tsc3(X1, a.xc[1], a.hc[1], jn, wy);
+    tsc3(X2, a.xc[2], a.hc[2], kn, wz);
+    for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int b = 0; b < 3; b++) {  // (nine nodes' loads in flight)
+            const int jc = jn - 1 + b, kc = kn - 1 + c;
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const int ic = in - 1 + d;
+                const double fw = wx[d] * wy[b] * wz[c];
+                const bool ok = ic >= 1 && ic <= a.cn[0] && jc >= 1 && jc <= a.cn[1] && kc >= 1 && kc <= a.cn[2];
+                const int64_t oc = ok ? csol.at(ic - 1, jc - 1, kc - 1) : 0;
                 for (int q = 0; q < ncomp; q++) {
-                    double cs = ok ? csol.p[q * csol.cs + oc] : 0.0;
-                    double sm = ok ? samp.p[q * samp.cs + oc] : 0.0;
-                    double add_sample = sm + 0.0;
-                    double add = nnb ? sm + 0.0 : 0.0;
-                    acc[q] = acc[q] + fw * ((cs - add_sample) + add);
+                    double cs = csol.p[q * csol.cs + oc], sm = samp.p[q * samp.cs + oc];
+                    if (!ok) cs = sm = 0.0;
+                    acc[q] = acc[q] + fw * ((cs - sm) + (nnb ? sm : 0.0));
                 }
             }
+        }
     for (int q = 0; q < ncomp; q++) sol.p[q * sol.cs + o] = acc[q];
 }
 int face_interp(Ctx *c, int ncomp, const InterpArgs &a, GView csol, GView samp, GView sol) {
@@ -554,26 +570,38 @@ __global__ void __launch_bounds__(256) k_face_interp_mb(MbArgs a, const MbBlock 
     const int64_t o = ((int64_t)(k - 1) * B.n[1] + (j - 1)) * B.n[0] + (i - 1);
     const double *own = fine + B.off;
     double acc[3] = {own[o], own[B3 + o], own[2 * B3 + o]};
-    for (int kc = kn - 1; kc <= kn + 1; kc++)
-        for (int jc = jn - 1; jc <= jn + 1; jc++)
-            for (int ic = in - 1; ic <= in + 1; ic++) {
-                const double xc = (X0 - a.xc[0] - (double)(ic - 1) * a.hc[0]) / a.hc[0];
-                const double yc = (X1 - a.xc[1] - (double)(jc - 1) * a.hc[1]) / a.hc[1];
-                const double zc = (X2 - a.xc[2] - (double)(kc - 1) * a.hc[2]) / a.hc[2];
-                const double fw = tsc(xc) * tsc(yc) * tsc(zc);
+    // (a sample counts where its block's footprint holds the stencil: elsewhere the reference
+    // takes it off and adds it back)
+    double wx[3], wy[3], wz[3];
+    tsc3(X0, a.xc[0], a.hc[0], in, wx);
+    tsc3(X1, a.xc[1], a.hc[1], jn, wy);
+    tsc3(X2, a.xc[2], a.hc[2], kn, wz);
+    const uint64_t all = a.nblocks == 64 ? ~(uint64_t)0 : ((uint64_t)1 << a.nblocks) - 1;
+    for (int c = 0; c < 3; c++)
+        for (int b2 = 0; b2 < 3; b2++) {
+            const int jc = jn - 1 + b2, kc = kn - 1 + c;
+            double v[3][3];
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const int ic = in - 1 + d;
                 const bool ok = ic >= 1 && ic <= a.cn[0] && jc >= 1 && jc <= a.cn[1] && kc >= 1 && kc <= a.cn[2];
                 const int64_t oc = ok ? csol.at(ic - 1, jc - 1, kc - 1) : 0;
-                for (int q = 0; q < 3; q++) {
-                    double add_sample = 0.0, add = 0.0;
-                    for (int bc = 0; bc < a.nblocks; bc++) {
-                        const double sm = ok ? samp[(int64_t)bc * a.sstride + q * csol.cs + oc] : 0.0;
-                        add_sample = sm + add_sample;
-                        if ((nnb >> bc) & 1) add = sm + add;
-                    }
-                    const double cs = ok ? csol.p[q * csol.cs + oc] : 0.0;
-                    acc[q] = acc[q] + fw * ((cs - add_sample) + add);
+                for (int q = 0; q < 3; q++) v[d][q] = ok ? csol.p[q * csol.cs + oc] : 0.0;
+            }
+            for (uint64_t left = all & ~nnb; left; left &= left - 1) {
+                const double *sb = samp + (int64_t)__builtin_ctzll(left) * a.sstride;
+#pragma unroll
+                for (int d = 0; d < 3; d++) {  // (a footprint that holds the stencil lies inside the coarse grid)
+                    const int64_t oc = csol.at(in - 2 + d, jc - 1, kc - 1);
+                    for (int q = 0; q < 3; q++) v[d][q] = v[d][q] - sb[q * csol.cs + oc];
                 }
             }
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const double fw = wx[d] * wy[b2] * wz[c];
+                for (int q = 0; q < 3; q++) acc[q] = acc[q] + fw * v[d][q];
+            }
+        }
     // neighbours whose footprint covers the stencil: their fine solution at the node (BBound)
     for (int kb = B.bk - 1; kb <= B.bk + 1; kb++)
         for (int jb = B.bj - 1; jb <= B.bj + 1; jb++)
