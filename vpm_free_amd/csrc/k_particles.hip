@@ -365,7 +365,11 @@ __global__ void k_row_counts(const int *__restrict__ start, int cnx, int64_t nro
 // it (W((x - x0)/h - (i - 1)) for node i), formed once per tile, in chunks of whole rows that
 // fit; every thread then sums its node's 16 rows, the four cells of each, rows z-outer,
 // y-inner, cells and particles in cell order: deterministic, no atomics.  A row with more particles than a chunk holds is read straight from memory in the
-// same order.  Tiles without particles are written by k_p2m_zero_tiles.
+// same order.  Tiles without particles are written by k_p2m_zero_tiles.  On grids of up to
+// SMALL_TILES tiles (about 128^3 nodes) there is no list: every tile gets a work-group, which reads
+// its 49 row ends itself and writes zeros if it finds no particle -- six small launches (row
+// counts, flags, scan, list, zeros, copy: some 40 us) less for at most 50 MB of zeros.
+constexpr int SMALL_TILES = 8192;
 // Round of the one-work-group-per-tile launches (xcd_slice): 256 work-groups per XCD.
 constexpr int64_t XCD_ROUND = 2048;
 
@@ -488,8 +492,8 @@ __global__ void __launch_bounds__(256) k_p2m_tile(Grid g, const int *__restrict_
     const int tid = threadIdx.x;
     const int ntx = (vnx + PT_X - 1) / PT_X, nty = (vny + PT_Y - 1) / PT_Y;
     const int64_t slot = xcd_slice(blockIdx.x, gridDim.x, XCD_ROUND);
-    if (slot >= *nlist) return;
-    const int tile = list[slot];
+    if (list && slot >= *nlist) return;
+    const int tile = list ? list[slot] : (int)slot;
     const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
     const int lx = tid & (PT_X - 1), ly = (tid / PT_X) & (PT_Y - 1), lz = tid / (PT_X * PT_Y);
     const int va = tx * PT_X + lx, vb = ty * PT_Y + ly, vc = tz * PT_Z + lz;
@@ -501,7 +505,12 @@ __global__ void __launch_bounds__(256) k_p2m_tile(Grid g, const int *__restrict_
     if (tid < PT_ROWS) {
         const int cj = J0 - 2 + tid % PC_Y, ck = K0 - 2 + tid / PC_Y;
         int ok = cj >= -1 && cj <= g.n[1] + 1 && ck >= -1 && ck <= g.n[2] + 1;
-        if (ok) ok = rowcnt[(cj + 1) + (int64_t)cny * (ck + 1)] > 0;
+        if (ok) {
+            const int64_t row = (cj + 1) + (int64_t)cny * (ck + 1);
+            // (without the counts: the row's particles near the tile only)
+            ok = rowcnt ? rowcnt[row] > 0
+                        : start[row * cnx + min(I0 + PT_X + 2, g.n[0] + 2) + 1] > start[row * cnx + max(I0 - 2, -1) + 1];
+        }
         rowok[tid] = ok;
         if (ok) any = 1;
     }
@@ -642,6 +651,7 @@ int p2m_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
         if (!ensure(c, c->tile_pos, sizeof(int) * (size_t)(tiles0 + 1), &st)) return st;
         if (!ensure(c, c->tile_list, sizeof(int) * (size_t)tiles0, &st)) return st;
         if (keep_zeros && !ensure(c, c->zt_prev, sizeof(int) * (size_t)tiles0, &st)) return st;
+        const bool small = tiles0 <= SMALL_TILES;
         if (kclass >= 0) mark(c, ST_COUNT + kclass, 0);
         if (n > 0) {
             const dim3 gs((unsigned)((n + 255) / 256));
@@ -652,14 +662,18 @@ int p2m_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
                 hipLaunchKernelGGL(k_p2m_sorted<double>, gs, dim3(256), 0, c->stream, perm, start + s.ncells, n,
                                    g, xp, qp, qstride, (double *)Rv);
         }
-        hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((nrows + 255) / 256)), dim3(256), 0, c->stream, start,
-                           s.cn[0], nrows, rowcnt);
         const int ntx = (vn[0] + PT_X - 1) / PT_X, nty = (vn[1] + PT_Y - 1) / PT_Y;
         const int64_t tiles = (int64_t)ntx * nty * ((vn[2] + PT_Z - 1) / PT_Z);
         int *flag = (int *)ensure(c, c->tile_flag, sizeof(int) * (size_t)tiles, &st); if (st) return st;
         int *pos = (int *)ensure(c, c->tile_pos, sizeof(int) * (size_t)(tiles + 1), &st); if (st) return st;
         int *list = (int *)ensure(c, c->tile_list, sizeof(int) * (size_t)tiles, &st); if (st) return st;
         const unsigned gt = (unsigned)((tiles + 255) / 256);
+        if (small) {  // every node is written by its tile
+            c->zt_valid = false;
+            rowcnt = nullptr;
+        } else {
+        hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((nrows + 255) / 256)), dim3(256), 0, c->stream, start,
+                           s.cn[0], nrows, rowcnt);
         hipLaunchKernelGGL(k_p2m_tile_flags, dim3(gt), dim3(256), 0, c->stream, (int)tiles, ntx, nty, vn[0], vn[1],
                            vn[2], g, s.cn[1], rowcnt, wlo[1], wlo[2], flag);
         VPMX_TRY(exclusive_scan(c, flag, pos, tiles));
@@ -690,9 +704,10 @@ int p2m_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
             c->tile_map_ntx = ntx;
             c->tile_map_nty = nty;
         }
+        }
         const void *fn = f32 ? (const void *)k_p2m_tile<float> : (const void *)k_p2m_tile<double>;
         int cnx = s.cn[0], cny = s.cn[1], vx = vn[0], vy = vn[1], vz = vn[2], w0 = wlo[0], w1 = wlo[1], w2 = wlo[2];
-        const int *lst = list, *nl = pos + tiles;
+        const int *lst = small ? nullptr : list, *nl = small ? nullptr : pos + tiles;
         void *args[] = {(void *)&g, (void *)&start, (void *)&rowcnt, &cnx, &cny, &Rv, &div,
                         &out, &vx, &vy, &vz, &w0, &w1, &w2, (void *)&lst, (void *)&nl};
         VPMX_HIP(c, hipLaunchKernel(fn, dim3((unsigned)tiles), dim3(256), args, 0, c->stream));
@@ -801,9 +816,9 @@ __global__ void __launch_bounds__(256) k_m2p_tile(Grid g, const int *__restrict_
     __shared__ T nodes[M2P_NX * M2P_NY * M2P_NZ * 6];
     __shared__ int rs[M2P_ROWS + 1], rp[M2P_ROWS];
     const int ntx = (cnx + M2P_TX - 1) / M2P_TX, nty = (cny + M2P_TY - 1) / M2P_TY;
-    const int ntot = *nlist;
+    const int ntot = list ? *nlist : ntx * nty * ((cnz + M2P_TZ - 1) / M2P_TZ);
     for (int li = (int)xcd_slice(blockIdx.x, gridDim.x, gridDim.x); li < ntot; li += gridDim.x) {
-    const int tile = list[li];
+    const int tile = list ? list[li] : li;  // (no list: every tile, see SMALL_TILES)
     const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
     // cell indices (stored index = cell + 1) of the tile: [cx0, cx0 + TX) clipped to the grid
     const int cx0 = tx * M2P_TX, cy0 = ty * M2P_TY, cz0 = tz * M2P_TZ;
@@ -833,6 +848,10 @@ __global__ void __launch_bounds__(256) k_m2p_tile(Grid g, const int *__restrict_
     }
     __syncthreads();
     const int total = rs[M2P_ROWS];
+    if (total == 0) {  // (the whole work-group)
+        __syncthreads();
+        continue;
+    }
     // node region: a particle of stored cell cs (inode = cs - 1, the sort's cell) reaches the
     // nodes inode-1 .. inode+2 = cs-2 .. cs+1, so the tile's cells [cx0, cx0+TX) reach global
     // nodes (1-based) cx0-2 .. cx0+TX: region index a <-> node cx0 - 2 + a, a in [0, TX+3)
@@ -920,19 +939,22 @@ int m2p_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
         // timed as a whole (tile list and the tiles)
         mark(c, ST_COUNT + K_M2P, 0, true);  // (the interpolation stage starts here)
         hipLaunchKernelGGL(k_m2p_outside, grid, dim3(256), 0, c->stream, keys, n, c->dn, up, gp);
-        hipLaunchKernelGGL(k_zero_int, dim3(gt), dim3(256), 0, c->stream, flag, (int64_t)tiles);
-        hipLaunchKernelGGL(k_m2p_flag_particles, grid, dim3(256), 0, c->stream, keys, n, c->dn, s.cn[0], s.cn[1], ntx,
-                           nty, flag);
-        VPMX_TRY(exclusive_scan(c, flag, pos, tiles));
-        hipLaunchKernelGGL(k_m2p_tile_list, dim3(gt), dim3(256), 0, c->stream, tiles, flag, pos, list);
+        const bool small = tiles <= SMALL_TILES;
+        if (!small) {
+            hipLaunchKernelGGL(k_zero_int, dim3(gt), dim3(256), 0, c->stream, flag, (int64_t)tiles);
+            hipLaunchKernelGGL(k_m2p_flag_particles, grid, dim3(256), 0, c->stream, keys, n, c->dn, s.cn[0], s.cn[1],
+                               ntx, nty, flag);
+            VPMX_TRY(exclusive_scan(c, flag, pos, tiles));
+            hipLaunchKernelGGL(k_m2p_tile_list, dim3(gt), dim3(256), 0, c->stream, tiles, flag, pos, list);
+        }
         // persistent: the work-groups per CU the tuner picks, at most what one CU holds (LDS-bound:
         // 40 KB of FP64 node values, 20 KB of FP32 in the mixed form); the kernel's results do
         // not depend on the grid, so the tuner's trials are real launches
         const bool f32 = c->precision == 1;
         const void *fn = f32 ? (const void *)k_m2p_tile<float> : (const void *)k_m2p_tile<double>;
         int gn = (int)s.cn[0], gny = (int)s.cn[1], gnz = (int)s.cn[2];
-        const int *nl = pos + tiles;
-        void *args[] = {(void *)&g, (void *)&start, (void *)&perm, &gn, &gny, &gnz, (void *)&list, (void *)&nl,
+        const int *nl = small ? nullptr : pos + tiles, *lst = small ? nullptr : list;
+        void *args[] = {(void *)&g, (void *)&start, (void *)&perm, &gn, &gny, &gnz, (void *)&lst, (void *)&nl,
                         (void *)&xp, (void *)&qp, &qstride, &itype, &vel, &sol, &up, &gp};
         char key[128];
         std::snprintf(key, sizeof key, "interpolation tiles %s cells=%dx%dx%d", f32 ? "FP32" : "FP64", gn, gny, gnz);
@@ -942,8 +964,11 @@ int m2p_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
             VPMX_HIP(c, hipLaunchKernel(fn, dim3((unsigned)(pc * c->num_cu)), dim3(256), args, 0, c->stream));
             return VPMX_OK;
         };
-        VPMX_TRY(tune(c, key, 1, &fn, names, 0, 256, trial, &ch));
-        const unsigned wg = (unsigned)(ch.per_cu * c->num_cu);
+        unsigned wg = (unsigned)tiles;
+        if (!small) {
+            VPMX_TRY(tune(c, key, 1, &fn, names, 0, 256, trial, &ch));
+            wg = (unsigned)(ch.per_cu * c->num_cu);
+        }
         VPMX_HIP(c, hipLaunchKernel(fn, dim3(wg), dim3(256), args, 0, c->stream));
         VPMX_HIP(c, hipGetLastError());
         mark(c, ST_COUNT + K_M2P, 1);
