@@ -34,7 +34,7 @@ __host__ __device__ inline void face_dims(const int n[3], int f, int *N0, int *N
 // The one-sided 5-point normal derivative (1/h_n)(25/12 f0 - 4 f1 + 3 f2 - 4/3 f3 + 1/4 f4) at
 // every node of every face, once per node (a node is a corner of up to four face cells):
 // thread per (face, node), the in-plane index with the faster memory stride first.
-__global__ void __launch_bounds__(256) k_face_node_derivs(Grid g, GView s0, int ncomp, FaceNodes fo, double *fd) {
+__global__ void __launch_bounds__(256) k_face_node_derivs(Grid g, GView s0, int ncomp, FaceNodes fo, double *fd, int zf) {
 #pragma clang fp contract(off)
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nn = fo.off[6] / ncomp;
@@ -54,7 +54,9 @@ __global__ void __launch_bounds__(256) k_face_node_derivs(Grid g, GView s0, int 
         for (int st = 0; st < 5; st++) {
             const int q = pl + sg * st;
             const int ii = axis == 0 ? q : a, jj = axis == 1 ? q : (axis == 0 ? a : b), kk = axis == 2 ? q : b;
-            v[st] = sp[s0.at(ii - 1, jj - 1, kk - 1)];
+            // zf: the faces are zero and not read
+            const bool edge = ii == 1 || ii == g.n[0] || jj == 1 || jj == g.n[1] || kk == 1 || kk == g.n[2];
+            v[st] = zf && edge ? 0.0 : sp[s0.at(ii - 1, jj - 1, kk - 1)];
         }
         fd[fo.off[f] + (int64_t)c * N0 * N1 + r] = (1.0 / hn) * ((((a1 * v[0] + a2 * v[1]) + a3 * v[2]) + a4 * v[3]) + a5 * v[4]);
     }
@@ -153,7 +155,7 @@ int normal_derivs_cells(Ctx *c, int ncomp, const Grid &g, const double *fd, doub
     return VPMX_OK;
 }
 
-int normal_derivs(Ctx *c, int ncomp, const Grid &g, GView s0, double *sig, double *cxyz, double *wgt, int64_t *nbound) {
+int normal_derivs(Ctx *c, int ncomp, const Grid &g, GView s0, double *sig, double *cxyz, double *wgt, int64_t *nbound, bool zero_faces) {
     if (g.n[0] < 6 || g.n[1] < 6 || g.n[2] < 6) return fail(c, VPMX_ERR_ARG, "normal derivatives need >= 6 nodes per axis");
     // the derivative at each face node once, then each cell's four-corner average
     const FaceNodes fo = face_nodes(ncomp, g.n);
@@ -162,7 +164,7 @@ int normal_derivs(Ctx *c, int ncomp, const Grid &g, GView s0, double *sig, doubl
     if (st) return st;
     const int64_t nn = fo.off[6] / ncomp;
     hipLaunchKernelGGL(k_face_node_derivs, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, c->stream, g, s0, ncomp,
-                       fo, fd);
+                       fo, fd, zero_faces ? 1 : 0);
     VPMX_HIP(c, hipGetLastError());
     return normal_derivs_cells(c, ncomp, g, fd, sig, cxyz, wgt, nbound);
 }
@@ -551,16 +553,18 @@ static int boundary_sums_lattice(Ctx *c, const Grid &g, int64_t ns, const double
 }
 
 int boundary_sums(Ctx *c, int ncomp, const Grid &g, int64_t ns, const double *sig, const double *cxyz,
-                  const double *wgt, GView sol, bool fine, int levmax, int ibctyp, const GView *scratch) {
+                  const double *wgt, GView sol, bool fine, int levmax, int ibctyp, const GView *scratch, bool fresh) {
     if (ncomp != 3) return fail(c, VPMX_ERR_UNSUP, "boundary sums: 3 components");
     const int NX = g.n[0], NY = g.n[1], NZ = g.n[2];
     int64_t nt = 2 * ((int64_t)NY * NZ + (int64_t)(NX - 2) * NZ + (int64_t)(NX - 2) * (NY - 2));
     const double *a = wgt, *ds = wgt + 3 * ns;
     if (ibctyp == 3) {  // panel sources: calc_boundinf_3d_s / calc_boundinf_3d_lev_s
         if (levmax < 0 && !scratch) return fail(c, VPMX_ERR_STATE, "panel sums need a scratch grid");
+        if (fresh) VPMX_TRY(zero_faces(c, g.n, sol));
         return boundary_sums_panels(c, g, ns, sig, cxyz, ds, sol, fine, levmax, scratch ? *scratch : sol);
     }
     if (levmax >= 0) {  // Bounds3d_lev (infdomain_3d with itree = 1, pinfdomain.f90:128-150)
+        if (fresh) VPMX_TRY(zero_faces(c, g.n, sol));
         if (fine) mark(c, ST_BOUNDS, 0);
         VPMX_TRY(boundary_sums_tree(c, g, ns, sig, cxyz, ds, sol, levmax, fine, false));
         if (fine) mark(c, ST_BOUNDS, 1);
@@ -570,21 +574,23 @@ int boundary_sums(Ctx *c, int ncomp, const Grid &g, int64_t ns, const double *si
     if (g.h[2] < hmin) hmin = g.h[2];
     // nearest source-target distance is h_min/sqrt(2) (face-cell centroid vs node)
     if (hmin * 0.70710678 <= 1.5e-5) {
+        if (fresh) VPMX_TRY(zero_faces(c, g.n, sol));
         hipLaunchKernelGGL(k_boundsum_exact, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, c->stream, g, nt, ns, cxyz,
                            sig, ds, sol);
         VPMX_HIP(c, hipGetLastError());
         return VPMX_OK;
     }
-    return point_sums(c, g, ns, cxyz, a, sol, fine);
+    return point_sums(c, g, ns, cxyz, a, sol, fine, fresh);
 }
 
-int point_sums(Ctx *c, const Grid &g, int64_t ns, const double *cxyz, const double *a, GView sol, bool fine) {
+int point_sums(Ctx *c, const Grid &g, int64_t ns, const double *cxyz, const double *a, GView sol, bool fine,
+               bool fresh) {
     const int NX = g.n[0], NY = g.n[1], NZ = g.n[2];
     int64_t nt = 2 * ((int64_t)NY * NZ + (int64_t)(NX - 2) * NZ + (int64_t)(NX - 2) * (NY - 2));
     if (fine && c->bs_mode == 2) {
         mark(c, ST_BOUNDS, 0);
         mark(c, ST_COUNT + K_BOUNDSUM, 0, true);
-        const int st = boundary_sums_spectral(c, g, ns, a, sol, 0);
+        const int st = boundary_sums_spectral(c, g, ns, a, sol, 0, fresh);
         if (st == VPMX_OK) {
             mark(c, ST_COUNT + K_BOUNDSUM, 1);
             mark(c, ST_BOUNDS, 1, true);
@@ -595,10 +601,11 @@ int point_sums(Ctx *c, const Grid &g, int64_t ns, const double *cxyz, const doub
         unmark(c, ST_COUNT + K_BOUNDSUM);  // nothing ran: drop the interval
         mark(c, ST_BOUNDS, 1);  // faces too long for the in-LDS transforms: lattice kernel
     } else if (c->bs_mode == 2) {  // the coarse grid: its own plan
-        const int st = boundary_sums_spectral(c, g, ns, a, sol, 1);
+        const int st = boundary_sums_spectral(c, g, ns, a, sol, 1, fresh);
         if (st == VPMX_OK) return VPMX_OK;
         if (st != VPMX_ERR_UNSUP) return st;
     }
+    if (fresh) VPMX_TRY(zero_faces(c, g.n, sol));
     if (c->bs_mode != 1) return boundary_sums_lattice(c, g, ns, a, sol, fine);
     int64_t tblocks = (nt + BS_THREADS * BS_TPT - 1) / (BS_THREADS * BS_TPT);
     // split sources so the launch has >= ~2048 work-groups, each with >= 1024 sources

@@ -27,8 +27,7 @@
 // length Lq >= M + K - 1 along q (the table holds FFT(r_w) / Lq, nw x Lq values, instead of
 // the nw x M x K matrices).  Only the perpendicular family needs a matrix product.
 //
-// The products run in rocBLAS (FP64, atomics off, so the results do not depend on
-// scheduling); the transforms run in LDS with the Stockham FFT of the Poisson passes.  A
+// The products run on the matrix cores (k_dgemm.hip); the transforms run in LDS with the Stockham FFT of the Poisson passes.  A
 // final pass adds, for every boundary node, the six pair contributions of its owner face
 // in a fixed order (X faces own their edges, Y faces their z-edges).
 
@@ -70,6 +69,25 @@ struct SpecPair {  // where the contribution of source face A to target face B s
     int64_t base;  // offset of component 0 in Ores ([col][p][kt])
     int M, nC, tax, cax, flipp, pad;
 };
+
+// One matrix family's share of a launch: all families whose transforms have the same form run in
+// one (a cubic block has three, a flat one seven; each alone is a launch of 5-10 us on a small
+// grid).  fwd0 / inv0 / q0: its first work-group; gf / gi: work-groups per column.
+struct SpecJob {
+    SpecFft f;
+    WavePlan wf, wq;
+    SpecTab t;
+    const double2 *tw, *twq, *T2;
+    const SpecCol *cols;
+    int64_t b_off, c_off, o_off;
+    int ncol, gf, gi, fwd0, inv0, q0;
+};
+// The job of a work-group (jobs of one launch, first work-groups ascending).
+#define SPEC_JOB(first)                                        \
+    int ji = 0;                                                \
+    while (ji + 1 < nj && (int)blockIdx.x >= jobs[ji + 1].first) ji++; \
+    const SpecJob &J = jobs[ji];                               \
+    const int local = (int)blockIdx.x - J.first;
 
 // ------------------------------------------------------------------ kernels
 __device__ __forceinline__ int residue_offset(int r, int L, int nC, bool *ok) {
@@ -157,17 +175,22 @@ __device__ __forceinline__ void bsx_fft(double2 *A, const double2 *twl, const Sp
 // A^ of every column as two real columns: Bm[2 col][w][q] = Re, Bm[2 col + 1][w][q] = Im,
 // lines q of the block, one column per blockIdx.y.
 template <int FFT>
-__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsx_fwd(SpecFft f, WavePlan P, SpecTab t, const double2 *tw,
-                                                                 const SpecCol *cols, const double *a, int64_t ns,
-                                                                 double *Bm) {
+__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsx_fwd(const SpecJob *__restrict__ jobs, int nj, const double *a,
+                                                                 int64_t ns, double *Bm) {
 #pragma clang fp contract(off)
     extern __shared__ double2 lds[];
     constexpr int NT = bsx_threads<FFT>();
+    SPEC_JOB(fwd0)
+    const SpecFft &f = J.f;
+    const WavePlan &P = J.wf;
+    const SpecTab &t = J.t;
+    const double2 *tw = J.tw;
+    Bm += J.b_off;
     const int L = f.L, np = FFT == -2 ? f.npairs : BW_WAVES, nl = 2 * np;
     double2 *A = lds, *twl = lds + np * L;
     double *Ad = (double *)A;
-    const int tid = threadIdx.x, q0 = blockIdx.x * nl, col = blockIdx.y;
-    const SpecCol cd = cols[col];
+    const int tid = threadIdx.x, col = local / J.gf, q0 = (local - col * J.gf) * nl;
+    const SpecCol cd = J.cols[col];
     const double *src = a + (int64_t)cd.comp * ns + cd.src_off;
     const int ncell = t.nC - 1;  // source cells along C
     for (int i = tid; i < L; i += NT) twl[i] = tw[i];
@@ -210,14 +233,20 @@ __global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsx_fwd(SpecFft f, WaveP
 // Inverse real FFT over w of O^ = exp(-pi i w / L) (Cm[2 col][w][p] + i Cm[2 col + 1][w][p]),
 // first nC outputs -> Ores[col][p][kt].
 template <int FFT>
-__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsx_inv(SpecFft f, WavePlan P, SpecTab t, const double2 *tw,
-                                                                 const double *Cm, double *Ores, int64_t ores_off) {
+__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsx_inv(const SpecJob *__restrict__ jobs, int nj,
+                                                                 const double *Cm, double *Ores) {
 #pragma clang fp contract(off)
     extern __shared__ double2 lds[];
     constexpr int NT = bsx_threads<FFT>();
+    SPEC_JOB(inv0)
+    const SpecFft &f = J.f;
+    const WavePlan &P = J.wf;
+    const SpecTab &t = J.t;
+    const double2 *tw = J.tw;
+    Cm += J.c_off;
     const int L = f.L, np = FFT == -2 ? f.npairs : BW_WAVES, nl = 2 * np;
     double2 *A = lds, *twl = lds + np * L;
-    const int tid = threadIdx.x, p0 = blockIdx.x * nl, col = blockIdx.y;
+    const int tid = threadIdx.x, col = local / J.gi, p0 = (local - col * J.gi) * nl;
     const int64_t cst = (int64_t)t.nw * t.M;
     const double *in = Cm + 2 * col * cst;
     for (int i = tid; i < L; i += NT) twl[i] = tw[i];
@@ -241,7 +270,7 @@ __global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsx_inv(SpecFft f, WaveP
     bsx_fft<FFT>(A, twl, f, P);
     // z_n = FFT(Z)[(L - n) mod L] / L
     const double invL = 1.0 / (double)L;
-    double *out = Ores + ores_off + (int64_t)col * t.M * t.nC;
+    double *out = Ores + J.o_off + (int64_t)col * t.M * t.nC;
     for (int i = tid; i < nl * t.nC; i += NT) {
         const int l = i / t.nC, n = i - l * t.nC, p = p0 + l;
         if (p >= t.M) continue;
@@ -327,16 +356,22 @@ __global__ void __launch_bounds__(DST_THREADS) k_bsx_qconv(SpecFft fq, SpecTab t
 // barriers after the twiddles are staged, QC_WAVES sequences per work-group.
 constexpr int QC_WAVES = 4, QC_LMAX = 576;
 template <int FFT>  // 0: the 576-point compile-time plan, -1: the runtime plan P
-__global__ void __launch_bounds__(64 * QC_WAVES) k_bsx_qconv_w(WavePlan P, SpecTab t, const double2 *twq,
-                                                               const double2 *T2, const double *Bm, double *Cm,
-                                                               int ncol, int cj) {
+__global__ void __launch_bounds__(64 * QC_WAVES) k_bsx_qconv_w(const SpecJob *__restrict__ jobs, int nj, const double *Bm,
+                                                               double *Cm, int cj) {
 #pragma clang fp contract(off)
     extern __shared__ double2 lds[];
+    SPEC_JOB(q0)
+    const WavePlan &P = J.wq;
+    const SpecTab &t = J.t;
+    const double2 *twq = J.twq, *T2 = J.T2;
+    const int ncol = J.ncol;
+    Bm += J.b_off;
+    Cm += J.c_off;
     const int Lq = P.L, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     double2 *twl = lds + QC_WAVES * Lq;
     for (int i = threadIdx.x; i < Lq; i += 64 * QC_WAVES) twl[i] = twq[i];
     __syncthreads();
-    const int seq = blockIdx.x * QC_WAVES + wv;  // col * nw + w
+    const int seq = local * QC_WAVES + wv;  // col * nw + w
     if (seq >= ncol * t.nw) return;               // no work-group barrier below
     const int col = seq / t.nw, w = seq - col * t.nw;
     const int64_t cb = (int64_t)t.nw * t.K, cc = (int64_t)t.nw * t.M;
@@ -374,7 +409,7 @@ __host__ __device__ inline void gather_face(const int n[3], int B, int *na, int 
     *nb = ax == 2 ? n[1] - 2 : n[2];
 }
 __global__ void __launch_bounds__(64 * GATHER_WAVES) k_bsx_gather(Grid g, const SpecPair *pairs, const double *Ores,
-                                                                  GView sol) {
+                                                                  GView sol, int fresh) {
 #pragma clang fp contract(off)
     const int B = blockIdx.y, ax = B >> 1, hi = B & 1;
     int na, nb;
@@ -410,6 +445,12 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) k_bsx_gather(Grid g, const 
         acc2 += o[2 * cst];
     }
     const int64_t n = sol.at(i - 1, j - 1, k - 1);
+    if (fresh) {
+        sol.p[n] = acc0;
+        sol.p[sol.cs + n] = acc1;
+        sol.p[2 * sol.cs + n] = acc2;
+        return;
+    }
     sol.p[n] += acc0;
     sol.p[sol.cs + n] += acc1;
     sol.p[2 * sol.cs + n] += acc2;
@@ -426,17 +467,22 @@ __global__ void __launch_bounds__(64 * GATHER_WAVES) k_bsx_gather(Grid g, const 
 // Node lines p of the column's target face B (owned nodes, else 0), n < nC along C, ->
 // their half spectra: Bm[2 col][w][p] = Re, Bm[2 col + 1][w][p] = Im.
 template <int FFT>
-__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsxT_fwd(SpecFft f, WavePlan P, SpecTab t, const double2 *tw,
-                                                                  const SpecCol *cols, const SpecPair *pairs, Grid g,
-                                                                  GView gb, double *Bm) {
+__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsxT_fwd(const SpecJob *__restrict__ jobs, int nj,
+                                                                  const SpecPair *pairs, Grid g, GView gb, double *Bm) {
 #pragma clang fp contract(off)
     extern __shared__ double2 lds[];
     constexpr int NT = bsx_threads<FFT>();
+    SPEC_JOB(fwd0)
+    const SpecFft &f = J.f;
+    const WavePlan &P = J.wf;
+    const SpecTab &t = J.t;
+    const double2 *tw = J.tw;
+    Bm += J.b_off;
     const int L = f.L, np = FFT == -2 ? f.npairs : BW_WAVES, nl = 2 * np;
     double2 *A = lds, *twl = lds + np * L;
     double *Ad = (double *)A;
-    const int tid = threadIdx.x, p0 = blockIdx.x * nl, col = blockIdx.y;
-    const SpecCol cd = cols[col];
+    const int tid = threadIdx.x, col = local / J.gf, p0 = (local - col * J.gf) * nl;
+    const SpecCol cd = J.cols[col];
     const SpecPair PP = pairs[cd.pair];
     const int B = cd.pair / 6, ax = B >> 1, hi = B & 1;
     const double *src = gb.p + (int64_t)cd.comp * gb.cs;
@@ -473,16 +519,21 @@ __global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsxT_fwd(SpecFft f, Wave
 // first nC - 1 outputs (source cells along C) -> apart[B][comp][s] at the source's index in
 // face A's array (every (B, A) column writes its own slice, so no two columns meet).
 template <int FFT>
-__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsxT_inv(SpecFft f, WavePlan P, SpecTab t, const double2 *tw,
-                                                                  const SpecCol *cols, const double *Cm, int64_t ns,
-                                                                  double *apart) {
+__global__ void __launch_bounds__(bsx_threads<FFT>()) k_bsxT_inv(const SpecJob *__restrict__ jobs, int nj,
+                                                                  const double *Cm, int64_t ns, double *apart) {
 #pragma clang fp contract(off)
     extern __shared__ double2 lds[];
     constexpr int NT = bsx_threads<FFT>();
+    SPEC_JOB(inv0)
+    const SpecFft &f = J.f;
+    const WavePlan &P = J.wf;
+    const SpecTab &t = J.t;
+    const double2 *tw = J.tw;
+    Cm += J.c_off;
     const int L = f.L, np = FFT == -2 ? f.npairs : BW_WAVES, nl = 2 * np;
     double2 *A = lds, *twl = lds + np * L;
-    const int tid = threadIdx.x, q0 = blockIdx.x * nl, col = blockIdx.y;
-    const SpecCol cd = cols[col];
+    const int tid = threadIdx.x, col = local / J.gi, q0 = (local - col * J.gi) * nl;
+    const SpecCol cd = J.cols[col];
     const int64_t cst = (int64_t)t.nw * t.K;
     const double *in = Cm + 2 * col * cst;
     for (int i = tid; i < L; i += NT) twl[i] = tw[i];
@@ -545,7 +596,18 @@ struct SpecTable {
     int64_t b_off = 0, c_off = 0, o_off = 0;  // column 0 in Bm, Cm (real and imaginary columns) and Ores
 };
 
+// The launches of one direction: the jobs by form of their transforms (0, -1, -2) and, for the
+// parallel families' convolutions, by theirs (0: 576 points, 1: the runtime plan).
+struct SpecLaunch {
+    struct Part {
+        int first = 0, n = 0, fwd = 0, inv = 0;  // jobs, work-groups
+        size_t lds = 0;
+    } form[3], conv[2];
+    SpecJob *jobs = nullptr, *qjobs = nullptr;
+};
+
 struct SpecPlan {
+    SpecLaunch run[2];  // the sums and their transpose
     int n[3] = {0, 0, 0};
     double h[3] = {0, 0, 0};
     std::vector<SpecTable> tabs;
@@ -563,6 +625,10 @@ static void free_plan(SpecPlan *P) {
         if (T.G) (void)hipFree(T.G);
         if (T.T2) (void)hipFree(T.T2);
         if (T.cols_d) (void)hipFree(T.cols_d);
+    }
+    for (auto &R : P->run) {
+        if (R.jobs) (void)hipFree(R.jobs);
+        if (R.qjobs) (void)hipFree(R.qjobs);
     }
     if (P->pairs_d) (void)hipFree(P->pairs_d);
     if (P->Bm) (void)hipFree(P->Bm);
@@ -822,54 +888,145 @@ static int get_plan(Ctx *c, const Grid &g, int slot, SpecPlan **out) {
     return VPMX_OK;
 }
 
-int boundary_sums_spectral(Ctx *c, const Grid &g, int64_t ns, const double *a, GView sol, int slot) {
-    SpecPlan *P = nullptr;
-    VPMX_TRY(get_plan(c, g, slot, &P));
-    for (auto &T : P->tabs) {
-        const int np = T.form == -2 ? T.f.npairs : BW_WAVES, nl = 2 * np, ncol = (int)T.cols.size();
-        const size_t lds = sizeof(double2) * (size_t)(np + 1) * T.t.L;
-        const dim3 gf((unsigned)((T.t.K + nl - 1) / nl), (unsigned)ncol), gi((unsigned)((T.t.M + nl - 1) / nl), (unsigned)ncol);
-        if (T.form == 0)
-            hipLaunchKernelGGL(k_bsx_fwd<0>, gf, dim3(bsx_threads<0>()), lds, c->stream, T.f, T.wf, T.t, T.tw, T.cols_d,
-                               a, ns, P->Bm + T.b_off);
-        else if (T.form == -1)
-            hipLaunchKernelGGL(k_bsx_fwd<-1>, gf, dim3(bsx_threads<-1>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               T.cols_d, a, ns, P->Bm + T.b_off);
+// The launches of direction `tr` (0 the sums, 1 their transpose, which exchanges M and K), built
+// on first use.
+static int get_launch(Ctx *c, SpecPlan *P, int tr, SpecLaunch **out) {
+    SpecLaunch &R = P->run[tr];
+    *out = &R;
+    if (R.jobs) return VPMX_OK;
+    SpecLaunch L;
+    std::vector<SpecJob> jobs, qjobs;
+    auto job = [&](const SpecTable &T, int64_t bo, int64_t co) {
+        SpecJob J{};
+        J.f = T.f;
+        J.wf = T.wf;
+        J.wq = T.wq;
+        J.t = T.t;
+        J.tw = T.tw;
+        J.twq = T.twq;
+        J.T2 = T.T2;
+        J.cols = T.cols_d;
+        J.b_off = bo;
+        J.c_off = co;
+        J.o_off = T.o_off;
+        J.ncol = (int)T.cols.size();
+        return J;
+    };
+    for (int q = 0; q < 3; q++) {
+        auto &F = L.form[q];
+        F.first = (int)jobs.size();
+        int64_t bo = 0, co = 0;
+        for (auto &T : P->tabs) {
+            const int64_t b = tr ? bo : T.b_off, o = tr ? co : T.c_off;
+            bo += 2 * (int64_t)T.cols.size() * T.t.nw * T.t.M;
+            co += 2 * (int64_t)T.cols.size() * T.t.nw * T.t.K;
+            if (T.form != -q) continue;
+            SpecJob J = job(T, b, o);
+            const int np = q == 2 ? T.f.npairs : BW_WAVES, nl = 2 * np;
+            J.gf = ((tr ? T.t.M : T.t.K) + nl - 1) / nl;
+            J.gi = ((tr ? T.t.K : T.t.M) + nl - 1) / nl;
+            J.fwd0 = F.fwd;
+            J.inv0 = F.inv;
+            F.fwd += J.gf * J.ncol;
+            F.inv += J.gi * J.ncol;
+            const size_t lds = sizeof(double2) * (size_t)(np + 1) * T.t.L;
+            F.lds = lds > F.lds ? lds : F.lds;
+            jobs.push_back(J);
+        }
+        F.n = (int)jobs.size() - F.first;
+    }
+    for (int q = 0; q < 2; q++) {
+        auto &F = L.conv[q];
+        F.first = (int)qjobs.size();
+        int64_t bo = 0, co = 0;
+        for (auto &T : P->tabs) {
+            const int64_t b = tr ? bo : T.b_off, o = tr ? co : T.c_off;
+            bo += 2 * (int64_t)T.cols.size() * T.t.nw * T.t.M;
+            co += 2 * (int64_t)T.cols.size() * T.t.nw * T.t.K;
+            if (T.t.type != 1 || T.wq.L <= 0 || (T.t.Lq == 576 ? 0 : 1) != q) continue;
+            SpecJob J = job(T, b, o);
+            if (tr) std::swap(J.t.M, J.t.K);
+            J.q0 = F.fwd;
+            F.fwd += (J.ncol * T.t.nw + QC_WAVES - 1) / QC_WAVES;
+            const size_t lds = sizeof(double2) * (size_t)(QC_WAVES + 1) * T.t.Lq;
+            F.lds = lds > F.lds ? lds : F.lds;
+            qjobs.push_back(J);
+        }
+        F.n = (int)qjobs.size() - F.first;
+    }
+    VPMX_HIP(c, hipMalloc((void **)&L.qjobs, sizeof(SpecJob) * (qjobs.size() + 1)));
+    if (hipMalloc((void **)&L.jobs, sizeof(SpecJob) * (jobs.size() + 1)) != hipSuccess) {
+        (void)hipFree(L.qjobs);
+        return fail(c, VPMX_ERR_HIP, "spectral boundary sums: hipMalloc");
+    }
+    R = L;
+    VPMX_HIP(c, hipMemcpy(R.jobs, jobs.data(), sizeof(SpecJob) * jobs.size(), hipMemcpyHostToDevice));
+    if (!qjobs.empty()) VPMX_HIP(c, hipMemcpy(R.qjobs, qjobs.data(), sizeof(SpecJob) * qjobs.size(), hipMemcpyHostToDevice));
+    return VPMX_OK;
+}
+
+// The parallel families' convolutions; the ones too long for a wave each run the work-group form.
+static int run_convs(Ctx *c, SpecPlan *P, const SpecLaunch &R, int tr, const double *Bm, double *Cm) {
+    for (int q = 0; q < 2; q++) {
+        const auto &F = R.conv[q];
+        if (!F.n) continue;
+        if (q == 0)
+            hipLaunchKernelGGL(k_bsx_qconv_w<0>, dim3((unsigned)F.fwd), dim3(64 * QC_WAVES), F.lds, c->stream,
+                               R.qjobs + F.first, F.n, Bm, Cm, tr);
         else
-            hipLaunchKernelGGL(k_bsx_fwd<-2>, gf, dim3(bsx_threads<-2>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               T.cols_d, a, ns, P->Bm + T.b_off);
+            hipLaunchKernelGGL(k_bsx_qconv_w<-1>, dim3((unsigned)F.fwd), dim3(64 * QC_WAVES), F.lds, c->stream,
+                               R.qjobs + F.first, F.n, Bm, Cm, tr);
         VPMX_HIP(c, hipGetLastError());
-        if (T.t.type == 1 && T.wq.L > 0) {
-            const size_t ldsq = sizeof(double2) * (size_t)(QC_WAVES + 1) * T.t.Lq;
-            const int nseq = ncol * T.t.nw;
-            const dim3 gq((unsigned)((nseq + QC_WAVES - 1) / QC_WAVES));
-            if (T.t.Lq == 576)
-                hipLaunchKernelGGL(k_bsx_qconv_w<0>, gq, dim3(64 * QC_WAVES), ldsq, c->stream, T.wq, T.t, T.twq, T.T2,
-                                   P->Bm + T.b_off, P->Cm + T.c_off, ncol, 0);
-            else
-                hipLaunchKernelGGL(k_bsx_qconv_w<-1>, gq, dim3(64 * QC_WAVES), ldsq, c->stream, T.wq, T.t, T.twq, T.T2,
-                                   P->Bm + T.b_off, P->Cm + T.c_off, ncol, 0);
-            VPMX_HIP(c, hipGetLastError());
-        } else if (T.t.type == 1) {
+    }
+    int64_t bo = 0, co = 0;
+    for (auto &T : P->tabs) {
+        const int ncol = (int)T.cols.size();
+        const double *b = Bm + (tr ? bo : T.b_off);
+        double *o = Cm + (tr ? co : T.c_off);
+        bo += 2 * (int64_t)ncol * T.t.nw * T.t.M;
+        co += 2 * (int64_t)ncol * T.t.nw * T.t.K;
+        if (T.t.type == 1 && T.wq.L <= 0) {
+            SpecTab t = T.t;
+            if (tr) std::swap(t.M, t.K);
             const size_t ldsq = sizeof(double2) * (size_t)(T.fq.npairs + 1) * T.t.Lq;
             hipLaunchKernelGGL(k_bsx_qconv, dim3((unsigned)((T.t.nw + T.fq.npairs - 1) / T.fq.npairs), (unsigned)ncol),
-                               dim3(DST_THREADS), ldsq, c->stream, T.fq, T.t, T.twq, T.T2, P->Bm + T.b_off,
-                               P->Cm + T.c_off, 0);
+                               dim3(DST_THREADS), ldsq, c->stream, T.fq, t, T.twq, T.T2, b, o, tr);
             VPMX_HIP(c, hipGetLastError());
-        } else {
+        } else if (T.t.type == 0 && !tr) {
             // per frequency w: C_w (M x 2 ncol) = G_w (M x K) B_w (K x 2 ncol)
-            VPMX_TRY(dgemm(c, false, false, T.t.M, 2 * ncol, T.t.K, T.G, T.t.M, (int64_t)T.t.M * T.t.K,
-                           P->Bm + T.b_off, T.t.nw * T.t.K, T.t.K, P->Cm + T.c_off, T.t.nw * T.t.M, T.t.M, T.t.nw));
+            VPMX_TRY(dgemm(c, false, false, T.t.M, 2 * ncol, T.t.K, T.G, T.t.M, (int64_t)T.t.M * T.t.K, b,
+                           T.t.nw * T.t.K, T.t.K, o, T.t.nw * T.t.M, T.t.M, T.t.nw));
+        } else if (T.t.type == 0) {
+            // per frequency w: C_w (K x 2 ncol) = G_w^T (K x M) B_w (M x 2 ncol)
+            VPMX_TRY(dgemm(c, true, false, T.t.K, 2 * ncol, T.t.M, T.G, T.t.M, (int64_t)T.t.M * T.t.K, b,
+                           T.t.nw * T.t.M, T.t.M, o, T.t.nw * T.t.K, T.t.K, T.t.nw));
         }
-        if (T.form == 0)
-            hipLaunchKernelGGL(k_bsx_inv<0>, gi, dim3(bsx_threads<0>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               P->Cm + T.c_off, P->Ores, T.o_off);
-        else if (T.form == -1)
-            hipLaunchKernelGGL(k_bsx_inv<-1>, gi, dim3(bsx_threads<-1>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               P->Cm + T.c_off, P->Ores, T.o_off);
-        else
-            hipLaunchKernelGGL(k_bsx_inv<-2>, gi, dim3(bsx_threads<-2>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               P->Cm + T.c_off, P->Ores, T.o_off);
+    }
+    return VPMX_OK;
+}
+
+int boundary_sums_spectral(Ctx *c, const Grid &g, int64_t ns, const double *a, GView sol, int slot, bool fresh) {
+    SpecPlan *P = nullptr;
+    VPMX_TRY(get_plan(c, g, slot, &P));
+    SpecLaunch *R = nullptr;
+    VPMX_TRY(get_launch(c, P, 0, &R));
+    for (int q = 0; q < 3; q++) {
+        const auto &F = R->form[q];
+        if (!F.n) continue;
+        const SpecJob *j = R->jobs + F.first;
+        if (q == 0) hipLaunchKernelGGL(k_bsx_fwd<0>, dim3((unsigned)F.fwd), dim3(bsx_threads<0>()), F.lds, c->stream, j, F.n, a, ns, P->Bm);
+        else if (q == 1) hipLaunchKernelGGL(k_bsx_fwd<-1>, dim3((unsigned)F.fwd), dim3(bsx_threads<-1>()), F.lds, c->stream, j, F.n, a, ns, P->Bm);
+        else hipLaunchKernelGGL(k_bsx_fwd<-2>, dim3((unsigned)F.fwd), dim3(bsx_threads<-2>()), F.lds, c->stream, j, F.n, a, ns, P->Bm);
+        VPMX_HIP(c, hipGetLastError());
+    }
+    VPMX_TRY(run_convs(c, P, *R, 0, P->Bm, P->Cm));
+    for (int q = 0; q < 3; q++) {
+        const auto &F = R->form[q];
+        if (!F.n) continue;
+        const SpecJob *j = R->jobs + F.first;
+        if (q == 0) hipLaunchKernelGGL(k_bsx_inv<0>, dim3((unsigned)F.inv), dim3(bsx_threads<0>()), F.lds, c->stream, j, F.n, P->Cm, P->Ores);
+        else if (q == 1) hipLaunchKernelGGL(k_bsx_inv<-1>, dim3((unsigned)F.inv), dim3(bsx_threads<-1>()), F.lds, c->stream, j, F.n, P->Cm, P->Ores);
+        else hipLaunchKernelGGL(k_bsx_inv<-2>, dim3((unsigned)F.inv), dim3(bsx_threads<-2>()), F.lds, c->stream, j, F.n, P->Cm, P->Ores);
         VPMX_HIP(c, hipGetLastError());
     }
     int maxp = 0;
@@ -880,7 +1037,7 @@ int boundary_sums_spectral(Ctx *c, const Grid &g, int64_t ns, const double *a, G
         maxp = np > maxp ? np : maxp;
     }
     hipLaunchKernelGGL(k_bsx_gather, dim3((unsigned)((maxp + GATHER_WAVES - 1) / GATHER_WAVES), 6u),
-                       dim3(64 * GATHER_WAVES), 0, c->stream, g, P->pairs_d, P->Ores, sol);
+                       dim3(64 * GATHER_WAVES), 0, c->stream, g, P->pairs_d, P->Ores, sol, fresh ? 1 : 0);
     VPMX_HIP(c, hipGetLastError());
     // FP64 work of the call: the real products and q convolutions, plus ~5 L log2 L flops per
     // complex FFT along C
@@ -896,6 +1053,8 @@ int boundary_sums_spectral(Ctx *c, const Grid &g, int64_t ns, const double *a, G
 int boundary_sums_spectral_adj(Ctx *c, const Grid &g, int64_t ns, GView gb, double *abar, int slot) {
     SpecPlan *P = nullptr;
     VPMX_TRY(get_plan(c, g, slot, &P));
+    SpecLaunch *R = nullptr;
+    VPMX_TRY(get_launch(c, P, 1, &R));
     int64_t nbT = 0, ncT = 0;
     for (auto &T : P->tabs) {
         const int64_t N = (int64_t)T.cols.size();
@@ -915,60 +1074,23 @@ int boundary_sums_spectral_adj(Ctx *c, const Grid &g, int64_t ns, GView gb, doub
         VPMX_HIP(c, hipMalloc((void **)&P->apart, sizeof(double) * 18 * (size_t)ns));
         P->apart_ns = ns;
     }
-    int64_t bo = 0, co = 0;
-    for (auto &T : P->tabs) {
-        const int np = T.form == -2 ? T.f.npairs : BW_WAVES, nl = 2 * np, ncol = (int)T.cols.size();
-        const size_t lds = sizeof(double2) * (size_t)(np + 1) * T.t.L;
-        double *Bm = P->BmT + bo, *Cm = P->CmT + co;
-        bo += 2 * (int64_t)ncol * T.t.nw * T.t.M;
-        co += 2 * (int64_t)ncol * T.t.nw * T.t.K;
-        const dim3 gf((unsigned)((T.t.M + nl - 1) / nl), (unsigned)ncol), gi((unsigned)((T.t.K + nl - 1) / nl), (unsigned)ncol);
-        if (T.form == 0)
-            hipLaunchKernelGGL(k_bsxT_fwd<0>, gf, dim3(bsx_threads<0>()), lds, c->stream, T.f, T.wf, T.t, T.tw, T.cols_d,
-                               P->pairs_d, g, gb, Bm);
-        else if (T.form == -1)
-            hipLaunchKernelGGL(k_bsxT_fwd<-1>, gf, dim3(bsx_threads<-1>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               T.cols_d, P->pairs_d, g, gb, Bm);
-        else
-            hipLaunchKernelGGL(k_bsxT_fwd<-2>, gf, dim3(bsx_threads<-2>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               T.cols_d, P->pairs_d, g, gb, Bm);
+    for (int q = 0; q < 3; q++) {
+        const auto &F = R->form[q];
+        if (!F.n) continue;
+        const SpecJob *j = R->jobs + F.first;
+        if (q == 0) hipLaunchKernelGGL(k_bsxT_fwd<0>, dim3((unsigned)F.fwd), dim3(bsx_threads<0>()), F.lds, c->stream, j, F.n, P->pairs_d, g, gb, P->BmT);
+        else if (q == 1) hipLaunchKernelGGL(k_bsxT_fwd<-1>, dim3((unsigned)F.fwd), dim3(bsx_threads<-1>()), F.lds, c->stream, j, F.n, P->pairs_d, g, gb, P->BmT);
+        else hipLaunchKernelGGL(k_bsxT_fwd<-2>, dim3((unsigned)F.fwd), dim3(bsx_threads<-2>()), F.lds, c->stream, j, F.n, P->pairs_d, g, gb, P->BmT);
         VPMX_HIP(c, hipGetLastError());
-        if (T.t.type == 1) {
-            // the q correlation: the forward's convolution with M and K exchanged and the
-            // conjugate spectrum
-            SpecTab tT = T.t;
-            tT.M = T.t.K;
-            tT.K = T.t.M;
-            if (T.wq.L > 0) {
-                const size_t ldsq = sizeof(double2) * (size_t)(QC_WAVES + 1) * T.t.Lq;
-                const int nseq = ncol * T.t.nw;
-                const dim3 gq((unsigned)((nseq + QC_WAVES - 1) / QC_WAVES));
-                if (T.t.Lq == 576)
-                    hipLaunchKernelGGL(k_bsx_qconv_w<0>, gq, dim3(64 * QC_WAVES), ldsq, c->stream, T.wq, tT, T.twq, T.T2,
-                                       Bm, Cm, ncol, 1);
-                else
-                    hipLaunchKernelGGL(k_bsx_qconv_w<-1>, gq, dim3(64 * QC_WAVES), ldsq, c->stream, T.wq, tT, T.twq,
-                                       T.T2, Bm, Cm, ncol, 1);
-            } else {
-                const size_t ldsq = sizeof(double2) * (size_t)(T.fq.npairs + 1) * T.t.Lq;
-                hipLaunchKernelGGL(k_bsx_qconv, dim3((unsigned)((T.t.nw + T.fq.npairs - 1) / T.fq.npairs), (unsigned)ncol),
-                                   dim3(DST_THREADS), ldsq, c->stream, T.fq, tT, T.twq, T.T2, Bm, Cm, 1);
-            }
-            VPMX_HIP(c, hipGetLastError());
-        } else {
-            // per frequency w: C_w (K x 2 ncol) = G_w^T (K x M) B_w (M x 2 ncol)
-            VPMX_TRY(dgemm(c, true, false, T.t.K, 2 * ncol, T.t.M, T.G, T.t.M, (int64_t)T.t.M * T.t.K, Bm,
-                           T.t.nw * T.t.M, T.t.M, Cm, T.t.nw * T.t.K, T.t.K, T.t.nw));
-        }
-        if (T.form == 0)
-            hipLaunchKernelGGL(k_bsxT_inv<0>, gi, dim3(bsx_threads<0>()), lds, c->stream, T.f, T.wf, T.t, T.tw, T.cols_d,
-                               Cm, ns, P->apart);
-        else if (T.form == -1)
-            hipLaunchKernelGGL(k_bsxT_inv<-1>, gi, dim3(bsx_threads<-1>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               T.cols_d, Cm, ns, P->apart);
-        else
-            hipLaunchKernelGGL(k_bsxT_inv<-2>, gi, dim3(bsx_threads<-2>()), lds, c->stream, T.f, T.wf, T.t, T.tw,
-                               T.cols_d, Cm, ns, P->apart);
+    }
+    VPMX_TRY(run_convs(c, P, *R, 1, P->BmT, P->CmT));
+    for (int q = 0; q < 3; q++) {
+        const auto &F = R->form[q];
+        if (!F.n) continue;
+        const SpecJob *j = R->jobs + F.first;
+        if (q == 0) hipLaunchKernelGGL(k_bsxT_inv<0>, dim3((unsigned)F.inv), dim3(bsx_threads<0>()), F.lds, c->stream, j, F.n, P->CmT, ns, P->apart);
+        else if (q == 1) hipLaunchKernelGGL(k_bsxT_inv<-1>, dim3((unsigned)F.inv), dim3(bsx_threads<-1>()), F.lds, c->stream, j, F.n, P->CmT, ns, P->apart);
+        else hipLaunchKernelGGL(k_bsxT_inv<-2>, dim3((unsigned)F.inv), dim3(bsx_threads<-2>()), F.lds, c->stream, j, F.n, P->CmT, ns, P->apart);
         VPMX_HIP(c, hipGetLastError());
     }
     hipLaunchKernelGGL(k_bsxT_reduce, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, c->stream, ns, P->apart, abar);

@@ -427,6 +427,41 @@ int coarse_laplacian(Ctx *c, int ncomp, const int cn[3], const int lo[3], const 
     return VPMX_OK;
 }
 
+__global__ void k_coarse_problem(int ncomp, int nx, int ny, int nz, int lx, int ly, int lz, int hx, int hy, int hz, int nc,
+                                 double c0, double c1, double c2, GView fine, GView samp, GView rhs) {
+#pragma clang fp contract(off)
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)nx * ny * nz) return;
+    const int i = (int)(t % nx) + 1, j = (int)((t / nx) % ny) + 1, k = (int)(t / ((int64_t)nx * ny)) + 1;
+    const bool on = i >= lx && i <= hx && j >= ly && j <= hy && k >= lz && k <= hz;
+    const bool in = i > lx && i < hx && j > ly && j < hy && k > lz && k < hz;
+    const int64_t o = rhs.at(i - 1, j - 1, k - 1), os = samp.at(i - 1, j - 1, k - 1);
+    const int64_t of = on ? fine.at((i - lx) * nc, (j - ly) * nc, (k - lz) * nc) : 0;
+    const int64_t dy = nc * fine.py, dz = nc * fine.pz;
+    for (int q = 0; q < ncomp; q++) {
+        const double *F = fine.p + q * fine.cs + of;
+        const double sc = on ? F[0] : 0.0;
+        double v = 0.0;
+        if (in) {
+            const double ax = ((F[nc] - 2 * sc) + F[-nc]) / c0;
+            const double ay = ((F[dy] - 2 * sc) + F[-dy]) / c1;
+            const double az = ((F[dz] - 2 * sc) + F[-dz]) / c2;
+            v = 0.0 + ((ax + ay) + az);
+        }
+        samp.p[q * samp.cs + os] = sc;
+        rhs.p[q * rhs.cs + o] = v;
+    }
+}
+int coarse_problem(Ctx *c, int ncomp, const int cn[3], const int lo[3], const int hi[3], int nc, const double hc[3],
+                   GView fine, GView samp, GView rhs) {
+    const int64_t nt = (int64_t)cn[0] * cn[1] * cn[2];
+    hipLaunchKernelGGL(k_coarse_problem, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, c->stream, ncomp, cn[0], cn[1],
+                       cn[2], lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], nc, hc[0] * hc[0], hc[1] * hc[1], hc[2] * hc[2],
+                       fine, samp, rhs);
+    VPMX_HIP(c, hipGetLastError());
+    return VPMX_OK;
+}
+
 __device__ __forceinline__ double tsc(double x) {
 #pragma clang fp contract(off)
     double a = fabs(x);

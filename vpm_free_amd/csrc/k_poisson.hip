@@ -2453,7 +2453,7 @@ static int partial_values(Ctx *c, const DstArgs &a, int ncomp, bool f32, const S
 }
 
 int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GView rhs, const GView *bc, GView out,
-                      int reuse, int form, double *face_nd, const SolvePartial *part) {
+                      int reuse, int form, double *face_nd, const SolvePartial *part, bool skip_faces) {
     int st = VPMX_OK;
     int m[3] = {wn[0] - 2, wn[1] - 2, wn[2] - 2};
     if (m[0] < 1 || m[1] < 1 || m[2] < 1) return fail(c, VPMX_ERR_ARG, "Poisson window needs >= 3 nodes per axis");
@@ -2588,7 +2588,7 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
         if (mm(0, fi)) VPMX_TRY(dstm_x_inv(c, di, a.w, out));
         else VPMX_TRY(run_pass<DST_XI>(c, a, ncomp, ax[0], fi));
     }
-    if (!bc) VPMX_TRY(zero_faces(c, wn, out, ncomp));
+    if (!bc && !skip_faces) VPMX_TRY(zero_faces(c, wn, out, ncomp));
     return VPMX_OK;
 }
 

@@ -99,8 +99,9 @@ static void collect_times(Ctx *, const bool *) {}
 // SOL(faces) += boundary sums (ibctyp 2 point sources, 3 panels; tree form with levmax
 // levels when levmax >= 0, pmlib.f90:69 ibctyp/itree/levmax), then the Dirichlet solve of
 // the whole grid.
+// fresh: sol counts as zero whatever it holds; its faces and (without part) interior are written.
 static int pmesh_inf(Ctx *c, const Grid &g, GView rhs, GView sol, DBuf &s0buf, bool fine, int levmax, int ibctyp,
-                     const SolvePartial *part = nullptr) {
+                     bool fresh, const SolvePartial *part = nullptr) {
     int st = VPMX_OK;
     const int n[3] = {g.n[0], g.n[1], g.n[2]};
     int64_t G = (int64_t)n[0] * n[1] * n[2];
@@ -125,11 +126,11 @@ static int pmesh_inf(Ctx *c, const Grid &g, GView rhs, GView sol, DBuf &s0buf, b
         VPMX_TRY(poisson_dirichlet(c, 3, n, h, rhs, nullptr, s0v, ru, SOLVE_CTX, fd));  // keeps its forward transforms
         VPMX_TRY(normal_derivs_cells(c, 3, g, fd, sig, cxyz, wgt, &nb));
     } else {
-        VPMX_TRY(poisson_dirichlet(c, 3, n, h, rhs, nullptr, s0v, ru));  // keeps its forward transforms
-        VPMX_TRY(normal_derivs(c, 3, g, s0v, sig, cxyz, wgt, &nb));
+        VPMX_TRY(poisson_dirichlet(c, 3, n, h, rhs, nullptr, s0v, ru, SOLVE_CTX, nullptr, nullptr, true));  // keeps its forward transforms
+        VPMX_TRY(normal_derivs(c, 3, g, s0v, sig, cxyz, wgt, &nb, true));
     }
     // SOL_0 is dead once the sources exist: scratch of the panel sums
-    VPMX_TRY(boundary_sums(c, 3, g, nb, sig, cxyz, wgt, sol, fine, levmax, ibctyp, &s0v));
+    VPMX_TRY(boundary_sums(c, 3, g, nb, sig, cxyz, wgt, sol, fine, levmax, ibctyp, &s0v, fresh));
     // same RHS: reuses them (part: only the nodes the caller reads)
     VPMX_TRY(poisson_dirichlet(c, 3, n, h, rhs, &sol, sol, 2 * ru, SOLVE_CTX, nullptr, part));
     return VPMX_OK;
@@ -172,8 +173,7 @@ static int yaps_single(Ctx *c, bool *used) {
     Grid gb = make_grid(G.nnbl, &G.xbound_bl[0], G.dpm);
     // 1. fine infinite-domain solve over the whole block
     mark(c, ST_FINE, 0, true);
-    // the boundary sums accumulate on the faces; the second solve writes every interior node
-    VPMX_TRY(zero_faces(c, nb, sv));
+    // the boundary sums write the faces; the second solve writes every interior node
     c->dst_timed_m = gb.n[1] - 2;  // the block's y lines are the timed sine-transform passes
     // tree levels: ilevmax on the block, ilevmax-1 on the coarse grid (yaps3d.f90:46-48, 286-292)
     const bool tree = P.iyntree == 1;
@@ -195,7 +195,7 @@ static int yaps_single(Ctx *c, bool *used) {
                          part.ys[0] < part.ys[1] && part.zs[0] < part.zs[1] && part.xs[1] == nb[0] + 1 - part.xs[0] &&
                          part.ys[1] == nb[1] + 1 - part.ys[0] && nb[0] <= 322 && P.ncoarse >= 1;
     const bool use_part = part_ok && (c->fine_partial == 1 || (c->fine_partial < 0 && B >= SPECTRAL_MIN_NODES));
-    VPMX_TRY(pmesh_inf(c, gb, rv, sv, c->sol0, true, tree ? G.ilevmax : -1, P.ibctyp, use_part ? &part : nullptr));
+    VPMX_TRY(pmesh_inf(c, gb, rv, sv, c->sol0, true, tree ? G.ilevmax : -1, P.ibctyp, true, use_part ? &part : nullptr));
     mark(c, ST_FINE, 1);
     used[ST_FINE] = used[ST_BOUNDS] = true;
     // 2. coarse correction
@@ -223,15 +223,12 @@ static int yaps_single(Ctx *c, bool *used) {
         // the reference records NN_coarse_map at i = 1 and i = NNbl; with (NNbl-1) a multiple
         // of ncoarse the last sample is i = NNbl
     }
-    int *cmap_d = nullptr;
-    VPMX_TRY(upload_cmap(c, cmap, &cmap_d));
     GView smv = view(samp, cn), rcv = view(rhsc, cn), scv = view(solc, cn);
-    VPMX_TRY(fill(c, samp, 3 * GC, 0.0));
-    VPMX_TRY(coarse_sample(c, 3, ns, ncs, cmap_d, sv, smv, cn));
-    VPMX_TRY(coarse_laplacian(c, 3, cn, fp_lo, fp_hi, G.dpm_coarse, smv, rcv));
-    VPMX_TRY(fill(c, solc, 3 * GC, 0.0));
+    for (int d = 0; d < 3; d++)
+        if (fp_hi[d] - fp_lo[d] != ns[d] - 1) return fail(c, VPMX_ERR_STATE, "block samples are not consecutive coarse nodes");
+    VPMX_TRY(coarse_problem(c, 3, cn, fp_lo, fp_hi, ncs, G.dpm_coarse, sv, smv, rcv));
     Grid gc = make_grid(G.nn_coarse, G.xbound_coarse, G.dpm_coarse);
-    VPMX_TRY(pmesh_inf(c, gc, rcv, scv, c->sol0_c, false, tree ? G.ilevmax - 1 : -1, P.ibctyp));
+    VPMX_TRY(pmesh_inf(c, gc, rcv, scv, c->sol0_c, false, tree ? G.ilevmax - 1 : -1, P.ibctyp, true));
     mark(c, ST_COARSE, 1);
     used[ST_COARSE] = true;
     // 3. TSC correction of the inner-box faces
@@ -298,11 +295,10 @@ static int yaps_multi(Ctx *c, bool *used) {
         return fail(c, VPMX_ERR_UNSUP, "tree = 1 needs at least one level on the coarse grid (ilevmax >= 1)");
     // 1. fine infinite-domain solves
     mark(c, ST_FINE, 0);
-    VPMX_TRY(fill(c, sol_bl, tot, 0.0));
     c->dst_timed_m = G.nnbl[1] - 2;
     for (int b = 0; b < NB; b++) {
         Grid gb = make_grid(block_n(G, b), &G.xbound_bl[6 * b], G.dpm);
-        VPMX_TRY(pmesh_inf(c, gb, bview(rhs_bl, b), bview(sol_bl, b), c->sol0, true, tree ? G.ilevmax : -1, P.ibctyp));
+        VPMX_TRY(pmesh_inf(c, gb, bview(rhs_bl, b), bview(sol_bl, b), c->sol0, true, tree ? G.ilevmax : -1, P.ibctyp, true));
     }
     mark(c, ST_FINE, 1);
     used[ST_FINE] = used[ST_BOUNDS] = true;
@@ -372,9 +368,8 @@ static int yaps_multi(Ctx *c, bool *used) {
         VPMX_TRY(coarse_laplacian(c, 3, cn, blk[b].fp_lo, blk[b].fp_hi, G.dpm_coarse, cview(samp, b), view(rhsc, cn),
                                   true));
     }
-    VPMX_TRY(fill(c, solc, 3 * GC, 0.0));
     Grid gc = make_grid(G.nn_coarse, G.xbound_coarse, G.dpm_coarse);
-    VPMX_TRY(pmesh_inf(c, gc, view(rhsc, cn), view(solc, cn), c->sol0_c, false, tree ? G.ilevmax - 1 : -1, P.ibctyp));
+    VPMX_TRY(pmesh_inf(c, gc, view(rhsc, cn), view(solc, cn), c->sol0_c, false, tree ? G.ilevmax - 1 : -1, P.ibctyp, true));
     mark(c, ST_COARSE, 1);
     used[ST_COARSE] = true;
     // 3. interp_stencil on every block's inner-box faces
@@ -1581,7 +1576,7 @@ int32_t vpmx_stage_pmesh_inf_lev(vpmx_ctx *p, const double xbound[6], const doub
     VPMX_TRY(aos_to_soa(c, nc, n, ra, view(ss, n)));
     Grid g = make_grid(nn, xbound, dpm);
     if (ibctyp != 2 && ibctyp != 3) return fail(c, VPMX_ERR_ARG, "ibctyp must be 2 or 3");
-    VPMX_TRY(pmesh_inf(c, g, view(rs, n), view(ss, n), c->sol0, true, itree == 1 ? levmax : -1, ibctyp));
+    VPMX_TRY(pmesh_inf(c, g, view(rs, n), view(ss, n), c->sol0, true, itree == 1 ? levmax : -1, ibctyp, false));
     VPMX_TRY(soa_to_aos(c, nc, nc, n, view(ss, n), 0.0, ra));
     VPMX_HIP(c, hipMemcpyAsync(sol, ra, sizeof(double) * nc * G, hipMemcpyDeviceToHost, c->stream));
     VPMX_HIP(c, hipStreamSynchronize(c->stream));

@@ -134,9 +134,10 @@ struct SolvePartial {
     int xs[2], ys[2], zs[2];
     int step;
 };
+// skip_faces: a zero-BC solve leaves the faces of `out` unwritten.
 int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GView rhs, const GView *bc,
                       GView out, int reuse = 0, int form = SOLVE_CTX, double *face_nd = nullptr,
-                      const SolvePartial *part = nullptr);
+                      const SolvePartial *part = nullptr, bool skip_faces = false);
 
 // Complex FFT plan of length L (Stockham radices, device twiddle table exp(-2 pi i t / L)),
 // cached per context.
@@ -147,8 +148,9 @@ struct FftShape {
 int fft_shape(Ctx *c, int L, FftShape *out);
 
 // Boundary (k_boundary.hip)
+// (zero_faces: s0 is zero on its faces, whose values are not read)
 int normal_derivs(Ctx *c, int ncomp, const Grid &g, GView s0, double *sig, double *cxyz, double *wgt,
-                  int64_t *nbound);
+                  int64_t *nbound, bool zero_faces = false);
 // The same in two steps: the face-node table (ncomp values per node of each face, faces XMIN,
 // XMAX, YMIN, YMAX, ZMIN, ZMAX, each ncomp x N0 x N1 with (N0, N1) = (NY, NZ), (NX, NZ),
 // (NX, NY), first index fastest; the context keeps its buffer), filled by the caller, then the
@@ -158,20 +160,23 @@ int normal_derivs_cells(Ctx *c, int ncomp, const Grid &g, const double *fd, doub
                         int64_t *nbound);
 // levmax >= 0: the tree form with that many levels (pm.inp tree = 1), else the direct sums;
 // ibctyp 2 point sources, 3 constant-source panels (needs `scratch`, a grid of sol's shape
-// whose boundary nodes it may overwrite, for the direct form).
+// whose boundary nodes it may overwrite, for the direct form).  fresh: sol's faces count as zero
+// whatever they hold (the spectral form then writes them instead of adding to them).
 int boundary_sums(Ctx *c, int ncomp, const Grid &g, int64_t nbound, const double *sig, const double *cxyz,
                   const double *wgt, GView sol, bool fine, int levmax = -1, int ibctyp = 2,
-                  const GView *scratch = nullptr);
+                  const GView *scratch = nullptr, bool fresh = false);
 // SOL(t) += sum_s a(c, s) / |x_t - x_s| over the face-cell centres (spectral / lattice /
 // direct evaluation by the context's setting).
-int point_sums(Ctx *c, const Grid &g, int64_t nbound, const double *cxyz, const double *a, GView sol, bool fine);
+int point_sums(Ctx *c, const Grid &g, int64_t nbound, const double *cxyz, const double *a, GView sol, bool fine,
+               bool fresh = false);
 // Panel sources (k_panel.hip), direct or tree form.
 int boundary_sums_panels(Ctx *c, const Grid &g, int64_t nb, const double *sig, const double *cxyz, const double *ds,
                          GView sol, bool fine, int levmax, GView scratch);
 // Spectral evaluation of the same sums (k_bspec.hip); returns VPMX_ERR_UNSUP when the
 // block's faces are too long for its in-LDS FFTs, so the caller can use the lattice kernel.
 // slot: 0 the fine block, 1 the coarse grid (each keeps its own plan across calls).
-int boundary_sums_spectral(Ctx *c, const Grid &g, int64_t nbound, const double *a, GView sol, int slot);
+int boundary_sums_spectral(Ctx *c, const Grid &g, int64_t nbound, const double *a, GView sol, int slot,
+                           bool fresh = false);
 // Its transpose: abar(c, s) = sum over boundary nodes t of gbar(c, t) / |x_t - x_s| (the adjoint
 // of the sources a); VPMX_ERR_UNSUP where the forward plan does not build.
 int boundary_sums_spectral_adj(Ctx *c, const Grid &g, int64_t nbound, GView gb, double *abar, int slot);
@@ -202,6 +207,10 @@ int coarse_sample(Ctx *c, int ncomp, const int nsamp[3], int nc, const int *cmap
                   const int cn[3]);
 int coarse_laplacian(Ctx *c, int ncomp, const int cn[3], const int lo[3], const int hi[3], const double hc[3],
                      GView samp, GView rhs, bool accumulate = false);
+// Samples (0 outside the footprint lo..hi, 1-based) and their Laplacian (0 outside its interior) on
+// every coarse node in one launch; coarse node lo + a holds the fine node a * nc of its axis.
+int coarse_problem(Ctx *c, int ncomp, const int cn[3], const int lo[3], const int hi[3], int nc, const double hc[3],
+                   GView fine, GView samp, GView rhs);
 struct InterpArgs {
     int nbl[6];           // inner box NNbl_bl (1-based)
     double xbl[3], h[3];  // block origin and fine spacing
