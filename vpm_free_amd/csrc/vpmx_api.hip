@@ -15,6 +15,7 @@
 #include <cstring>
 #include <vector>
 
+#include "transfer.h"
 #include "vpmx_ctx.h"
 #include "vpmx_internal.h"
 
@@ -610,8 +611,8 @@ static int upload_particles(Ctx *c, const double *xp, const double *qp, int64_t 
     ensure(c, c->up, sizeof(double) * 3 * (size_t)(n ? n : 1), &st); if (st) return st;
     ensure(c, c->gp, sizeof(double) * 3 * (size_t)(n ? n : 1), &st); if (st) return st;
     if (n) {
-        VPMX_HIP(c, hipMemcpyAsync(dx, xp, sizeof(double) * 3 * n, hipMemcpyHostToDevice, c->stream));
-        VPMX_HIP(c, hipMemcpyAsync(dq, qp, sizeof(double) * nr * n, hipMemcpyHostToDevice, c->stream));
+        const Copy q[2] = {{dx, xp, sizeof(double) * 3 * (size_t)n}, {dq, qp, sizeof(double) * nr * (size_t)n}};
+        VPMX_TRY(copy_in(c, q, 2));
     }
     c->np = n;
     c->neqpm = neqpm;
@@ -1161,6 +1162,7 @@ void vpmx_destroy(vpmx_ctx *p) {
         for (DBuf &b : ck) release(b);
     free_bspec(c);
     free_tree(c);
+    free_transfer(c);
     free_fft_plans(c);
     for (int k = 0; k < K_COUNT; k++) {
         for (hipEvent_t e : c->kev0[k]) (void)hipEventDestroy(e);
@@ -1279,8 +1281,9 @@ int32_t vpmx_vpm(vpmx_ctx *p, double *xp, double *qp, double *up, double *gp, in
     VPMX_TRY(run_vpm(c, whattodo, (const double *)c->xp.p, (const double *)c->qp.p, (double *)c->up.p,
                      (double *)c->gp.p, nvr, ni));
     if (whattodo == 2 || whattodo == 4 || whattodo == 5) {
-        if (up) VPMX_HIP(c, hipMemcpyAsync(up, c->up.p, sizeof(double) * 3 * nvr, hipMemcpyDeviceToHost, c->stream));
-        if (gp) VPMX_HIP(c, hipMemcpyAsync(gp, c->gp.p, sizeof(double) * 3 * nvr, hipMemcpyDeviceToHost, c->stream));
+        const size_t b = sizeof(double) * 3 * (size_t)nvr;
+        const Copy q[2] = {{up, c->up.p, up ? b : 0}, {gp, c->gp.p, gp ? b : 0}};
+        VPMX_TRY(copy_out(c, q, 2));
     }
     VPMX_HIP(c, hipStreamSynchronize(c->stream));
     return VPMX_OK;
@@ -1304,12 +1307,9 @@ int32_t vpmx_remesh_fetch(vpmx_ctx *p, double *xp_out, double *qp_out) {
     if (c->rm_count < 0) return fail(c, VPMX_ERR_STATE, "no remesh result to fetch");
     int nr = c->neqpm + 1;
     if (c->rm_count > 0) {
-        if (xp_out)
-            VPMX_HIP(c, hipMemcpyAsync(xp_out, c->rm_xp, sizeof(double) * 3 * c->rm_count, hipMemcpyDeviceToHost,
-                                       c->stream));
-        if (qp_out)
-            VPMX_HIP(c, hipMemcpyAsync(qp_out, c->rm_qp, sizeof(double) * nr * c->rm_count, hipMemcpyDeviceToHost,
-                                       c->stream));
+        const size_t m = sizeof(double) * (size_t)c->rm_count;
+        const Copy q[2] = {{xp_out, c->rm_xp, xp_out ? 3 * m : 0}, {qp_out, c->rm_qp, qp_out ? nr * m : 0}};
+        VPMX_TRY(copy_out(c, q, 2));
     }
     VPMX_HIP(c, hipStreamSynchronize(c->stream));
     return VPMX_OK;
@@ -1341,7 +1341,8 @@ int32_t vpmx_get_grid(vpmx_ctx *p, int32_t which, double *dst, int64_t capacity)
     } else {
         return fail(c, VPMX_ERR_ARG, "get_grid: which must be 0..3");
     }
-    VPMX_HIP(c, hipMemcpyAsync(dst, stage, sizeof(double) * ncd * GG, hipMemcpyDeviceToHost, c->stream));
+    const Copy q = {dst, stage, sizeof(double) * (size_t)ncd * (size_t)GG};
+    VPMX_TRY(copy_out(c, &q, 1));
     VPMX_HIP(c, hipStreamSynchronize(c->stream));
     return VPMX_OK;
 }
@@ -1368,10 +1369,10 @@ int32_t vpmx_particles_download(vpmx_ctx *p, double *xp, double *qp, double *up,
     int64_t n = c->np;
     int nr = c->neqpm + 1;
     if (n > 0) {
-        if (xp) VPMX_HIP(c, hipMemcpyAsync(xp, c->xp.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, c->stream));
-        if (qp) VPMX_HIP(c, hipMemcpyAsync(qp, c->qp.p, sizeof(double) * nr * n, hipMemcpyDeviceToHost, c->stream));
-        if (up) VPMX_HIP(c, hipMemcpyAsync(up, c->up.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, c->stream));
-        if (gp) VPMX_HIP(c, hipMemcpyAsync(gp, c->gp.p, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, c->stream));
+        const size_t m = sizeof(double) * (size_t)n;
+        const Copy q[4] = {{xp, c->xp.p, xp ? 3 * m : 0}, {qp, c->qp.p, qp ? nr * m : 0},
+                           {up, c->up.p, up ? 3 * m : 0}, {gp, c->gp.p, gp ? 3 * m : 0}};
+        VPMX_TRY(copy_out(c, q, 4));
     }
     VPMX_HIP(c, hipStreamSynchronize(c->stream));
     return VPMX_OK;
@@ -1451,12 +1452,14 @@ int32_t vpmx_adjoint_probe_energy(vpmx_ctx *p, const double *xp, const double *q
     if (st) return st;
     double *g = (double *)ensure(c, c->adj_q, sizeof(double) * 6 * (size_t)(nvr > 0 ? nvr : 1), &st);
     if (st) return st;
-    if (nprobe) VPMX_HIP(c, hipMemcpyAsync(pd, probes, sizeof(double) * 3 * nprobe, hipMemcpyHostToDevice, c->stream));
+    const Copy pr = {pd, probes, sizeof(double) * 3 * (size_t)nprobe};
+    VPMX_TRY(copy_in(c, &pr, 1));
     VPMX_TRY(adjoint_probe_energy(c, (const double *)c->xp.p, (const double *)c->qp.p, nvr, pd, nprobe, J, g,
                                   g + 3 * nvr));
     if (nvr) {
-        VPMX_HIP(c, hipMemcpyAsync(dq, g, sizeof(double) * 3 * nvr, hipMemcpyDeviceToHost, c->stream));
-        VPMX_HIP(c, hipMemcpyAsync(dx, g + 3 * nvr, sizeof(double) * 3 * nvr, hipMemcpyDeviceToHost, c->stream));
+        const size_t m = sizeof(double) * 3 * (size_t)nvr;
+        const Copy q[2] = {{dq, g, m}, {dx, g + 3 * nvr, m}};
+        VPMX_TRY(copy_out(c, q, 2));
     }
     VPMX_HIP(c, hipStreamSynchronize(c->stream));
     return VPMX_OK;
@@ -1475,15 +1478,17 @@ int32_t vpmx_adjoint_rollout(vpmx_ctx *p, const double *xp, const double *qp, in
     int st = VPMX_OK;
     double *pd = (double *)ensure(c, c->adj_p, sizeof(double) * 3 * (size_t)(nprobe > 0 ? nprobe : 1), &st);
     if (st) return st;
-    if (nprobe) VPMX_HIP(c, hipMemcpyAsync(pd, probes, sizeof(double) * 3 * nprobe, hipMemcpyHostToDevice, c->stream));
+    const Copy pr = {pd, probes, sizeof(double) * 3 * (size_t)nprobe};
+    VPMX_TRY(copy_in(c, &pr, 1));
     const int saved_prec = c->precision;
     c->precision = 0;
     const int r = adjoint_rollout(c, nsteps, dt, uinf, ckpt, pd, nprobe, J);
     c->precision = saved_prec;
     VPMX_TRY(r);
     if (nvr) {
-        VPMX_HIP(c, hipMemcpyAsync(dq, c->adj_qb.p, sizeof(double) * 3 * nvr, hipMemcpyDeviceToHost, c->stream));
-        VPMX_HIP(c, hipMemcpyAsync(dx, c->adj_xb.p, sizeof(double) * 3 * nvr, hipMemcpyDeviceToHost, c->stream));
+        const size_t m = sizeof(double) * 3 * (size_t)nvr;
+        const Copy q[2] = {{dq, c->adj_qb.p, m}, {dx, c->adj_xb.p, m}};
+        VPMX_TRY(copy_out(c, q, 2));
     }
     VPMX_HIP(c, hipStreamSynchronize(c->stream));
     return VPMX_OK;
