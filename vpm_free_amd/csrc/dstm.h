@@ -16,9 +16,9 @@ struct DmSolve {
 };
 
 // Whether the x and y transforms of a plane fit one work-group (k_dstm_plane), and whether lines
-// of m points take the matrix passes at all.
+// of m points take the matrix passes at all (forward: a pass of the forward transform alone).
 bool dstm_plane_fits(const Ctx *c, const int m[3]);
-bool dstm_line_fits(int m, bool f32);
+bool dstm_line_fits(int m, bool f32, bool forward = false);
 
 // RHS (interior of the view, Dirichlet values of bc folded in) -> x and y transforms in w; and
 // back: x and y transforms of w into the interior of out.  One launch each (FP64 arrays).

@@ -594,39 +594,11 @@ template <> struct FixedFft<8> {  // 544 = 17.8.4 (FP32, 273-node inner box): th
         wave_fft_s<C, Buf, CR, 544, 1, 17, 8, 4>(b, tw, lane);
     }
 };
-template <> struct FixedFft<9> {  // 272 = 4.4.17 with the radix-17 outputs split over 4 lanes
-    static constexpr int L = 272;
-    template <class C, class Buf, bool CR = false>
-    static __device__ __forceinline__ void run(Buf b, const C *tw, int lane) {
-        wave_fft_sx<C, Buf, false, true, 272, 1, 4, 4, 17>(b, tw, lane);
-    }
-};
 template <> struct FixedFft<10> {  // 544 = 17.8.4 with the radix-17 outputs split over 2 lanes
     static constexpr int L = 544;
     template <class C, class Buf, bool CR = false>
     static __device__ __forceinline__ void run(Buf b, const C *tw, int lane) {
         wave_fft_sx<C, Buf, false, true, 544, 1, 17, 8, 4>(b, tw, lane);
-    }
-};
-template <> struct FixedFft<11> {  // 160 = 8.4.5 (FP64, 161-node block: the 128^3 class)
-    static constexpr int L = 160;
-    template <class C, class Buf, bool CR = false>
-    static __device__ __forceinline__ void run(Buf b, const C *tw, int lane) {
-        wave_fft_s<C, Buf, CR, 160, 1, 8, 4, 5>(b, tw, lane);
-    }
-};
-template <> struct FixedFft<12> {  // 144 = 4.4.9 (FP64, 145-node inner box of the 128^3 class)
-    static constexpr int L = 144;
-    template <class C, class Buf, bool CR = false>
-    static __device__ __forceinline__ void run(Buf b, const C *tw, int lane) {
-        wave_fft_s<C, Buf, CR, 144, 1, 4, 4, 9>(b, tw, lane);
-    }
-};
-template <> struct FixedFft<14> {  // 272 = 16.17, the radix-17 outputs split over 4 lanes: two stages
-    static constexpr int L = 272;
-    template <class C, class Buf, bool CR = false>
-    static __device__ __forceinline__ void run(Buf b, const C *tw, int lane) {
-        wave_fft_sx<C, Buf, false, true, 272, 1, 16, 17>(b, tw, lane);
     }
 };
 template <> struct FixedFft<2> {  // 288 = 4.4.2.9 (FP64, 289-node block)
@@ -642,13 +614,6 @@ template <> struct FixedFft<5> {  // 544 = 17.4.4.2 (FP32, 273-node inner box; t
     template <class C, class Buf, bool CR = false>
     static __device__ __forceinline__ void run(Buf b, const C *tw, int lane) {
         wave_fft_s<C, Buf, CR, 544, 1, 17, 4, 4, 2>(b, tw, lane);
-    }
-};
-template <> struct FixedFft<3> {  // 272 = 4.4.17 (FP64, 273-node inner box)
-    static constexpr int L = 272;
-    template <class C, class Buf, bool CR = false>
-    static __device__ __forceinline__ void run(Buf b, const C *tw, int lane) {
-        wave_fft_s<C, Buf, CR, 272, 1, 4, 4, 17>(b, tw, lane);
     }
 };
 

@@ -32,10 +32,15 @@ namespace vpmx {
 typedef double dm_acc __attribute__((ext_vector_type(4)));
 
 // Longest lines of the matrix passes.  The products grow with the square of the length, the FFT
-// passes (k_dst_wave) hardly: solves of 3 components, us per pass x forward / y / z, products
-// against FFT -- FP64 159 points 59/47/84 against 74/63/133, 287 points 471/394/680 against
-// 398/371/728; FP32 arrays (FP64 products) cost the same products for half the bytes.
-constexpr int DM_MAX = 224, DM_MAX32 = 176;
+// passes hardly, but these depend on the factors of m + 1.  Whole solves of m^3 points, 3
+// components, us, products against FFT.  FP64: 231 (8.29) 1233/4330, 239 1289/1489, 255 1548/1650,
+// 263 (8.3.11) 1980/2991, 271 (16.17) 2065/2450, 279 2323/2489, 287 (32.9) 2420/2212, 303 3155/13325,
+// 319 4355/6821, 367 7405/23249 -- the products but for the 288-point transform, whose z forward
+// pass alone loses too (465 against 618).  FP32 arrays (FP64 sums: half the bytes, the same
+// products): 191 481/563, 207 759/881, 215 847/793, 239 1189/1139, 255 1332/1117, 271 1907/1261,
+// but with factors over 17 (no register transform) 231 1139/3079, 247 1296/3649.
+// DM_MAX: three row blocks a wave (24 of them).
+constexpr int DM_MAX = 367, DM_MAX32 = 208, DM_PLANE = 224;
 constexpr int DM_PAD = 8;  // zero rows after a line: the products run over whole pairs of k-steps
 
 // The folded transform of one length.  Segments: outputs k = k0 + ks i (i < nk, 1-based wave
@@ -545,7 +550,18 @@ static int dm_plan(Ctx *c, int m, DmPlan *out) {
     return VPMX_OK;
 }
 
-bool dstm_line_fits(int m, bool f32) { return m >= 1 && m <= (f32 ? DM_MAX32 : DM_MAX); }
+// n without its factors up to p
+static int dm_without(int n, int p) {
+    for (int q = 2; q <= p; q++)
+        while (n % q == 0) n /= q;
+    return n;
+}
+bool dstm_line_fits(int m, bool f32, bool forward) {
+    if (m < 1 || m > DM_MAX) return false;
+    if (f32) return m <= DM_MAX32 || dm_without(m + 1, 17) > 1;
+    const bool fft = m >= 256 && m < 288 && dm_without(m + 1, 3) == 1;
+    return forward || !fft;
+}
 
 static int dm_pitch(int m) {  // 2 (mod 4): 16 lines of two neighbouring points fall on all banks
     int p = m + DM_PAD;
@@ -566,7 +582,7 @@ static int dm_plane_jobs(const int m[3]) {
 
 bool dstm_plane_fits(const Ctx *c, const int m[3]) {
     for (int d = 0; d < 3; d++)
-        if (!dstm_line_fits(m[d], false)) return false;
+        if (m[d] < 1 || m[d] > DM_PLANE) return false;
     // above about 96 x 96 points a plane's work-group is one long chain (load, two products, two
     // folds): the separate passes are faster (y + x 79 points: 19.4 against 20.4 us, 95: 27 against
     // 30, 143: 83 against 116), below it one launch less counts more

@@ -848,15 +848,15 @@ __host__ __device__ constexpr int wave_pad_shift(bool dbl, int mode, int fix) {
     // the 8.8.9 plan: one slot per 8 elements keeps its radix-8 stores (strides 8 and 64
     // elements for groups of 8 lanes) on distinct banks in every pass
     if (fix == 6 || fix == 7 || fix == 8 || fix == 10) return 3;
-    // the 16.4.9 and 16.17 plans: their radix-16 stage writes 16 consecutive elements per lane
-    // (lanes 16 elements apart), which one slot per 16 elements spreads over the banks
-    if (fix == 13 || fix == 14) return 4;
+    // the 16.4.9 plan: its radix-16 stage writes 16 consecutive elements per lane (lanes 16
+    // elements apart), which one slot per 16 elements spreads over the banks
+    if (fix == 13) return 4;
     return fix < 0 ? 0 : (mode == DST_Y || (mode == DST_Z && (dbl || fix == 0)) || (!dbl && fix == 0 && mode == DST_XF)) ? (dbl ? 3 : 4) : 0;
 }
-// Radix-17 roots as constants in the 272- and 544-point plans (measured per pass: faster where
-// the extra registers cost no occupancy).
+// Radix-17 roots as constants in the 544-point plans (measured per pass: faster where the extra
+// registers cost no occupancy).
 __host__ __device__ constexpr bool const_roots(bool dbl, int mode, int fix) {
-    return dbl ? (fix == 3 && mode != DST_Z) : ((fix == 5 || fix == 8) && (mode == DST_Z || mode == DST_XI));
+    return !dbl && ((fix == 5 || fix == 8) && (mode == DST_Z || mode == DST_XI));
 }
 
 // T: arithmetic and work-array type (double: plain FP64 form, half-length transforms;
@@ -1073,8 +1073,8 @@ __global__ void __launch_bounds__(NL * WV_PS) k_dst_wave(DstArgs a, WavePlan P) 
 }
 // The same with the registers capped for W waves per SIMD (W = 4: 128 VGPRs, two 8-wave
 // work-groups per CU; W = 6: 80 VGPRs, three).  Measured on the 289- and 273-node blocks:
-// the FP64 x and y passes of the 289-node block, the FP64 x inverse and the FP32 z pass of
-// the 273-node box gain from four waves despite a few spilled registers, the FP32 x inverse
+// the FP64 x and y passes of the 289-node block and the FP32 z pass of the 273-node box
+// gain from four waves despite a few spilled registers, the FP32 x inverse
 // pass of the 289-node block from six; the other passes lose more to the spills than the
 // occupancy brings (the FP32 y pass at six waves: 8 % slower), or already fit.
 template <int W, int MODE, int MAXR, class T, int FIX, int NL = WV_NL>
@@ -1083,7 +1083,7 @@ k_dst_wave_cap(DstArgs a, WavePlan P) {
     dst_wave_body<MODE, MAXR, T, FIX, NL>(a, P);
 }
 __host__ __device__ constexpr int wave_cap(bool dbl, int mode, int fix) {
-    if (dbl) return ((fix == 2 && (mode == DST_XF || mode == DST_Y)) || (fix == 3 && mode == DST_XI)) ? 4 : 0;
+    if (dbl) return fix == 2 && (mode == DST_XF || mode == DST_Y) ? 4 : 0;
     if (fix == 0 && mode == DST_XI) return 6;
     return (fix == 5 && mode == DST_Z) ? 4 : 0;
 }
@@ -1470,23 +1470,18 @@ static int launch_wave(Ctx *c, DstArgs a, int ncomp, int rc, const FftPlan *fp) 
             if (fp->radix[q] != rr[q]) return false;
         return true;
     };
-    static const int r576[] = {4, 4, 4, 3, 3}, r288[] = {4, 4, 2, 3, 3}, r272[] = {4, 4, 17}, r544[] = {4, 4, 2, 17};
+    static const int r576[] = {4, 4, 4, 3, 3}, r288[] = {4, 4, 2, 3, 3}, r544[] = {4, 4, 2, 17};
     int fix = -1;
     if (sizeof(T) == 4 && fp->L == 576 && same(r576, 5)) fix = 0;
     if (sizeof(T) == 8 && fp->L == 288 && same(r288, 5)) fix = 2;
-    if (sizeof(T) == 8 && fp->L == 272 && same(r272, 3)) fix = 3;
     if (sizeof(T) == 4 && fp->L == 544 && same(r544, 4)) fix = 5;
-    static const int r160[] = {4, 4, 2, 5}, r144[] = {4, 4, 3, 3};
-    if (sizeof(T) == 8 && fp->L == 160 && same(r160, 4)) fix = 11;
-    if (sizeof(T) == 8 && fp->L == 144 && same(r144, 4)) fix = 12;
     // kernel variants: with a compile-time plan the registers capped for four waves per SIMD
     // (six for the FP32 x inverse of the 576-point plan) or not, each in both batch orders;
     // FP32 compile-time plans also with 32-line batches (1024 threads) -- the tuner times all
     constexpr bool dbl = sizeof(T) == 8;
     // (each length's plan is instantiated only for the form that uses it)
-    constexpr int c2 = wave_cap(dbl, MODE, 2), c3 = wave_cap(dbl, MODE, 3), c0 = wave_cap(dbl, MODE, 0),
-                  c5 = wave_cap(dbl, MODE, 5);
-    constexpr int k2 = c2 ? c2 : 4, k3 = c3 ? c3 : 4, k0 = c0 ? c0 : 4, k5 = c5 ? c5 : 4;
+    constexpr int c2 = wave_cap(dbl, MODE, 2), c0 = wave_cap(dbl, MODE, 0), c5 = wave_cap(dbl, MODE, 5);
+    constexpr int k2 = c2 ? c2 : 4, k0 = c0 ? c0 : 4, k5 = c5 ? c5 : 4;
     struct Var {
         const void *fn;
         const char *name;
@@ -1502,15 +1497,6 @@ static int launch_wave(Ctx *c, DstArgs a, int ncomp, int rc, const FftPlan *fp) 
         if (fix == 2) {
             unc = (const void *)k_dst_wave<MODE, 4, T, 2>;
             cap = (const void *)k_dst_wave_cap<k2, MODE, 4, T, 2>;
-        } else if (fix == 3) {
-            unc = (const void *)k_dst_wave<MODE, 17, T, 3>;
-            cap = (const void *)k_dst_wave_cap<k3, MODE, 17, T, 3>;
-        } else if (fix == 11) {
-            unc = (const void *)k_dst_wave<MODE, 9, T, 11>;
-            cap = (const void *)k_dst_wave_cap<4, MODE, 9, T, 11>;
-        } else if (fix == 12) {
-            unc = (const void *)k_dst_wave<MODE, 9, T, 12>;
-            cap = (const void *)k_dst_wave_cap<4, MODE, 9, T, 12>;
         }
     } else {
         if (fix == 0) {
@@ -1535,17 +1521,6 @@ static int launch_wave(Ctx *c, DstArgs a, int ncomp, int rc, const FftPlan *fp) 
             add(cap32, "capped, 32-line batches", 32, 0, fix);
         }
         if constexpr (dbl) {
-            if (fix == 3) {  // the same plan with the radix-17 outputs split over four lanes
-                add((const void *)k_dst_wave<MODE, 17, T, 9>, "radix-17 split", 16, 0, 9);
-                add((const void *)k_dst_wave_cap<k3, MODE, 17, T, 9>, "radix-17 split, capped", 16, 0, 9);
-                add((const void *)k_dst_wave<MODE, 17, T, 9>, "radix-17 split, batch halves in turn", 16, 1, 9);
-                add((const void *)k_dst_wave_cap<k3, MODE, 17, T, 9>, "radix-17 split, capped, batch halves in turn",
-                    16, 1, 9);
-                // and the two-stage 16.17 plan, radix-17 split
-                add((const void *)k_dst_wave<MODE, 17, T, 14>, "16.17 plan, radix-17 split", 16, 0, 14);
-                add((const void *)k_dst_wave<MODE, 17, T, 14>, "16.17 plan, radix-17 split, batch halves in turn", 16,
-                    1, 14);
-            }
             if (fix == 2) {  // the three-stage 8.4.9 plan of the same length
                 add((const void *)k_dst_wave<MODE, 9, T, 7>, "8.4.9 plan", 16, 0, 7);
                 add((const void *)k_dst_wave_cap<k2, MODE, 9, T, 7>, "8.4.9 plan, capped", 16, 0, 7);
@@ -1704,25 +1679,18 @@ static int launch_zmix(Ctx *c, DstArgs a, int ncomp, const AxisPlan &X, double *
             if (fp->radix[q] != rr[q]) return false;
         return true;
     };
-    static const int r576[] = {4, 4, 4, 3, 3}, r288[] = {4, 4, 2, 3, 3}, r272[] = {4, 4, 17}, r544[] = {4, 4, 2, 17};
+    static const int r576[] = {4, 4, 4, 3, 3}, r288[] = {4, 4, 2, 3, 3};
     // kernels (compile-time plans of both forms, or runtime plans), each in both batch orders
     struct ZK {
         const void *fn;
         int fix32, fix64;
         const char *name;
     };
-    ZK zk[4];
-    int nk = 1;
+    ZK zk;
     if (f32->L == 576 && same(f32, r576, 5) && f64->L == 288 && same(f64, r288, 5)) {
-        zk[0] = {(const void *)k_dst_zmix<4, 0, 2>, 0, 2, "FP32 forward, FP64 inverse"};
-    } else if (f32->L == 544 && same(f32, r544, 4) && f64->L == 272 && same(f64, r272, 3)) {
-        zk[0] = {(const void *)k_dst_zmix<17, 5, 3>, 5, 3, "FP32 forward, FP64 inverse"};
-        zk[1] = {(const void *)k_dst_zmix<17, 10, 9>, 10, 9, "FP32 forward (17.8.4), FP64 inverse, radix-17 split"};
-        zk[2] = {(const void *)k_dst_zmix<17, 5, 9>, 5, 9, "FP32 forward, FP64 inverse with radix-17 split"};
-        zk[3] = {(const void *)k_dst_zmix<17, 5, 14>, 5, 14, "FP32 forward, FP64 inverse 16.17 with radix-17 split"};
-        nk = 4;
+        zk = {(const void *)k_dst_zmix<4, 0, 2>, 0, 2, "FP32 forward, FP64 inverse"};
     } else {
-        zk[0] = {rc == 4 ? (const void *)k_dst_zmix<4, -1, -1>
+        zk = {rc == 4 ? (const void *)k_dst_zmix<4, -1, -1>
                  : rc == 7 ? (const void *)k_dst_zmix<7, -1, -1>
                  : rc == 17 ? (const void *)k_dst_zmix<17, -1, -1> : (const void *)k_dst_zmix<37, -1, -1>,
                  -1, -1, "FP32 forward, FP64 inverse"};
@@ -1735,20 +1703,11 @@ static int launch_zmix(Ctx *c, DstArgs a, int ncomp, const AxisPlan &X, double *
         const int Wq = (Np32 + 1) / 2 > Np64 ? (Np32 + 1) / 2 : Np64;
         return sizeof(double2) * (size_t)(8 * Wq + f32->L / 2 + f64->L);
     };
-    const void *fns[8];
-    const char *names[8];
-    size_t ldsv[8];
-    int thr[8];
-    char nbuf[8][96];
-    for (int q = 0; q < nk; q++)
-        for (int o = 0; o < 2; o++) {
-            const int v = 2 * q + o;
-            fns[v] = zk[q].fn;
-            std::snprintf(nbuf[v], sizeof nbuf[v], "%s%s", zk[q].name, o ? ", batch halves in turn" : "");
-            names[v] = nbuf[v];
-            ldsv[v] = lds_of(zk[q].fix32, zk[q].fix64);
-            thr[v] = DST_THREADS;
-        }
+    const std::string swapped = std::string(zk.name) + ", batch halves in turn";
+    const void *fns[2] = {zk.fn, zk.fn};
+    const char *names[2] = {zk.name, swapped.c_str()};
+    const size_t ldsv[2] = {lds_of(zk.fix32, zk.fix64), lds_of(zk.fix32, zk.fix64)};
+    const int thr[2] = {DST_THREADS, DST_THREADS};
     const int64_t nbatch = (a.nlines + 15) / 16;
     auto grid_of = [&](int per_cu) {
         int64_t resident = (int64_t)c->num_cu * per_cu / 16 * 16;
@@ -1780,7 +1739,7 @@ static int launch_zmix(Ctx *c, DstArgs a, int ncomp, const AxisPlan &X, double *
             VPMX_HIP(c, hipLaunchKernel(fns[fi], grid_of(pc), dim3(DST_THREADS), targs, ldsv[fi], c->stream));
             return VPMX_OK;
         };
-        VPMX_TRY(tune_v(c, key, 2 * nk, fns, names, ldsv, thr, trial, &ch));
+        VPMX_TRY(tune_v(c, key, 2, fns, names, ldsv, thr, trial, &ch));
     }
     a.order = ch.fi & 1;
     const void *fn = fns[ch.fi];
@@ -2492,13 +2451,17 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     const bool inv64 = !planes && form == SOLVE_INV64 && wave32 && wave64 && c->dst_kernel == 4;
     const bool f32 = !planes && ((form == SOLVE_FP32 && wave32) || inv64);
     // a pass whose lines are short enough: products with the sine matrix (k_dstm.hip)
-    auto mm = [&](int d, bool in32) { return c->dst_kernel == 4 && dstm_line_fits(m[d], in32); };
+    // (its z pass counts the values of a component in 32 bits)
+    const bool z32 = (int64_t)((m[0] + 31) / 32 * 32) * m[1] * m[2] < ((int64_t)1 << 31);
+    auto mm = [&](int d, bool in32, bool forward = false) {
+        return c->dst_kernel == 4 && dstm_line_fits(m[d], in32, forward) && (d < 2 || z32);
+    };
     if (inv64) reuse = 0;  // (the fine solves' reuse keeps FP32 arrays)
     // the kept transforms are worth their corrections (six launches) on large grids only
     if ((int64_t)wn[0] * wn[1] * wn[2] < SPECTRAL_MIN_NODES) reuse = 0;
-    // one-wave kernels on every axis: rows of the work array padded to 128 bytes
-    const bool wave_all = f32 || planes || (c->dst_kernel == 4 && wave_class(ax[0], false) && wave_class(ax[1], false) &&
-                                  wave_class(ax[2], false));
+    // one-wave kernels or products on every axis: rows of the work array padded to 128 bytes
+    auto padded = [&](int d) { return mm(d, false) || (c->dst_kernel == 4 && wave_class(ax[d], false)); };
+    const bool wave_all = f32 || planes || (padded(0) && padded(1) && padded(2));
     if (wave_all) {
         const int q = f32 ? 32 : 16;
         a.px = (m[0] + q - 1) / q * q;
@@ -2529,7 +2492,7 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
         if (mm(1, f32)) VPMX_TRY(dstm_y(c, ds, w, timed));
         else VPMX_TRY(run_pass<DST_Y>(c, a, ncomp, ax[1], f32));
         c->save_key[5] = -1;
-        // keep them: the rest of this solve runs in a second array (one-wave kernels only; the
+        // keep them: the rest of this solve runs in a second array (padded rows only; the
         // correction pass takes a row per work-group)
         if (reuse == 1 && !bc && wave_all && a.px <= 320) {
             double *w2 = (double *)ensure(c, c->dst_save, wbytes, &st);
@@ -2543,7 +2506,8 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     // faces' sums
     a.nlines = (int64_t)a.px * m[1];
     FaceBufs fb{};
-    const bool zspec = face_nd && !inv64 && (f32 || mm(2, false) || (c->dst_kernel == 4 && wave_class(ax[2], false)));
+    const bool zmm = mm(2, f32) || (face_nd && !f32 && mm(2, false, true));
+    const bool zspec = face_nd && !inv64 && (f32 || zmm || (c->dst_kernel == 4 && wave_class(ax[2], false)));
     if (face_nd) {
         VPMX_TRY(face_bufs(c, m[0], m[1], m[2], ncomp, &fb));
         if (zspec) {
@@ -2558,7 +2522,7 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
         if (mm(2, false)) VPMX_TRY(dstm_z(c, ds, a.w, w64, false, a.lam, a.norm, nullptr, nullptr, timed));
         else VPMX_TRY(launch_zmix(c, a, ncomp, ax[2], w64));
         a.w = a.wo = w64;
-    } else if (mm(2, f32)) {
+    } else if (zmm) {
         VPMX_TRY(dstm_z(c, ds, a.w, a.wo, f32, a.lam, a.norm, a.zsum, a.zw, timed));
         a.w = a.wo;
     } else {
