@@ -96,17 +96,25 @@ double wall_ms() {
 static void collect_times(Ctx *, const bool *) {}
 
 // ---------------------------------------------------------------- pmesh (iynbc=1)
+// Whether a grid's normal derivatives come from the solve's spectrum.
+static bool spectral_derivs(const Ctx *c, const int n[3]) {
+    return c->face_derivs == 1 ||
+           (c->face_derivs < 0 && (int64_t)n[0] * n[1] * n[2] >= SPECTRAL_MIN_NODES && n[0] <= 322);
+}
+
 // pmesh(iynbc=1) on grid g: SOL_0 = zero-BC solve, sources from its normal derivatives,
 // SOL(faces) += boundary sums (ibctyp 2 point sources, 3 panels; tree form with levmax
 // levels when levmax >= 0, pmlib.f90:69 ibctyp/itree/levmax), then the Dirichlet solve of
 // the whole grid.
 // fresh: sol counts as zero whatever it holds; its faces and (without part) interior are written.
+// nblk > 1: that many grids of g's size, their arrays one after another (three components each)
+// and their origins at xb[6 b]; the solves take them as 3 nblk components.
 static int pmesh_inf(Ctx *c, const Grid &g, GView rhs, GView sol, DBuf &s0buf, bool fine, int levmax, int ibctyp,
-                     bool fresh, const SolvePartial *part = nullptr) {
+                     bool fresh, const SolvePartial *part = nullptr, int nblk = 1, const double *xb = nullptr) {
     int st = VPMX_OK;
     const int n[3] = {g.n[0], g.n[1], g.n[2]};
     int64_t G = (int64_t)n[0] * n[1] * n[2];
-    double *s0 = (double *)ensure(c, s0buf, sizeof(double) * 3 * (size_t)G, &st);
+    double *s0 = (double *)ensure(c, s0buf, sizeof(double) * 3 * (size_t)G * nblk, &st);
     if (st) return st;
     GView s0v = view(s0, n);
     int32_t win[6] = {1, 1, 1, n[0], n[1], n[2]};
@@ -120,20 +128,27 @@ static int pmesh_inf(Ctx *c, const Grid &g, GView rhs, GView sol, DBuf &s0buf, b
     int64_t nb = 0;
     // SOL_0 is read only through its normal derivatives at the faces: on large grids they come
     // straight from its spectrum (no inverse y and x passes), else from the solved field
-    const bool spectral = c->face_derivs == 1 || (c->face_derivs < 0 && G >= SPECTRAL_MIN_NODES && n[0] <= 322);
-    if (spectral) {
+    if (nblk == 1 && spectral_derivs(c, n)) {
         double *fd = normal_derivs_table(c, 3, n, &st);
         if (st) return st;
         VPMX_TRY(poisson_dirichlet(c, 3, n, h, rhs, nullptr, s0v, ru, SOLVE_CTX, fd));  // keeps its forward transforms
         VPMX_TRY(normal_derivs_cells(c, 3, g, fd, sig, cxyz, wgt, &nb));
+        // SOL_0 is dead once the sources exist: scratch of the panel sums
+        VPMX_TRY(boundary_sums(c, 3, g, nb, sig, cxyz, wgt, sol, fine, levmax, ibctyp, &s0v, fresh));
     } else {
-        VPMX_TRY(poisson_dirichlet(c, 3, n, h, rhs, nullptr, s0v, ru, SOLVE_CTX, nullptr, nullptr, true));  // keeps its forward transforms
-        VPMX_TRY(normal_derivs(c, 3, g, s0v, sig, cxyz, wgt, &nb, true));
+        VPMX_TRY(poisson_dirichlet(c, 3 * nblk, n, h, rhs, nullptr, s0v, ru, SOLVE_CTX, nullptr, nullptr, true));  // keeps its forward transforms
+        for (int b = 0; b < nblk; b++) {
+            Grid gb = g;
+            if (xb) std::copy(xb + 6 * b, xb + 6 * b + 3, gb.x0);
+            GView s0b = s0v, sb = sol;
+            s0b.p += 3 * G * b;
+            sb.p += 3 * G * b;
+            VPMX_TRY(normal_derivs(c, 3, gb, s0b, sig, cxyz, wgt, &nb, true));
+            VPMX_TRY(boundary_sums(c, 3, gb, nb, sig, cxyz, wgt, sb, fine, levmax, ibctyp, &s0b, fresh));
+        }
     }
-    // SOL_0 is dead once the sources exist: scratch of the panel sums
-    VPMX_TRY(boundary_sums(c, 3, g, nb, sig, cxyz, wgt, sol, fine, levmax, ibctyp, &s0v, fresh));
     // same RHS: reuses them (part: only the nodes the caller reads)
-    VPMX_TRY(poisson_dirichlet(c, 3, n, h, rhs, &sol, sol, 2 * ru, SOLVE_CTX, nullptr, part));
+    VPMX_TRY(poisson_dirichlet(c, 3 * nblk, n, h, rhs, &sol, sol, 2 * ru, SOLVE_CTX, nullptr, part));
     return VPMX_OK;
 }
 
@@ -275,6 +290,23 @@ static int64_t block_offsets(const vpmx_geom &G, std::vector<int64_t> &off) {
 }
 static const int32_t *block_n(const vpmx_geom &G, int b) { return &G.nnbl[3 * b]; }
 
+// Blocks from b on that the solves take together, as 3 components each: neighbours in memory of one
+// size, with one inner box, while they are small.  A 64^3 block's solve leaves most of the chip idle
+// at each of its three launches (8 of 67^3 points: one by one 1.9 ms, together 1.1); blocks of
+// SPECTRAL_MIN_NODES fill it alone.  BLOCK_BATCH bounds the work arrays (24 bytes a node).
+constexpr int64_t BLOCK_BATCH = 1 << 25;
+static int same_blocks(const Ctx *c, int b) {
+    const vpmx_geom &G = c->geom;
+    const int32_t *n = block_n(G, b), *w = &G.nnbl_bl[6 * b];
+    const int64_t nodes = (int64_t)n[0] * n[1] * n[2];
+    if (nodes >= SPECTRAL_MIN_NODES || spectral_derivs(c, n)) return 1;
+    int e = b + 1;
+    while (e < G.nblocks && (e + 1 - b) * nodes <= BLOCK_BATCH && std::equal(n, n + 3, block_n(G, e)) &&
+           std::equal(w, w + 6, &G.nnbl_bl[6 * e]))
+        e++;
+    return e - b;
+}
+
 // yaps3d.f90:1-453 with BLOCKS = NBI*NBJ*NBK blocks on this device, the work of every rank
 // in turn: all fine infinite-domain solves; the coarse problem from every block's samples
 // (Laplacians summed in block order); the coarse solve; interp_stencil on every block's
@@ -297,9 +329,11 @@ static int yaps_multi(Ctx *c, bool *used) {
     // 1. fine infinite-domain solves
     mark(c, ST_FINE, 0);
     c->dst_timed_m = G.nnbl[1] - 2;
-    for (int b = 0; b < NB; b++) {
+    for (int b = 0, nb; b < NB; b += nb) {
+        nb = same_blocks(c, b);
         Grid gb = make_grid(block_n(G, b), &G.xbound_bl[6 * b], G.dpm);
-        VPMX_TRY(pmesh_inf(c, gb, bview(rhs_bl, b), bview(sol_bl, b), c->sol0, true, tree ? G.ilevmax : -1, P.ibctyp, true));
+        VPMX_TRY(pmesh_inf(c, gb, bview(rhs_bl, b), bview(sol_bl, b), c->sol0, true, tree ? G.ilevmax : -1, P.ibctyp, true,
+                           nullptr, nb, &G.xbound_bl[6 * b]));
     }
     mark(c, ST_FINE, 1);
     used[ST_FINE] = used[ST_BOUNDS] = true;
@@ -394,14 +428,15 @@ static int yaps_multi(Ctx *c, bool *used) {
     used[ST_BC] = true;
     // 4. inner-box solves
     mark(c, ST_FINAL, 0, true);
-    for (int b = 0; b < NB; b++) {
+    for (int b = 0, nb; b < NB; b += nb) {
+        nb = same_blocks(c, b);
         const int32_t *w = &G.nnbl_bl[6 * b];
         int wn[3] = {w[3] - w[0] + 1, w[4] - w[1] + 1, w[5] - w[2] + 1};
         double h[3];
         window_h(&G.xbound_bl[6 * b], G.dpm, w, h);
         GView rin = view(rhs_bl + boff[b], wn, w[0] - 1, w[1] - 1, w[2] - 1, block_n(G, b));
         GView sin = view(sol_bl + boff[b], wn, w[0] - 1, w[1] - 1, w[2] - 1, block_n(G, b));
-        VPMX_TRY(poisson_dirichlet(c, 3, wn, h, rin, &sin, sin, 0, final_form(c)));
+        VPMX_TRY(poisson_dirichlet(c, 3 * nb, wn, h, rin, &sin, sin, 0, final_form(c)));
     }
     mark(c, ST_FINAL, 1);
     used[ST_FINAL] = true;
