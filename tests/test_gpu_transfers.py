@@ -5,13 +5,22 @@ import threading
 
 import numpy as np
 import pytest
-import torch
 
 pytestmark = pytest.mark.gpu
 
 # one particle; the last size of the small path and the first of the chunked one; chunk ends inside
 # and between the arrays; every thread busy
 SIZES = [1, 74898, 74899, 87381, 87382, 1200001]
+
+
+def pinned(a):
+    """A copy of the array in pinned host memory, and its address."""
+    import hip_mem as M
+    p = C.c_void_p()
+    assert M.runtime().hipHostMalloc(C.byref(p), C.c_size_t(a.nbytes), 0) == 0
+    b = np.ctypeslib.as_array((C.c_double * a.size).from_address(p.value)).reshape(a.shape)
+    b[:] = a
+    return b, p
 
 
 def cloud(n, seed):
@@ -25,12 +34,17 @@ def test_round_trip(vpmlib, n):
     with vpmlib.VPM(vpmlib.Params.make(0.125)) as c:
         for seed in (1, 2):
             x, q = cloud(n, seed)
+            held = []
             if seed == 2:
-                x, q = torch.from_numpy(x).pin_memory().numpy(), torch.from_numpy(q).pin_memory().numpy()
+                import hip_mem as M
+                (x, px), (q, pq) = pinned(x), pinned(q)
+                held = [px, pq]
             print("case: transfer", n, seed, flush=True)
             c.upload(x, q)
             xo, qo = c.download()[:2]
             assert np.array_equal(x, xo) and np.array_equal(q, qo)
+            for p in held:
+                M.runtime().hipHostFree(p)
 
 
 def test_contexts_on_threads(vpmlib):
@@ -60,7 +74,9 @@ def test_contexts_on_threads(vpmlib):
 
 @pytest.mark.parametrize("n", [5, 200000])
 def test_missing_array_is_refused(vpmlib, n):
-    """A null source is an error of the call, not a crash."""
+    """A null source is an error of the call, not a crash, and of that call alone."""
     with vpmlib.VPM(vpmlib.Params.make(0.125)) as c:
-        x, _ = cloud(n, 3)
+        x, q = cloud(n, 3)
         assert c._lib.vpmx_particles_upload(c._h, x.ctypes.data_as(C.POINTER(C.c_double)), None, n, 3) != 0
+        c.upload(x, q)
+        assert np.array_equal(c.download()[1], q)

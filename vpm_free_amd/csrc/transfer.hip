@@ -163,11 +163,17 @@ size_t total_bytes(const Copy *q, int n) {
     return b;
 }
 
-// Memory that the device reaches by itself (pinned, managed, the device's own), or none at all:
-// the runtime copies it, or refuses it.
+// A missing array is refused before any call of the runtime, whose last error would stay behind.
+bool missing(const Copy *q, int n) {
+    for (int i = 0; i < n; i++)
+        if (q[i].bytes && (!q[i].src || !q[i].dst)) return true;
+    return false;
+}
+
+// Memory that the device reaches by itself (pinned, managed, the device's own): the runtime
+// copies it.
 bool direct(const void *p) {
     hipPointerAttribute_t a;
-    if (!p) return true;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
@@ -195,6 +201,7 @@ int copy_direct(Ctx *c, bool in, const Copy *q, int n) {
 int copy_in(Ctx *c, const Copy *q, int n) {
     const size_t total = total_bytes(q, n);
     if (!total) return VPMX_OK;
+    if (missing(q, n)) return fail(c, VPMX_ERR_HIP, "copy: invalid argument (a null array)");
     if (any_direct(true, q, n)) return copy_direct(c, true, q, n);
     if (total > SMALL_COPY) return copy_large(c, true, q, n, total);
     char *b = nullptr;
@@ -212,6 +219,7 @@ int copy_in(Ctx *c, const Copy *q, int n) {
 int copy_out(Ctx *c, const Copy *q, int n) {
     const size_t total = total_bytes(q, n);
     if (!total) return VPMX_OK;
+    if (missing(q, n)) return fail(c, VPMX_ERR_HIP, "copy: invalid argument (a null array)");
     if (any_direct(false, q, n)) return copy_direct(c, false, q, n);
     if (total > SMALL_COPY) return copy_large(c, false, q, n, total);
     char *b = nullptr;

@@ -291,8 +291,8 @@ static int64_t block_offsets(const vpmx_geom &G, std::vector<int64_t> &off) {
 static const int32_t *block_n(const vpmx_geom &G, int b) { return &G.nnbl[3 * b]; }
 
 // Blocks from b on that the solves take together, as 3 components each: neighbours in memory of one
-// size, with one inner box, while they are small.  A 64^3 block's solve leaves most of the chip idle
-// at each of its three launches (8 of 67^3 points: one by one 1.9 ms, together 1.1); blocks of
+// size, with one inner box, while they are small.  A solve of 87^3 points leaves much of the chip
+// idle at each of its three launches (8 blocks, three solves each: 1.89 ms, together 1.19); blocks of
 // SPECTRAL_MIN_NODES fill it alone.  BLOCK_BATCH bounds the work arrays (24 bytes a node).
 constexpr int64_t BLOCK_BATCH = 1 << 25;
 static int same_blocks(const Ctx *c, int b) {
