@@ -100,7 +100,8 @@ int32_t vpmx_get_geometry(const vpmx_ctx *ctx, vpmx_geom *out);
 /* Arithmetic form (no reference counterpart: the reference is FP64 throughout).
  * 0 = plain FP64 form (default).  1 = mixed form: in FP32 the projection's weights and sums,
  * the sine-transform passes of the fine-block and coarse infinite-domain solves, the forward
- * passes and diagonal of the inner-box solve, and the interpolation's node values and sums; in
+ * passes and diagonal of the inner-box solve (their arrays; sums in FP64 where a pass is a matrix
+ * product, and small grids FP64 throughout), and the interpolation's node values and sums; in
  * FP64 the inner-box solve's inverse passes, the Green's-function boundary sums, the normal
  * derivatives, curl and stretching, remesh and diagnostics, and every particle array and grid
  * in HBM.  VPMX_PRECISION=mixed in the environment selects 1 at vpmx_create. */
@@ -108,8 +109,8 @@ int32_t vpmx_set_precision(vpmx_ctx *ctx, int32_t mode);
 /* Evaluation choices that leave the results unchanged beyond rounding (no counterpart in the
  * reference): "boundsum" -- the Green's-function boundary sums by 2 spectral convolution
  * (default), 0 direct sums over lattice tables, 1 direct sums over LDS source tiles;
- * "dst_reuse" -- 1 (default): the second fine solve of pmesh starts from the first one's
- * forward transforms, 0: both solves in full; "face_derivs" -- the normal derivatives of the
+ * "dst_reuse" -- 1 (default): on large grids the second fine solve of pmesh starts from the
+ * first one's forward transforms, 0: both solves in full; "face_derivs" -- the normal derivatives of the
  * zero-BC solve of pmesh (calc_normalderiv_3d): -1 (default) by grid size, 1 from its sine
  * spectrum after the z pass (no inverse y and x passes), 0 from the solved field;
  * "fine_partial" -- the second fine solve of a single yaps block: -1 (default) by grid size, 1 only
