@@ -12,6 +12,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "p2m_cells.h"
 #include "tune.h"
 #include "vpmx_internal.h"
 #include "vpmx_ctx.h"
@@ -373,9 +374,6 @@ constexpr int SMALL_TILES = 8192;
 // Round of the one-work-group-per-tile launches (xcd_slice): 256 work-groups per XCD.
 constexpr int64_t XCD_ROUND = 2048;
 
-constexpr int PT_X = 16, PT_Y = 4, PT_Z = 4;
-constexpr int PC_X = PT_X + 3, PC_Y = PT_Y + 3, PC_Z = PT_Z + 3;
-constexpr int PT_ROWS = PC_Y * PC_Z;
 // The staged particles in LDS, one array per field (neighbouring lanes read neighbouring
 // particles, so a field read is a unit-stride access across the wave): w[4 d + q][p] the
 // weight of the q-th node that visits particle p along axis d (nodes c_d - 1 .. c_d + 2 for
@@ -424,17 +422,16 @@ __global__ void k_p2m_sorted(const int *__restrict__ perm, const int *__restrict
 
 // Tiles whose 49 cell rows hold any particle (a superset of the tiles with work); thread per
 // tile, so the row-count loads of many tiles are in flight together.
-__global__ void k_p2m_tile_flags(int ntiles, int ntx, int nty, int vnx, int vny, int vnz, Grid g, int cny,
-                                 const int *__restrict__ rowcnt, int wlo1, int wlo2, int *__restrict__ flag) {
+__global__ void k_p2m_tile_flags(int ntiles, int ntx, int nty, Grid g, const int *__restrict__ rowcnt, int wlo1,
+                                 int wlo2, int *__restrict__ flag) {
     const int tile = blockIdx.x * blockDim.x + threadIdx.x;
     if (tile >= ntiles) return;
     const int ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
     const int J0 = ty * PT_Y - wlo1 + 1, K0 = tz * PT_Z - wlo2 + 1;
     int any = 0;
     for (int r = 0; r < PT_ROWS; r++) {
-        const int cj = J0 - 2 + r % PC_Y, ck = K0 - 2 + r / PC_Y;
-        if (cj >= -1 && cj <= g.n[1] + 1 && ck >= -1 && ck <= g.n[2] + 1)
-            any |= rowcnt[(cj + 1) + (int64_t)cny * (ck + 1)] > 0;
+        const int64_t row = p2m_row(J0, K0, r, g.n[1], g.n[2]);
+        if (row >= 0) any |= rowcnt[row] > 0;
     }
     flag[tile] = any;
 }
@@ -475,11 +472,9 @@ __global__ void __launch_bounds__(256) k_p2m_zero_changed(int ntiles, int ntx, i
 
 template <class T>
 __global__ void __launch_bounds__(256) k_p2m_tile(Grid g, const int *__restrict__ start,
-                                                  const int *__restrict__ rowcnt, int cnx, int cny,
-                                                  const T *__restrict__ R, double div, GView out, int vnx,
-                                                  int vny, int vnz, int wlo0,
-                                                  int wlo1, int wlo2, const int *__restrict__ list,
-                                                  const int *__restrict__ nlist) {
+                                                  const int *__restrict__ rowcnt, const T *__restrict__ R, double div,
+                                                  GView out, int vnx, int vny, int vnz, int wlo0, int wlo1, int wlo2,
+                                                  const int *__restrict__ list, const int *__restrict__ nlist) {
 #pragma clang fp contract(off)
     // particles per chunk (measured on the 273-node grid: 256 FP32 / 192 FP64 keep 5-6
     // work-groups per CU, enough to cover the load latencies of the row tables and staging)
@@ -503,14 +498,10 @@ __global__ void __launch_bounds__(256) k_p2m_tile(Grid g, const int *__restrict_
     if (tid == 0) any = 0;
     __syncthreads();
     if (tid < PT_ROWS) {
-        const int cj = J0 - 2 + tid % PC_Y, ck = K0 - 2 + tid / PC_Y;
-        int ok = cj >= -1 && cj <= g.n[1] + 1 && ck >= -1 && ck <= g.n[2] + 1;
-        if (ok) {
-            const int64_t row = (cj + 1) + (int64_t)cny * (ck + 1);
-            // (without the counts: the row's particles near the tile only)
-            ok = rowcnt ? rowcnt[row] > 0
-                        : start[row * cnx + min(I0 + PT_X + 2, g.n[0] + 2) + 1] > start[row * cnx + max(I0 - 2, -1) + 1];
-        }
+        const int64_t row = p2m_row(J0, K0, tid, g.n[1], g.n[2]);
+        int ok = row >= 0;
+        if (ok)  // (without the counts: the row's particles near the tile only)
+            ok = rowcnt ? rowcnt[row] > 0 : start[p2m_entry(I0, PC_X, row, g.n[0])] > start[p2m_entry(I0, 0, row, g.n[0])];
         rowok[tid] = ok;
         if (ok) any = 1;
     }
@@ -520,12 +511,7 @@ __global__ void __launch_bounds__(256) k_p2m_tile(Grid g, const int *__restrict_
         for (int e = tid; e < PT_ROWS * (PC_X + 1); e += blockDim.x) {
             const int r = e / (PC_X + 1), cidx = e - r * (PC_X + 1);
             int v = 0;
-            if (rowok[r]) {
-                const int cj = J0 - 2 + r % PC_Y, ck = K0 - 2 + r / PC_Y;
-                const int64_t row = (int64_t)cnx * ((cj + 1) + (int64_t)cny * (ck + 1));
-                const int cx = min(max(I0 - 2 + cidx, -1), g.n[0] + 2);
-                v = start[row + cx + 1];
-            }
+            if (rowok[r]) v = start[p2m_entry(I0, cidx, p2m_row(J0, K0, r, g.n[1], g.n[2]), g.n[0])];
             cst[r][cidx] = v;
         }
         __syncthreads();
@@ -674,8 +660,8 @@ int p2m_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
         } else {
         hipLaunchKernelGGL(k_row_counts, dim3((unsigned)((nrows + 255) / 256)), dim3(256), 0, c->stream, start,
                            s.cn[0], nrows, rowcnt);
-        hipLaunchKernelGGL(k_p2m_tile_flags, dim3(gt), dim3(256), 0, c->stream, (int)tiles, ntx, nty, vn[0], vn[1],
-                           vn[2], g, s.cn[1], rowcnt, wlo[1], wlo[2], flag);
+        hipLaunchKernelGGL(k_p2m_tile_flags, dim3(gt), dim3(256), 0, c->stream, (int)tiles, ntx, nty, g, rowcnt,
+                           wlo[1], wlo[2], flag);
         VPMX_TRY(exclusive_scan(c, flag, pos, tiles));
         hipLaunchKernelGGL(k_m2p_tile_list, dim3(gt), dim3(256), 0, c->stream, (int)tiles, flag, pos, list);
         if (zero_empty) {
@@ -706,10 +692,10 @@ int p2m_gather(Ctx *c, const Grid &g, const SortState &s, const double *xp, cons
         }
         }
         const void *fn = f32 ? (const void *)k_p2m_tile<float> : (const void *)k_p2m_tile<double>;
-        int cnx = s.cn[0], cny = s.cn[1], vx = vn[0], vy = vn[1], vz = vn[2], w0 = wlo[0], w1 = wlo[1], w2 = wlo[2];
+        int vx = vn[0], vy = vn[1], vz = vn[2], w0 = wlo[0], w1 = wlo[1], w2 = wlo[2];
         const int *lst = small ? nullptr : list, *nl = small ? nullptr : pos + tiles;
-        void *args[] = {(void *)&g, (void *)&start, (void *)&rowcnt, &cnx, &cny, &Rv, &div,
-                        &out, &vx, &vy, &vz, &w0, &w1, &w2, (void *)&lst, (void *)&nl};
+        void *args[] = {(void *)&g, (void *)&start, (void *)&rowcnt, &Rv, &div, &out,
+                         &vx, &vy, &vz, &w0, &w1, &w2, (void *)&lst, (void *)&nl};
         VPMX_HIP(c, hipLaunchKernel(fn, dim3((unsigned)tiles), dim3(256), args, 0, c->stream));
         VPMX_HIP(c, hipGetLastError());
         if (kclass >= 0) mark(c, ST_COUNT + kclass, 1);
