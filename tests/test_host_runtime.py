@@ -1,0 +1,73 @@
+"""Host-side handling of runtime calls that fail, on a stand-in for the HIP runtime (fake_hip.c: no GPU,
+kernels do nothing): each test runs in a process of its own that loads the stand-in before libvpmx."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes, sys
+import numpy as np
+F = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
+for f in (F.fake_calls, F.fake_done, F.fake_held):
+    f.restype = ctypes.c_long
+F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
+MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH = range(6)
+sys.path.insert(0, %r)
+from vpm_free_amd import vpm as V
+rng = np.random.default_rng(1)
+def fails(f, *a):
+    try:
+        f(*a)
+    except V.VpmError:
+        return True
+    return False
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    cc = shutil.which("gcc")
+    if not cc:
+        pytest.skip("no host compiler")
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run([cc, "-shared", "-fPIC", "-O1", "-w", os.path.join(HERE, "fake_hip.c"), "-o", so], check=True)
+
+    def go(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE % (so, os.path.dirname(HERE)) + code], capture_output=True,
+                           text=True, timeout=300)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+
+    return go
+
+
+@pytest.mark.parametrize("itree", [0, 1])
+def test_tables_after_a_failed_copy(run, itree):
+    """A table whose upload failed is uploaded by the next call: whichever copy of a first pmesh call
+    fails, that call is refused and the next one completes the set."""
+    run("""
+itree = %d
+n = np.array([13, 15, 17], np.int32)
+h = np.array([0.1, 0.11, 0.12])
+xb = np.zeros(6)
+a = rng.standard_normal((17, 15, 13, 3))
+def call(c):
+    c.stage_pmesh_inf(xb, h, n, a, np.zeros_like(a), itree=itree, levmax=2)
+with V.VPM(V.Params.make(0.125)) as c:
+    n0 = F.fake_done(MEMCPY)
+    call(c)
+    need = F.fake_done(MEMCPY) - n0
+assert need > 4
+for k in range(1, need + 1):
+    with V.VPM(V.Params.make(0.125)) as c:
+        n0 = F.fake_done(MEMCPY)
+        F.fake_fail(MEMCPY, k)
+        assert fails(call, c), k
+        F.fake_fail(MEMCPY, 0)
+        F.hipGetLastError()
+        call(c)
+        assert F.fake_done(MEMCPY) - n0 >= need, (k, F.fake_done(MEMCPY) - n0, need)
+""" % itree)

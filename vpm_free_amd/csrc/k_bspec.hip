@@ -954,14 +954,17 @@ static int get_launch(Ctx *c, SpecPlan *P, int tr, SpecLaunch **out) {
         }
         F.n = (int)qjobs.size() - F.first;
     }
-    VPMX_HIP(c, hipMalloc((void **)&L.qjobs, sizeof(SpecJob) * (qjobs.size() + 1)));
-    if (hipMalloc((void **)&L.jobs, sizeof(SpecJob) * (jobs.size() + 1)) != hipSuccess) {
-        (void)hipFree(L.qjobs);
-        return fail(c, VPMX_ERR_HIP, "spectral boundary sums: hipMalloc");
+    hipError_t e = hipMalloc((void **)&L.jobs, sizeof(SpecJob) * (jobs.size() + 1));
+    if (e == hipSuccess) e = hipMalloc((void **)&L.qjobs, sizeof(SpecJob) * (qjobs.size() + 1));
+    if (e == hipSuccess) e = hipMemcpy(L.jobs, jobs.data(), sizeof(SpecJob) * jobs.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess && !qjobs.empty())
+        e = hipMemcpy(L.qjobs, qjobs.data(), sizeof(SpecJob) * qjobs.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        if (L.jobs) (void)hipFree(L.jobs);
+        if (L.qjobs) (void)hipFree(L.qjobs);
+        return fail(c, VPMX_ERR_HIP, std::string("spectral boundary sums: job tables: ") + hipGetErrorString(e));
     }
-    R = L;
-    VPMX_HIP(c, hipMemcpy(R.jobs, jobs.data(), sizeof(SpecJob) * jobs.size(), hipMemcpyHostToDevice));
-    if (!qjobs.empty()) VPMX_HIP(c, hipMemcpy(R.qjobs, qjobs.data(), sizeof(SpecJob) * qjobs.size(), hipMemcpyHostToDevice));
+    R = L;  // (built: only once both tables are filled)
     return VPMX_OK;
 }
 
