@@ -71,3 +71,54 @@ for k in range(1, need + 1):
         call(c)
         assert F.fake_done(MEMCPY) - n0 >= need, (k, F.fake_done(MEMCPY) - n0, need)
 """ % itree)
+
+
+TRANSFERS = """
+def cloud(n):
+    return rng.standard_normal((n, 3)), rng.standard_normal((n, 4))
+def round_trip(c, n):
+    x, q = cloud(n)
+    c.upload(x, q)
+    xo, qo = c.download()[:2]
+    assert np.array_equal(x, xo) and np.array_equal(q, qo), n
+LARGE, SMALL = 700000, 500  # 39 MB in chunks, 28 kB through the pinned buffer
+"""
+
+
+@pytest.mark.parametrize("kind", ["HOSTMALLOC", "STREAM", "EVENT"])
+def test_transfer_slots_that_cannot_grow(run, kind):
+    """A refused allocation while the slots are set up leaves fewer of them, no error behind, and nothing
+    allocated twice by the attempts that follow."""
+    run(TRANSFERS + """
+kind = %s
+with V.VPM(V.Params.make(0.125)) as c:
+    c.upload(*cloud(SMALL))  # (its buffer is there)
+    for k in (1, 2, 3, 2, 1, 4):
+        F.fake_fail(kind, k)
+        round_trip(c, LARGE)
+        assert F.fake_last_error() == 0, k
+    F.fake_fail(kind, -1)
+    for n in (LARGE, SMALL, LARGE):
+        round_trip(c, n)
+    assert F.fake_last_error() == 0
+    F.fake_fail(kind, 0)
+    round_trip(c, LARGE)
+assert F.fake_held(1) <= 8, F.fake_held(1)
+""" % kind)
+
+
+def test_transfers_without_pinned_memory(run):
+    """No pinned memory at all: every transfer goes through the runtime's own copies, and the evaluation
+    after it finds no error."""
+    run(TRANSFERS + """
+F.fake_fail(HOSTMALLOC, -1)
+with V.VPM(V.Params.make(0.125)) as c:
+    for n in (SMALL, LARGE, SMALL):
+        round_trip(c, n)
+        assert F.fake_last_error() == 0, n
+    x, q = cloud(SMALL)
+    up, gp = np.zeros_like(x), np.zeros_like(x)
+    c.vpm(x, q, up, gp, SMALL, 3, 0, 0)
+    c.vpm(x, q, up, gp, SMALL, 3, 2, 1)
+assert F.fake_held(1) == 0
+""")

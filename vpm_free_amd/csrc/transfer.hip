@@ -8,7 +8,8 @@
 //   * larger ones are cut into chunks that several threads move through pinned slots, each with a
 //     copy in flight while it touches the other slot's host side (the page faults of a fresh
 //     result array spread over the threads too).  The slots and the threads' streams are one set
-//     per device, used by one transfer at a time and given back with the device's last context.
+//     per device, used by one transfer at a time and given back with the device's last context;
+//   * where no pinned memory is to be had, the runtime copies.
 // Particles in (MB: us) by the runtime / the pinned buffer / chunks: 0.11: 57 / 25 / 43; 1.9: 85 /
 // 72 / 108; 3.8: 146 / 120 / 168; 7.7: 254 / 233 / 303; 214: 7814 / 9742 / 4290.  Out: 0.2: 128 / 50 / 98;
 // 3.6: 213 / 206 / 191; 7.1: 1347 / 412 / 387; 14: 2549 / 794 / 459; 397: 39800 / 38200 / 9420.
@@ -43,18 +44,11 @@ struct Slots {
     char *mem[MAX_THREADS] = {};
     hipStream_t stream[MAX_THREADS] = {};
     hipEvent_t done[MAX_THREADS][2] = {};
-    // at least n threads' slots; the number there are (fewer when memory is short)
+    // at least n threads' slots; the number there are (fewer when memory is short; what a thread
+    // got before the call that failed stays for the next attempt)
     int grow(int n) {
-        while (ready < n) {
-            const int t = ready;
-            void *p = nullptr;
-            if (hipHostMalloc(&p, 2 * CHUNK, hipHostMallocDefault) != hipSuccess) break;
-            mem[t] = (char *)p;
-            if (hipStreamCreateWithFlags(&stream[t], hipStreamNonBlocking) != hipSuccess) break;
-            if (hipEventCreateWithFlags(&done[t][0], hipEventDisableTiming) != hipSuccess) break;
-            if (hipEventCreateWithFlags(&done[t][1], hipEventDisableTiming) != hipSuccess) break;
-            ready++;
-        }
+        while (ready < n && set_up(ready)) ready++;
+        if (ready < n) (void)hipGetLastError();  // (not an error of the transfer)
         return std::min(ready, n);
     }
     ~Slots() {
@@ -65,6 +59,27 @@ struct Slots {
             if (stream[t]) (void)hipStreamDestroy(stream[t]);
             if (mem[t]) (void)hipHostFree(mem[t]);
         }
+    }
+
+private:
+    bool set_up(int t) {
+        void *p = nullptr;
+        hipStream_t s;
+        hipEvent_t e;
+        if (!mem[t]) {
+            if (hipHostMalloc(&p, 2 * CHUNK, hipHostMallocDefault) != hipSuccess) return false;
+            mem[t] = (char *)p;
+        }
+        if (!stream[t]) {
+            if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return false;
+            stream[t] = s;
+        }
+        for (hipEvent_t &d : done[t])
+            if (!d) {
+                if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+                d = e;
+            }
+        return true;
     }
 };
 
@@ -110,20 +125,30 @@ hipError_t move_chunks(Slots &S, int t, bool in, const std::vector<Copy> &ch, st
     return e != hipSuccess ? e : last;
 }
 
+// The runtime's own copies.
+int copy_direct(Ctx *c, bool in, const Copy *q, int n) {
+    for (int i = 0; i < n; i++)
+        if (q[i].bytes)
+            VPMX_HIP(c, hipMemcpyAsync(q[i].dst, q[i].src, q[i].bytes,
+                                       in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, c->stream));
+    VPMX_HIP(c, hipStreamSynchronize(c->stream));
+    return VPMX_OK;
+}
+
 int copy_large(Ctx *c, bool in, const Copy *q, int n, size_t total) try {
     if (!c->slots) c->slots = slots_of(c->device);
     Slots &S = *static_cast<Slots *>(c->slots.get());
+    std::vector<Copy> ch;
+    for (int i = 0; i < n; i++)
+        for (size_t o = 0; o < q[i].bytes; o += CHUNK)
+            ch.push_back({(char *)q[i].dst + o, (const char *)q[i].src + o, std::min(CHUNK, q[i].bytes - o)});
     VPMX_HIP(c, hipStreamSynchronize(c->stream));  // what the copies read or overwrite
     std::lock_guard<std::mutex> lock(S.use);
     int nt = (int)std::min<size_t>(MAX_THREADS, total / PER_THREAD);
     const int cpus = (int)std::thread::hardware_concurrency();
     if (cpus > 0) nt = std::min(nt, cpus / 2);
     nt = S.grow(std::max(nt, 1));
-    if (nt < 1) return fail(c, VPMX_ERR_HIP, "pinned memory for the copies");
-    std::vector<Copy> ch;
-    for (int i = 0; i < n; i++)
-        for (size_t o = 0; o < q[i].bytes; o += CHUNK)
-            ch.push_back({(char *)q[i].dst + o, (const char *)q[i].src + o, std::min(CHUNK, q[i].bytes - o)});
+    if (nt < 1) return copy_direct(c, in, q, n);
     std::atomic<size_t> next{0};
     hipError_t err[MAX_THREADS];
     std::fill(err, err + MAX_THREADS, hipSuccess);
@@ -138,11 +163,11 @@ int copy_large(Ctx *c, bool in, const Copy *q, int n, size_t total) try {
     for (std::thread &t : th) t.join();
     for (hipError_t e : err) VPMX_HIP(c, e);
     return VPMX_OK;
-} catch (const std::bad_alloc &) {
-    return fail(c, VPMX_ERR_HIP, "host memory for the copies");
+} catch (const std::bad_alloc &) {  // (before the first copy)
+    return copy_direct(c, in, q, n);
 }
 
-// The context's pinned buffer, no longer read by an earlier copy.
+// The context's pinned buffer, no longer read by an earlier copy; null when there is no memory.
 int small_buffer(Ctx *c, size_t bytes, char **out) {
     if (c->pin_busy) VPMX_HIP(c, hipStreamSynchronize(c->stream));
     c->pin_busy = false;
@@ -150,8 +175,12 @@ int small_buffer(Ctx *c, size_t bytes, char **out) {
         if (c->pin) (void)hipHostFree(c->pin);
         c->pin = nullptr;
         c->pin_bytes = 0;
-        VPMX_HIP(c, hipHostMalloc(&c->pin, bytes + bytes / 4, hipHostMallocDefault));
-        c->pin_bytes = bytes + bytes / 4;
+        if (hipHostMalloc(&c->pin, bytes + bytes / 4, hipHostMallocDefault) == hipSuccess) {
+            c->pin_bytes = bytes + bytes / 4;
+        } else {
+            (void)hipGetLastError();
+            c->pin = nullptr;
+        }
     }
     *out = (char *)c->pin;
     return VPMX_OK;
@@ -187,15 +216,6 @@ bool any_direct(bool in, const Copy *q, int n) {
     return false;
 }
 
-int copy_direct(Ctx *c, bool in, const Copy *q, int n) {
-    for (int i = 0; i < n; i++)
-        if (q[i].bytes)
-            VPMX_HIP(c, hipMemcpyAsync(q[i].dst, q[i].src, q[i].bytes,
-                                       in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, c->stream));
-    VPMX_HIP(c, hipStreamSynchronize(c->stream));
-    return VPMX_OK;
-}
-
 }  // namespace
 
 int copy_in(Ctx *c, const Copy *q, int n) {
@@ -206,6 +226,7 @@ int copy_in(Ctx *c, const Copy *q, int n) {
     if (total > SMALL_COPY) return copy_large(c, true, q, n, total);
     char *b = nullptr;
     VPMX_TRY(small_buffer(c, total, &b));
+    if (!b) return copy_direct(c, true, q, n);
     for (int i = 0; i < n; i++) {
         if (!q[i].bytes) continue;
         std::memcpy(b, q[i].src, q[i].bytes);
@@ -224,6 +245,7 @@ int copy_out(Ctx *c, const Copy *q, int n) {
     if (total > SMALL_COPY) return copy_large(c, false, q, n, total);
     char *b = nullptr;
     VPMX_TRY(small_buffer(c, total, &b));
+    if (!b) return copy_direct(c, false, q, n);
     c->pin_busy = true;
     char *p = b;
     for (int i = 0; i < n; i++) {
