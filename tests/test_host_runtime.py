@@ -85,6 +85,19 @@ LARGE, SMALL = 700000, 500  # 39 MB in chunks, 28 kB through the pinned buffer
 """
 
 
+def test_transfer_slots_serve_every_context(run):
+    """Contexts one after another: the pinned slots and streams of large transfers are set up once."""
+    run(TRANSFERS + """
+for turn in range(4):
+    with V.VPM(V.Params.make(0.125)) as c:
+        base = F.fake_done(STREAM), F.fake_done(HOSTMALLOC)
+        round_trip(c, LARGE)
+        new = F.fake_done(STREAM) - base[0], F.fake_done(HOSTMALLOC) - base[1]
+        assert (min(new) > 0) if turn == 0 else new == (0, 0), (turn, new)
+assert F.fake_held(1) <= 8
+""")
+
+
 @pytest.mark.parametrize("kind", ["HOSTMALLOC", "STREAM", "EVENT"])
 def test_transfer_slots_that_cannot_grow(run, kind):
     """A refused allocation while the slots are set up leaves fewer of them, no error behind, and nothing

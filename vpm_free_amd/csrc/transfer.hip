@@ -8,7 +8,7 @@
 //   * larger ones are cut into chunks that several threads move through pinned slots, each with a
 //     copy in flight while it touches the other slot's host side (the page faults of a fresh
 //     result array spread over the threads too).  The slots and the threads' streams are one set
-//     per device, used by one transfer at a time and given back with the device's last context;
+//     per device, used by one transfer at a time;
 //   * where no pinned memory is to be had, the runtime copies.
 // Particles in (MB: us) by the runtime / the pinned buffer / chunks: 0.11: 57 / 25 / 43; 1.9: 85 /
 // 72 / 108; 3.8: 146 / 120 / 168; 7.7: 254 / 233 / 303; 214: 7814 / 9742 / 4290.  Out: 0.2: 128 / 50 / 98;
@@ -51,15 +51,6 @@ struct Slots {
         if (ready < n) (void)hipGetLastError();  // (not an error of the transfer)
         return std::min(ready, n);
     }
-    ~Slots() {
-        (void)hipSetDevice(device);
-        for (int t = 0; t < MAX_THREADS; t++) {
-            for (hipEvent_t e : done[t])
-                if (e) (void)hipEventDestroy(e);
-            if (stream[t]) (void)hipStreamDestroy(stream[t]);
-            if (mem[t]) (void)hipHostFree(mem[t]);
-        }
-    }
 
 private:
     bool set_up(int t) {
@@ -83,18 +74,20 @@ private:
     }
 };
 
-// The device's slots, shared by its contexts.
-std::shared_ptr<Slots> slots_of(int device) {
+// The device's slots, shared by its contexts and kept until the process ends (32 MB pinned and eight
+// streams a device at most): to set them up and run their first copies takes 8 ms, 40 ms in a new
+// process, and to take them down 3 ms, as much as they save on a transfer of 200 MB, which a program
+// that opens a context per evaluation would pay each time.
+Slots &slots_of(int device) {
     static std::mutex m;
-    static std::map<int, std::weak_ptr<Slots>> all;
+    static auto *all = new std::map<int, std::unique_ptr<Slots>>;  // (outlives the runtime's own shutdown)
     std::lock_guard<std::mutex> lock(m);
-    std::shared_ptr<Slots> s = all[device].lock();
+    std::unique_ptr<Slots> &s = (*all)[device];
     if (!s) {
-        s = std::make_shared<Slots>();
+        s.reset(new Slots());
         s->device = device;
-        all[device] = s;
     }
-    return s;
+    return *s;
 }
 
 // Moves chunks (taken off `next`) through thread t's two slots.
@@ -136,8 +129,7 @@ int copy_direct(Ctx *c, bool in, const Copy *q, int n) {
 }
 
 int copy_large(Ctx *c, bool in, const Copy *q, int n, size_t total) try {
-    if (!c->slots) c->slots = slots_of(c->device);
-    Slots &S = *static_cast<Slots *>(c->slots.get());
+    Slots &S = slots_of(c->device);
     std::vector<Copy> ch;
     for (int i = 0; i < n; i++)
         for (size_t o = 0; o < q[i].bytes; o += CHUNK)
@@ -266,7 +258,6 @@ void free_transfer(Ctx *c) {
     if (c->pin) (void)hipHostFree(c->pin);
     c->pin = nullptr;
     c->pin_bytes = 0;
-    c->slots.reset();
 }
 
 }  // namespace vpmx

@@ -1,7 +1,6 @@
 // The context behind the opaque vpmx_ctx handle.
 #pragma once
 #include <map>
-#include <memory>
 #include <string>
 #include <array>
 #include <vector>
@@ -40,12 +39,11 @@ struct Ctx : vpmx_ctx {
     vpmx_geom geom{};
     int precision = 0;
 
-    // copies to and from the caller's arrays (transfer.hip): the pinned buffer of small ones (busy:
-    // a copy into the device may still read it), the device's slots of large ones
+    // copies to and from the caller's arrays (transfer.hip): the pinned buffer of small ones, at most
+    // 5 MB (busy: a copy into the device may still read it)
     void *pin = nullptr;
     size_t pin_bytes = 0;
     bool pin_busy = false;
-    std::shared_ptr<void> slots;
 
     // resident particles
     DBuf xp, qp, up, gp, x0, q0;
