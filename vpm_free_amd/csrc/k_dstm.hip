@@ -34,11 +34,13 @@ typedef double dm_acc __attribute__((ext_vector_type(4)));
 // Longest lines of the matrix passes.  The products grow with the square of the length, the FFT
 // passes hardly, but these depend on the factors of m + 1.  Whole solves of m^3 points, 3
 // components, us, products against FFT.  FP64: 231 (8.29) 1233/4330, 239 1289/1489, 255 1548/1650,
-// 263 (8.3.11) 1980/2991, 271 (16.17) 2065/2450, 279 2323/2489, 287 (32.9) 2420/2212, 303 3155/13325,
-// 319 4355/6821, 367 7405/23249 -- the products but for the 288-point transform, whose z forward
-// pass alone loses too (465 against 618).  FP32 arrays (FP64 sums: half the bytes, the same
-// products): 191 481/563, 207 759/881, 215 847/793, 239 1189/1139, 255 1332/1117, 271 1907/1261,
-// but with factors over 17 (no register transform) 231 1139/3079, 247 1296/3649.
+// 263 (8.3.11) 1980/2991, 271 (16.17) 2065/2450, 279 2323/2489, and above 287 points, where an FFT line
+// no longer fits one wave, 303 3155/13325, 319 4355/6821, 367 7405/23249.  The 288-point transform has a
+// compile-time FFT plan and keeps it (by axis, products against FFT: x forward 600/425, y 440/370, z
+// 800/806, x inverse 550/385); only z forward alone is the products' (465/618).  FP32 arrays (FP64
+// sums: half the bytes, the same products): 191 481/563, 207 759/881, 215 847/793, 239 1189/1139, 255
+// 1332/1117, 271 1907/1261, but with factors over 17 (no register transform) 231 1139/3079, 247
+// 1296/3649.
 // DM_MAX: three row blocks a wave (24 of them).
 constexpr int DM_MAX = 367, DM_MAX32 = 208, DM_PLANE = 224;
 constexpr int DM_PAD = 8;  // zero rows after a line: the products run over whole pairs of k-steps
@@ -559,8 +561,7 @@ static int dm_without(int n, int p) {
 bool dstm_line_fits(int m, bool f32, bool forward) {
     if (m < 1 || m > DM_MAX) return false;
     if (f32) return m <= DM_MAX32 || dm_without(m + 1, 17) > 1;
-    const bool fft = m >= 256 && m < 288 && dm_without(m + 1, 3) == 1;
-    return forward || !fft;
+    return forward || m + 1 != 288;  // (the FP64 length with an FFT plan of its own)
 }
 
 static int dm_pitch(int m) {  // 2 (mod 4): 16 lines of two neighbouring points fall on all banks
