@@ -225,6 +225,7 @@ static int yaps_single(Ctx *c, bool *used) {
     int ns[3];
     std::vector<int> cmap;
     int fp_lo[3], fp_hi[3];
+    bool consecutive = true;  // the samples' coarse nodes (not when ncoarse changed after mode 0)
     for (int d = 0; d < 3; d++) {
         ns[d] = (nb[d] - 1) / ncs + 1;
         for (int a = 0; a < ns[d]; a++) {
@@ -232,6 +233,7 @@ static int yaps_single(Ctx *c, bool *used) {
             double X = G.xbound_bl[d] + (double)(i - 1) * G.dpm[d];
             int node = (int)std::lround((X - G.xbound_coarse[d]) / G.dpm_coarse[d]) + 1;
             if (node < 1 || node > cn[d]) return fail(c, VPMX_ERR_STATE, "coarse sample outside the coarse grid");
+            consecutive = consecutive && (a == 0 || node == cmap.back() + 1);
             cmap.push_back(node);
         }
         fp_lo[d] = cmap[cmap.size() - ns[d]];
@@ -240,9 +242,15 @@ static int yaps_single(Ctx *c, bool *used) {
         // of ncoarse the last sample is i = NNbl
     }
     GView smv = view(samp, cn), rcv = view(rhsc, cn), scv = view(solc, cn);
-    for (int d = 0; d < 3; d++)
-        if (fp_hi[d] - fp_lo[d] != ns[d] - 1) return fail(c, VPMX_ERR_STATE, "block samples are not consecutive coarse nodes");
-    VPMX_TRY(coarse_problem(c, 3, cn, fp_lo, fp_hi, ncs, G.dpm_coarse, sv, smv, rcv));
+    if (consecutive) {
+        VPMX_TRY(coarse_problem(c, 3, cn, fp_lo, fp_hi, ncs, G.dpm_coarse, sv, smv, rcv));
+    } else {
+        int *cmap_d = nullptr;
+        VPMX_TRY(upload_cmap(c, cmap, &cmap_d));
+        VPMX_TRY(fill(c, samp, 3 * GC, 0.0));
+        VPMX_TRY(coarse_sample(c, 3, ns, ncs, cmap_d, sv, smv, cn));
+        VPMX_TRY(coarse_laplacian(c, 3, cn, fp_lo, fp_hi, G.dpm_coarse, smv, rcv));
+    }
     Grid gc = make_grid(G.nn_coarse, G.xbound_coarse, G.dpm_coarse);
     VPMX_TRY(pmesh_inf(c, gc, rcv, scv, c->sol0_c, false, tree ? G.ilevmax - 1 : -1, P.ibctyp, true));
     mark(c, ST_COARSE, 1);
