@@ -135,3 +135,55 @@ with V.VPM(V.Params.make(0.125)) as c:
     c.vpm(x, q, up, gp, SMALL, 3, 2, 1)
 assert F.fake_held(1) == 0
 """)
+
+
+def test_every_line_length_has_its_passes(run):
+    """Solves with one axis of 1 to 420 points, in both precisions, find kernels for every length that
+    the transform plans take (prime factors of m + 1 up to 64)."""
+    run("""
+def factor(n):
+    p = 2
+    while n > 1:
+        while n % p == 0:
+            n //= p
+        if n > 1:
+            p += 1
+    return p
+win = lambda nn: np.array([1, 1, 1, *nn], np.int32)
+for prec in (0, 1):
+    with V.VPM(V.Params.make(0.125)) as c:
+        c.set_precision(prec)
+        for m in range(1, 421):
+            for axis in range(3):
+                nn = np.array([9, 10, 11], np.int32)
+                nn[axis] = m + 2
+                a = np.zeros((nn[2], nn[1], nn[0], 3))
+                args = (np.zeros(6), np.full(3, 0.1), nn, 3, win(nn), a)
+                if factor(m + 1) > 64:
+                    assert fails(c.stage_solve, *args), m
+                else:
+                    c.stage_solve(*args)
+                    c.stage_solve(*args, None, True)
+""")
+
+
+def test_every_block_length_in_the_mixed_form(run):
+    """Evaluations in the mixed form (its inner-box solves return in FP64) of boxes with one axis of up
+    to 330 nodes."""
+    run("""
+h = 0.125
+with V.VPM(V.Params.make(h)) as c:
+    c.set_precision(1)
+    for axis in range(3):
+        for cells in range(6, 330, 8):
+            ext = np.full(3, 3.0)
+            ext[axis] = cells
+            x = np.stack([np.zeros(3), ext * h])
+            q = np.ones((2, 4))
+            up, gp = np.zeros_like(x), np.zeros_like(x)
+            c.vpm(x, q, up, gp, 2, 3, 0, 0)
+            try:
+                c.vpm(x, q, up, gp, 2, 3, 2, 1)
+            except V.VpmError as e:
+                assert "prime factor" in str(e) or "too long" in str(e), (axis, cells, str(e))
+""")

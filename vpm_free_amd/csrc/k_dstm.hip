@@ -561,7 +561,7 @@ static int dm_without(int n, int p) {
 bool dstm_line_fits(int m, bool f32, bool forward) {
     if (m < 1 || m > DM_MAX) return false;
     if (f32) return m <= DM_MAX32 || dm_without(m + 1, 17) > 1;
-    return forward || m + 1 != 288;  // (the FP64 length with an FFT plan of its own)
+    return forward || m + 1 != FFT64_LENGTH;
 }
 
 static int dm_pitch(int m) {  // 2 (mod 4): 16 lines of two neighbouring points fall on all banks

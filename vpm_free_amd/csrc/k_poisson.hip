@@ -1098,18 +1098,18 @@ __host__ __device__ constexpr int wave_cap(bool dbl, int mode, int fix) {
 // everything after the diagonal runs, and is stored, in FP64.  Each wave's LDS region holds
 // either form's sequence (the FP32 one of 2(m+1) points and the FP64 one of m+1 points take
 // the same bytes); between the two transforms a wave holds the diagonal's outputs in
-// registers.
-template <int MAXR, int FIX32, int FIX64>
-__device__ __forceinline__ void dst_zmix_body(const DstArgs &a, const WavePlan &P32, const WavePlan &P64,
-                                              const double2 *__restrict__ tw64) {
+// registers.  Lines of 287 points only (the compile-time plans of 576 and 288 points): the other
+// lengths' FP64 inverse is a matrix product (k_dstm.hip).
+constexpr int ZMIX_FIX32 = 0, ZMIX_FIX64 = 2;
+static_assert(FixedFft<ZMIX_FIX64>::L == FFT64_LENGTH && FixedFft<ZMIX_FIX32>::L == 2 * FFT64_LENGTH, "one line length");
+__global__ void __launch_bounds__(DST_THREADS) k_dst_zmix(DstArgs a, const double2 *__restrict__ tw64) {
 #pragma clang fp contract(off)
+    constexpr int FIX32 = ZMIX_FIX32, FIX64 = ZMIX_FIX64;
     extern __shared__ double2 lds_raw[];
     __shared__ double lamxy[16];
     __shared__ double lzs[WAVE_LMAX];
     constexpr int nl = WV_NL;
-    const int N32 = FIX32 >= 0 ? fix_len<FIX32>() : P32.L;  // 2(m+1)
-    const int N64 = FIX64 >= 0 ? fix_len<FIX64>() : P64.L;  // m+1
-    const int m = N64 - 1;
+    constexpr int N32 = fix_len<FIX32>(), N64 = fix_len<FIX64>(), m = N64 - 1;  // 2(m+1), m+1
     const int nbatch = (int)((a.nlines + nl - 1) / nl);
     constexpr int S32 = wave_pad_shift(false, DST_Z, FIX32), S64 = wave_pad_shift(true, DST_Z, FIX64);
     constexpr bool CR32 = const_roots(false, DST_Z, FIX32), CR64 = const_roots(true, DST_Z, FIX64);
@@ -1169,8 +1169,7 @@ __device__ __forceinline__ void dst_zmix_body(const DstArgs &a, const WavePlan &
         // forward transform in FP32
         if (lane == 0) B32[0] = B32[m + 1] = make_float2(0.f, 0.f);
         __builtin_amdgcn_wave_barrier();
-        if constexpr (FIX32 >= 0) FixedFft<FIX32>::template run<float2, Buf32, CR32>(B32, tw32l, lane);
-        else wave_fft<MAXR>(B32, tw32l, P32, lane);
+        FixedFft<FIX32>::template run<float2, Buf32, CR32>(B32, tw32l, lane);
         // F = (-Im Z/2, Re Z/2) times -norm / lambda in FP64 (the FP32 values convert exactly),
         // held in registers while the region changes form
         const double la = lamxy[2 * wave], lb = lamxy[2 * wave + 1];
@@ -1196,8 +1195,7 @@ __device__ __forceinline__ void dst_zmix_body(const DstArgs &a, const WavePlan &
         __builtin_amdgcn_wave_barrier();
         // inverse transform in FP64 (half-length form)
         wave_pre<double2>(B64, a.sn, N64, lane, nullptr, 0.0);
-        if constexpr (FIX64 >= 0) FixedFft<FIX64>::template run<double2, Buf64, CR64>(B64, tw64l, lane);
-        else wave_fft<MAXR>(B64, tw64l, P64, lane);
+        FixedFft<FIX64>::template run<double2, Buf64, CR64>(B64, tw64l, lane);
         wave_post<double2>(B64, N64, lane);
         __syncthreads();
         const WaveAddr ad = wave_addr<DST_Z>(a, comp, b * nl + tline, tpt0);
@@ -1212,11 +1210,6 @@ __device__ __forceinline__ void dst_zmix_body(const DstArgs &a, const WavePlan &
         comp = compn;
         b = bn;
     }
-}
-
-template <int MAXR, int FIX32, int FIX64>
-__global__ void __launch_bounds__(DST_THREADS) k_dst_zmix(DstArgs a, WavePlan P32, WavePlan P64, const double2 *tw64) {
-    dst_zmix_body<MAXR, FIX32, FIX64>(a, P32, P64, tw64);
 }
 
 // Zero the six faces of a window (zero Dirichlet values of solve_eq_0_3d).
@@ -1464,17 +1457,10 @@ static int launch_wave(Ctx *c, DstArgs a, int ncomp, int rc, const FftPlan *fp) 
     }
     a.npairs = 8;
     // compile-time plans for the lengths of the common block sizes
-    auto same = [&](const int *rr, int n) {
-        if (fp->nstages != n) return false;
-        for (int q = 0; q < n; q++)
-            if (fp->radix[q] != rr[q]) return false;
-        return true;
-    };
-    static const int r576[] = {4, 4, 4, 3, 3}, r288[] = {4, 4, 2, 3, 3}, r544[] = {4, 4, 2, 17};
     int fix = -1;
-    if (sizeof(T) == 4 && fp->L == 576 && same(r576, 5)) fix = 0;
-    if (sizeof(T) == 8 && fp->L == 288 && same(r288, 5)) fix = 2;
-    if (sizeof(T) == 4 && fp->L == 544 && same(r544, 4)) fix = 5;
+    if (sizeof(T) == 4 && fp->L == 576) fix = 0;
+    if (sizeof(T) == 8 && fp->L == FFT64_LENGTH) fix = 2;
+    if (sizeof(T) == 4 && fp->L == 544) fix = 5;
     // kernel variants: with a compile-time plan the registers capped for four waves per SIMD
     // (six for the FP32 x inverse of the 576-point plan) or not, each in both batch orders;
     // FP32 compile-time plans also with 32-line batches (1024 threads) -- the tuner times all
@@ -1556,10 +1542,13 @@ static int launch_wave(Ctx *c, DstArgs a, int ncomp, int rc, const FftPlan *fp) 
             }
         }
     } else {
-        fix = -1;
-        const void *f = rc == 4 ? (const void *)k_dst_wave<MODE, 4, T, -1>
-                      : rc == 7 ? (const void *)k_dst_wave<MODE, 7, T, -1>
-                      : rc == 17 ? (const void *)k_dst_wave<MODE, 17, T, -1> : (const void *)k_dst_wave<MODE, 37, T, -1>;
+        // runtime plans: FP32 lines (the other FP64 lengths, and factors over 17, take products)
+        const void *f = nullptr;
+        if constexpr (!dbl)
+            f = rc == 4 ? (const void *)k_dst_wave<MODE, 4, T, -1>
+              : rc == 7 ? (const void *)k_dst_wave<MODE, 7, T, -1>
+              : rc == 17 ? (const void *)k_dst_wave<MODE, 17, T, -1> : nullptr;
+        if (!f) return fail(c, VPMX_ERR_STATE, "sine transforms: no one-wave plan of " + std::to_string(fp->L) + " points");
         add(f, "uncapped", 16, 0, -1);
         add(f, "uncapped, batch halves in turn", 16, 1, -1);
     }
@@ -1645,68 +1634,24 @@ static int launch_wave(Ctx *c, DstArgs a, int ncomp, int rc, const FftPlan *fp) 
     return VPMX_OK;
 }
 
-static WavePlan wave_plan(const FftPlan *fp) {
-    WavePlan P{};
-    P.L = fp->L;
-    P.nstages = fp->nstages;
-    int ns = 1;
-    for (int s = 0; s < fp->nstages; s++) {
-        P.R[s] = fp->radix[s];
-        P.Ns[s] = ns;
-        P.mg[s] = ns > 1 ? (unsigned)((1ull << 32) / (unsigned long long)ns + 1ull) : 0u;
-        ns *= fp->radix[s];
-    }
-    return P;
-}
-
 // The mixed z pass (k_dst_zmix) on the FP32 work array a.w, FP64 results into wo.
 static int launch_zmix(Ctx *c, DstArgs a, int ncomp, const AxisPlan &X, double *wo) {
     const FftPlan *f32 = X.full, *f64 = X.half;
-    const WavePlan P32 = wave_plan(f32), P64 = wave_plan(f64);
     setup_axis(a, (FftPlan *)f32, X.m);
-    const int rc32 = radix_class(a);
-    DstArgs ah = a;
-    setup_axis(ah, (FftPlan *)f64, X.m);
-    const int rc64 = radix_class(ah);
-    const int rc = rc32 > rc64 ? rc32 : rc64;
     a.sn = X.sn;
     a.wo = wo;
     a.npairs = 8;
     a.ncomp = ncomp;
-    auto same = [](const FftPlan *fp, const int *rr, int n) {
-        if (fp->nstages != n) return false;
-        for (int q = 0; q < n; q++)
-            if (fp->radix[q] != rr[q]) return false;
-        return true;
-    };
-    static const int r576[] = {4, 4, 4, 3, 3}, r288[] = {4, 4, 2, 3, 3};
-    // kernels (compile-time plans of both forms, or runtime plans), each in both batch orders
-    struct ZK {
-        const void *fn;
-        int fix32, fix64;
-        const char *name;
-    };
-    ZK zk;
-    if (f32->L == 576 && same(f32, r576, 5) && f64->L == 288 && same(f64, r288, 5)) {
-        zk = {(const void *)k_dst_zmix<4, 0, 2>, 0, 2, "FP32 forward, FP64 inverse"};
-    } else {
-        zk = {rc == 4 ? (const void *)k_dst_zmix<4, -1, -1>
-                 : rc == 7 ? (const void *)k_dst_zmix<7, -1, -1>
-                 : rc == 17 ? (const void *)k_dst_zmix<17, -1, -1> : (const void *)k_dst_zmix<37, -1, -1>,
-                 -1, -1, "FP32 forward, FP64 inverse"};
-    }
-    // the kernel's LDS layout: eight regions of Wq double2 slots, then both twiddle tables
-    auto lds_of = [&](int fix32, int fix64) {
-        const int S32 = wave_pad_shift(false, DST_Z, fix32), S64 = wave_pad_shift(true, DST_Z, fix64);
-        const int Np32 = S32 == 0 ? pad_len<0>(f32->L) : S32 == 3 ? pad_len<3>(f32->L) : pad_len<4>(f32->L);
-        const int Np64 = S64 == 0 ? pad_len<0>(f64->L) : S64 == 3 ? pad_len<3>(f64->L) : pad_len<4>(f64->L);
-        const int Wq = (Np32 + 1) / 2 > Np64 ? (Np32 + 1) / 2 : Np64;
-        return sizeof(double2) * (size_t)(8 * Wq + f32->L / 2 + f64->L);
-    };
-    const std::string swapped = std::string(zk.name) + ", batch halves in turn";
-    const void *fns[2] = {zk.fn, zk.fn};
-    const char *names[2] = {zk.name, swapped.c_str()};
-    const size_t ldsv[2] = {lds_of(zk.fix32, zk.fix64), lds_of(zk.fix32, zk.fix64)};
+    // the kernel in both batch orders; its LDS layout: eight regions of Wq double2 slots, then both
+    // twiddle tables
+    constexpr int S32 = wave_pad_shift(false, DST_Z, ZMIX_FIX32), S64 = wave_pad_shift(true, DST_Z, ZMIX_FIX64);
+    const int Np32 = pad_len<S32>(f32->L), Np64 = pad_len<S64>(f64->L);
+    const int Wq = (Np32 + 1) / 2 > Np64 ? (Np32 + 1) / 2 : Np64;
+    const size_t lds = sizeof(double2) * (size_t)(8 * Wq + f32->L / 2 + f64->L);
+    const void *fn = (const void *)k_dst_zmix;
+    const void *fns[2] = {fn, fn};
+    const char *names[2] = {"FP32 forward, FP64 inverse", "FP32 forward, FP64 inverse, batch halves in turn"};
+    const size_t ldsv[2] = {lds, lds};
     const int thr[2] = {DST_THREADS, DST_THREADS};
     const int64_t nbatch = (a.nlines + 15) / 16;
     auto grid_of = [&](int per_cu) {
@@ -1733,21 +1678,17 @@ static int launch_zmix(Ctx *c, DstArgs a, int ncomp, const AxisPlan &X, double *
             t.order = fi & 1;
             t.w = (double *)c->tune_scratch.p;
             t.wo = (double *)((char *)c->tune_scratch.p + sizeof(float) * (size_t)a.wcs * ncomp);
-            WavePlan p32 = P32, p64 = P64;
             const double2 *t64 = f64->tw;
-            void *targs[] = {&t, &p32, &p64, &t64};
-            VPMX_HIP(c, hipLaunchKernel(fns[fi], grid_of(pc), dim3(DST_THREADS), targs, ldsv[fi], c->stream));
+            void *targs[] = {&t, &t64};
+            VPMX_HIP(c, hipLaunchKernel(fn, grid_of(pc), dim3(DST_THREADS), targs, lds, c->stream));
             return VPMX_OK;
         };
         VPMX_TRY(tune_v(c, key, 2, fns, names, ldsv, thr, trial, &ch));
     }
     a.order = ch.fi & 1;
-    const void *fn = fns[ch.fi];
-    const size_t lds = ldsv[ch.fi];
     dim3 grid = grid_of(ch.per_cu);
     const double2 *tw64 = f64->tw;
-    WavePlan p32 = P32, p64 = P64;
-    void *args[] = {&a, &p32, &p64, &tw64};
+    void *args[] = {&a, &tw64};
     hipEvent_t e0, e1;
     if (a.m == c->dst_timed_m && kernel_events(c, K_DSTZ, &e0, &e1)) {
         // FP32 read + FP64 write of every interior point
@@ -1760,13 +1701,11 @@ static int launch_zmix(Ctx *c, DstArgs a, int ncomp, const AxisPlan &X, double *
     return VPMX_OK;
 }
 
-// The one-wave-per-pair kernel: FP64 lines of up to WAVE_LMAX - 1 points (FFT of m+1),
-// FP32 lines of up to WAVE_LMAX_F / 2 - 1 points (FFT of 2(m+1)), radices up to 37.
-static int wave_class(const AxisPlan &P, bool f32) {
-    const FftPlan *fp = f32 ? P.full : P.half;
-    if (fp->L > (f32 ? WAVE_LMAX_F : WAVE_LMAX) || fp->nstages > 12) return 0;
+// FP32 lines: up to WAVE_LMAX_F / 2 - 1 points (an FFT of 2(m+1) points in one wave), radices up to 37.
+static int wave_class(const AxisPlan &P) {
+    if (P.full->L > WAVE_LMAX_F || P.full->nstages > 12) return 0;
     DstArgs a{};
-    setup_axis(a, (FftPlan *)fp, P.m);
+    setup_axis(a, P.full, P.m);
     return radix_class(a);
 }
 
@@ -1774,13 +1713,12 @@ template <int MODE>
 static int run_pass(Ctx *c, DstArgs a, int ncomp, const AxisPlan &P, bool f32) {
     if (f32) {
         setup_axis(a, P.full, P.m);
-        return launch_wave<MODE, float>(c, a, ncomp, wave_class(P, true), P.full);
+        return launch_wave<MODE, float>(c, a, ncomp, wave_class(P), P.full);
     }
-    const int wc = wave_class(P, false);
-    if (c->dst_kernel == 4 && wc) {
+    if (c->dst_kernel == 4 && P.half->L == FFT64_LENGTH) {
         setup_axis(a, P.half, P.m);
         a.sn = P.sn;
-        return launch_wave<MODE, double>(c, a, ncomp, wc, P.half);
+        return launch_wave<MODE, double>(c, a, ncomp, 0, P.half);
     }
     if (c->dst_kernel >= 3) {
         setup_axis(a, P.half, P.m);
@@ -2441,26 +2379,24 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     VPMX_TRY(eigen(c, m[2], h[2], c->lam[2], &a.lam[2]));
     a.norm = (2.0 / (m[0] + 1)) * (2.0 / (m[1] + 1)) * (2.0 / (m[2] + 1));
     a.scale = 1.0;
-    // the FP32 passes run when every axis takes the one-wave kernel in both forms; SOLVE_CTX
-    // follows the context's precision (FP32 passes in the mixed form)
+    // the FP32 passes run when every axis' FP32 line fits the one-wave kernel; SOLVE_CTX follows the
+    // context's precision (FP32 passes in the mixed form)
     if (form == SOLVE_CTX) form = c->precision == 1 ? SOLVE_FP32 : SOLVE_FP64;
-    const bool wave32 = wave_class(ax[0], true) && wave_class(ax[1], true) && wave_class(ax[2], true);
-    const bool wave64 = wave_class(ax[0], false) && wave_class(ax[1], false) && wave_class(ax[2], false);
+    const bool wave32 = wave_class(ax[0]) && wave_class(ax[1]) && wave_class(ax[2]);
     // small grids in every form: FP64 products, whole planes per work-group (three launches)
     const bool planes = c->dst_kernel == 4 && dstm_plane_fits(c, m);
-    const bool inv64 = !planes && form == SOLVE_INV64 && wave32 && wave64 && c->dst_kernel == 4;
+    const bool inv64 = !planes && form == SOLVE_INV64 && wave32 && c->dst_kernel == 4;
     const bool f32 = !planes && ((form == SOLVE_FP32 && wave32) || inv64);
-    // a pass whose lines are short enough: products with the sine matrix (k_dstm.hip)
-    // (its z pass counts the values of a component in 32 bits)
-    const bool z32 = (int64_t)((m[0] + 31) / 32 * 32) * m[1] * m[2] < ((int64_t)1 << 31);
+    // a pass whose lines are short enough: products with the sine matrix (k_dstm.hip; they count
+    // the values of a component in 32 bits, at most 1024^3 by the length limit above)
     auto mm = [&](int d, bool in32, bool forward = false) {
-        return c->dst_kernel == 4 && dstm_line_fits(m[d], in32, forward) && (d < 2 || z32);
+        return c->dst_kernel == 4 && dstm_line_fits(m[d], in32, forward);
     };
     if (inv64) reuse = 0;  // (the fine solves' reuse keeps FP32 arrays)
     // the kept transforms are worth their corrections (six launches) on large grids only
     if ((int64_t)wn[0] * wn[1] * wn[2] < SPECTRAL_MIN_NODES) reuse = 0;
     // one-wave kernels or products on every axis: rows of the work array padded to 128 bytes
-    auto padded = [&](int d) { return mm(d, false) || (c->dst_kernel == 4 && wave_class(ax[d], false)); };
+    auto padded = [&](int d) { return mm(d, false) || (c->dst_kernel == 4 && m[d] + 1 == FFT64_LENGTH); };
     const bool wave_all = f32 || planes || (padded(0) && padded(1) && padded(2));
     if (wave_all) {
         const int q = f32 ? 32 : 16;
@@ -2507,7 +2443,7 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
     a.nlines = (int64_t)a.px * m[1];
     FaceBufs fb{};
     const bool zmm = mm(2, f32) || (face_nd && !f32 && mm(2, false, true));
-    const bool zspec = face_nd && !inv64 && (f32 || zmm || (c->dst_kernel == 4 && wave_class(ax[2], false)));
+    const bool zspec = face_nd && !inv64 && (f32 || zmm);
     if (face_nd) {
         VPMX_TRY(face_bufs(c, m[0], m[1], m[2], ncomp, &fb));
         if (zspec) {

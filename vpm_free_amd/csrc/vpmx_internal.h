@@ -139,6 +139,10 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
                       GView out, int reuse = 0, int form = SOLVE_CTX, double *face_nd = nullptr,
                       const SolvePartial *part = nullptr, bool skip_faces = false);
 
+// The one length whose FP64 sine transform (m + 1 points) keeps an FFT in one wave, with a
+// compile-time plan; the other lengths up to DM_MAX points are products (k_dstm.hip).
+constexpr int FFT64_LENGTH = 288;
+
 // Complex FFT plan of length L (Stockham radices, device twiddle table exp(-2 pi i t / L)),
 // cached per context.
 struct FftShape {
