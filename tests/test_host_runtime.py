@@ -12,7 +12,7 @@ PRELUDE = """
 import ctypes, sys
 import numpy as np
 F = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
-for f in (F.fake_calls, F.fake_done, F.fake_held):
+for f in (F.fake_calls, F.fake_done, F.fake_held, F.fake_thread_copies):
     f.restype = ctypes.c_long
 F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
 MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH = range(6)
@@ -134,6 +134,24 @@ with V.VPM(V.Params.make(0.125)) as c:
     c.vpm(x, q, up, gp, SMALL, 3, 0, 0)
     c.vpm(x, q, up, gp, SMALL, 3, 2, 1)
 assert F.fake_held(1) == 0
+""")
+
+
+def test_results_that_share_memory(run):
+    """Two result arrays in one buffer: the later one's values stay, as with one copy after the other,
+    and no threads move them."""
+    run(TRANSFERS + """
+P = ctypes.POINTER(ctypes.c_double)
+for n in (SMALL, LARGE):
+    with V.VPM(V.Params.make(0.125)) as c:
+        x, q = cloud(n)
+        c.upload(x, q)
+        was = F.fake_thread_copies()
+        buf = np.full(5 * n, 7.0)  # positions from 0, strengths from n
+        xp, qp = buf.ctypes.data, buf.ctypes.data + 8 * n
+        r = c._lib.vpmx_particles_download(c._h, ctypes.cast(xp, P), ctypes.cast(qp, P), None, None)
+        assert r == 0 and F.fake_thread_copies() == was
+        assert np.array_equal(buf[n:], q.ravel()) and np.array_equal(buf[:n], x.ravel()[:n]), n
 """)
 
 

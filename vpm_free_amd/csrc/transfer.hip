@@ -191,6 +191,17 @@ bool missing(const Copy *q, int n) {
     return false;
 }
 
+// Result arrays that share memory: the runtime writes them one after another, so the last one's
+// values stay (the threads of a large transfer would mix them).
+bool shared_results(const Copy *q, int n) {
+    for (int i = 0; i < n; i++)
+        for (int j = 0; j < i; j++)
+            if (q[i].bytes && q[j].bytes && (char *)q[i].dst < (char *)q[j].dst + q[j].bytes &&
+                (char *)q[j].dst < (char *)q[i].dst + q[i].bytes)
+                return true;
+    return false;
+}
+
 // Memory that the device reaches by itself (pinned, managed, the device's own): the runtime
 // copies it.
 bool direct(const void *p) {
@@ -233,7 +244,7 @@ int copy_out(Ctx *c, const Copy *q, int n) {
     const size_t total = total_bytes(q, n);
     if (!total) return VPMX_OK;
     if (missing(q, n)) return fail(c, VPMX_ERR_HIP, "copy: invalid argument (a null array)");
-    if (any_direct(false, q, n)) return copy_direct(c, false, q, n);
+    if (any_direct(false, q, n) || shared_results(q, n)) return copy_direct(c, false, q, n);
     if (total > SMALL_COPY) return copy_large(c, false, q, n, total);
     char *b = nullptr;
     VPMX_TRY(small_buffer(c, total, &b));
