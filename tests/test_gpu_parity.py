@@ -136,7 +136,7 @@ def test_vpm_mode2_ring(vpmlib, oracle, h, sigma):
 @pytest.mark.parametrize("prec", [0, 1])
 def test_vpm_mode2_spectral_shortcuts(vpmlib, oracle, h, sigma, tree, prec):
     """vpm(2) with both spectral shortcuts of the fine solves forced on small blocks (they are
-    taken by default from 96^3 nodes): the zero-BC solve's normal derivatives from its spectrum
+    taken by default from 150^3 nodes): the zero-BC solve's normal derivatives from its spectrum
     (face_derivs = 1), and the second solve evaluated only on the inner box's faces and at the
     coarse samples (fine_partial = 1) -- the nodes yaps reads.  Every grid, UP and GP against the
     oracle at 1e-12 in FP64, at the mixed form's 1e-5 in the mixed form."""
@@ -211,7 +211,8 @@ def test_rk2_step_and_diagnostics(vpmlib, oracle):
 
 @pytest.mark.parametrize("nn", [(35, 23, 27), (38, 12, 20), (47, 45, 13)])
 def test_solve_all_radix_classes(ctx, oracle, nn):
-    """DST lengths 2(m+1) with prime factors 17, 11, 13, 37, 5, 23 and 3 (every radix class)."""
+    """Lengths m + 1 with prime factors 17, 11, 13, 37, 5, 23 and 3: matrix products over whole planes,
+    which do not depend on them."""
     rng = np.random.default_rng(sum(nn))
     nn = np.array(nn, np.int32)
     xb = np.array([0.3, -0.2, 0.1, 0, 0, 0])
@@ -225,6 +226,37 @@ def test_solve_all_radix_classes(ctx, oracle, nn):
     assert rel_l2(got, ref) <= TOL
 
 
+# lines that still take an FFT, by their largest radix: FP64 lines above the products' 367 points
+# (4: 384, 512; 7: 375, 392; 17: 374, 390; 37: 370, 391; above 37: 376, 410, 427), FP32 lines above 208
+# points without larger factors (4: 243, 256; 7: 245, 280; 17: 242, 255, 264, 286, and the compile-time
+# plans of 272 and 288)
+FFT64 = [384, 512, 375, 392, 374, 390, 370, 391, 376, 410, 427]
+FFT32 = [243, 256, 245, 280, 242, 255, 264, 286, 272, 288]
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("length,prec", [(n, 0) for n in FFT64] + [(n, 1) for n in FFT32])
+def test_solve_fft_lines(ctx, oracle, length, prec, axis):
+    """One long axis of m = length - 1 points, Dirichlet values on all faces: FP64 within 1e-12 of the
+    oracle, the mixed form (five FP32 passes) within 1e-6."""
+    rng = np.random.default_rng(length + axis)
+    nn = np.array([9, 12, 10], np.int32)
+    nn[axis] = length + 1
+    xb = np.array([0.3, -0.2, 0.1, 0, 0, 0])
+    dpm = np.array([0.05, 0.04, 0.06])
+    rhs = rng.standard_normal((nn[2], nn[1], nn[0], 3))
+    sol = rng.standard_normal((nn[2], nn[1], nn[0], 3))
+    win = np.array([1, 1, 1, nn[0], nn[1], nn[2]], np.int32)
+    say("case: solve FFT lines", nn.tolist(), "precision", prec)
+    ref = oracle.solve_window(xb, dpm, nn, win, rhs, sol=sol)
+    try:
+        ctx.set_precision(prec)
+        got = ctx.stage_solve(xb, dpm, nn, 3, win, rhs, sol=sol)
+    finally:
+        ctx.set_precision(0)
+    assert rel_l2(got, ref) <= (TOL if prec == 0 else 1e-6)
+
+
 def _lap7(u, h):
     """7-point Laplacian at the interior nodes of u (nz, ny, nx)."""
     c = u[1:-1, 1:-1, 1:-1]
@@ -235,12 +267,12 @@ def _lap7(u, h):
 
 @pytest.mark.parametrize("n", [289, 273, 161, 145])
 def test_solve_full_size_plans(ctx, n):
-    """The block sizes of the 256-cubed and 128-cubed workloads, where the sine transforms run
-    their compile-time FFT plans (FP64: 288 = 4.4.2.9 or 8.4.9, 272 = 4.4.17 with the radix-17
-    stage on one lane or split, 160 = 8.4.5, 144 = 4.4.9; FP32: 576 = 4.4.4.9 or 8.8.9, 544 =
-    17.4.4.2 or 17.8.4), padded LDS sequences and register-capped kernels, as the tuner picks
-    them -- sizes the oracle is too slow for.  The FP64 solution satisfies the 7-point equations
-    to rounding, and the mixed form agrees with it to FP32 accuracy."""
+    """The block sizes of the 256-cubed and 128-cubed workloads -- sizes the oracle is too slow for:
+    289 with the compile-time FFT plans of both forms (FP64 288 = 4.4.2.9 or 8.4.9, FP32 576 =
+    4.4.4.9, 8.8.9 or 16.4.9; padded LDS sequences, register-capped kernels, as the tuner picks
+    them), 273 with FP64 products and the FP32 plans of 544 = 17.4.4.2 or 17.8.4, 161 and 145 with
+    products in both forms.  The FP64 solution satisfies the 7-point equations to rounding, and the
+    mixed form agrees with it to FP32 accuracy."""
     rng = np.random.default_rng(n)
     nn = np.array([n, n, n], np.int32)
     h = np.array([1 / 64] * 3)
@@ -305,6 +337,30 @@ def test_boundary_sum_tree(vpmlib, oracle, nn, levmax):
     say("  rel L2 vs oracle tree %.2e (tree vs direct %.2e)" % (err, rel_l2(ref, direct)))
     assert rel_l2(ref, direct) > 1e3 * TOL  # the tree's sums are not the direct ones
     assert err <= TOL
+
+
+@pytest.mark.parametrize("nn,levmax,h", [((65, 57, 49), 3, 1 / 32), ((49, 65, 57), 2, 1 / 32), ((65, 57, 49), 3, 0.1),
+                                         ((57, 49, 65), 2, 0.3), ((33, 33, 33), 4, 1 / 32), ((17, 25, 33), 3, 1 / 32)])
+def test_boundary_sum_tree_ties(vpmlib, oracle, nn, levmax, h):
+    """Equal spacings: many targets lie at r = 10 sqrt(DS) of a group, exactly where the spacing is a
+    power of two and to rounding where it is not, and r < 10 sqrt(DS) decides which terms are taken (the
+    other choice changes the sums by 5e-7 to 2e-6).  24 trees in the smallest two: parts of one and of two."""
+    V = vpmlib
+    nn = np.array(nn, np.int32)
+    dpm = np.full(3, h)
+    xb = np.array([*(-h * np.array([24.0, 17.0, 20.0])), 0, 0, 0])
+    c0 = xb[:3] + (nn - 1) * h / 2
+    rhs = _blob_rhs(nn, xb, dpm, centre=tuple(c0 + h), s=8 * h)
+    sol = np.zeros_like(rhs)
+    say("case: tree boundary sums on ties", nn.tolist(), "levmax", levmax, "h", h)
+    try:
+        oracle.set_tree(levmax)
+        ref = oracle.pmesh_inf(xb, dpm, nn, rhs, sol)
+    finally:
+        oracle.set_tree(-1)
+    with V.VPM(V.Params.make(0.125)) as c:
+        got = c.stage_pmesh_inf(xb, dpm, nn, rhs, sol, itree=1, levmax=levmax)
+    assert rel_l2(got, ref) <= TOL
 
 
 @pytest.mark.parametrize("h,sigma", [(0.125, 0.2), (1 / 16, 0.1)])
@@ -540,6 +596,30 @@ def test_pmesh_inf_reuse_full_size(vpmlib, prec, tol):
     assert rel_l2(out["1"], out["0"]) <= tol
 
 
+@pytest.mark.parametrize("nn", [(251, 91, 161), (163, 251, 91), (95, 161, 243)])
+@pytest.mark.parametrize("prec,tol", [(0, TOL), (1, 2e-6)])
+def test_pmesh_inf_reuse_unequal(vpmlib, nn, prec, tol):
+    """The same on boxes above the size from which the transforms are kept, with three extents and
+    three spacings, short and long spans of rows in the correction, and, in the mixed form, FP32 lines
+    of products beside FFT lines on each axis."""
+    V = vpmlib
+    nn = np.array(nn, np.int32)
+    dpm = np.array([1 / 64, 1 / 51, 1 / 43])
+    xb = np.array([-1.1, -0.9, -1.3, 0, 0, 0])
+    c0 = xb[:3] + (nn - 1) * dpm / 2
+    rhs = _blob_rhs(nn, xb, dpm, centre=tuple(c0 + 0.02), s=0.25 * float(np.min((nn - 1) * dpm)))
+    sol = np.zeros_like(rhs)
+    say("case: pmesh_inf forward-pass reuse", nn.tolist(), "precision", prec)
+    out = {}
+    for reuse in (1, 0):
+        with V.VPM(V.Params.make(0.125)) as c:
+            c.set_option("dst_reuse", reuse)
+            c.set_precision(prec)
+            out[reuse] = c.stage_pmesh_inf(xb, dpm, nn, rhs, sol)
+    assert rel_l2(out[1], out[0]) <= tol
+    assert not np.array_equal(out[1], out[0])  # the correction ran
+
+
 @pytest.mark.parametrize("nn,levmax,ibctyp", [((33, 29, 31), -1, 2), ((65, 57, 49), -1, 2), ((43, 43, 43), 2, 2),
                                                ((33, 29, 31), -1, 3)])
 @pytest.mark.parametrize("prec", [0, 1])
@@ -649,10 +729,11 @@ def test_vpm_mode2_call_sequence_kept_zeros(vpmlib, oracle):
 
 def test_tuner_choices_keep_results(vpmlib):
     """The autotuner picks kernel variants and persistent grid sizes by timing them; at h=1/16
-    (runtime FFT plans, so the variants differ in register caps, batch order and grid size
-    only) the results are those of the fixed defaults bit for bit: every work item's sums do
-    not depend on which work-group takes it.  (The plan variants of the 288-, 544- and
-    576-point lengths round differently; the full-size parity tests cover them.)"""
+    (products of 16 or 32 lines, stencil and matrix tiles) the results are those of the fixed
+    defaults bit for bit: every work item's sums do not depend on which work-group takes it.  FFT
+    lines and tuned interpolation grids: test_kept_zeros_and_tuning (test_gpu_tiles.py).  (The
+    plan variants of the 288-, 544- and 576-point lengths round differently; the full-size parity
+    tests cover them.)"""
     V = vpmlib
     h = 1 / 16
     xp, qp = cases.single_ring(h=h, sigma=0.1)
@@ -678,12 +759,10 @@ def test_tuner_choices_keep_results(vpmlib):
 
 def test_tuner_variants_same_bits(vpmlib):
     """Every launch forced to its variant v (option tune_variant) gives the same velocity and
-    stretching grids, UP and GP bit for bit, for every v and both forms, at h=1/16 (runtime FFT
-    plans, so the variants differ in scheduling only), with the fine solves' spectral shortcuts
-    on: the curl/stretch tile shapes, with the velocity ring alone or with the stream function
-    kept in registers and one LDS plane, the FP64
-    matrix-product tile shapes, the face sums' rows in flight, the sine-transform batch
-    orders."""
+    stretching grids, UP and GP bit for bit, for every v and both forms, at h=1/16, with the fine
+    solves' spectral shortcuts on: the curl/stretch tile shapes, with the velocity ring alone or
+    with the stream function kept in registers and one LDS plane, the FP64 matrix-product tile
+    shapes, the face sums' rows in flight, the lines per work-group of the sine products."""
     V = vpmlib
     h = 1 / 16
     xp, qp = cases.single_ring(h=h, sigma=0.1)
@@ -707,3 +786,26 @@ def test_tuner_variants_same_bits(vpmlib):
                     assert np.array_equal(a, b), (v, prec, name, float(np.max(np.abs(a - b))))
             rep = c.tuning_report()
         assert "forced" in rep
+
+
+@pytest.mark.parametrize("nn,prec", [((244, 20, 21), 1), ((20, 244, 21), 1), ((21, 20, 244), 1), ((244, 226, 246), 1),
+                                     ((130, 131, 141), 0), ((210, 130, 300), 0)])
+def test_solve_variants_same_bits(vpmlib, nn, prec):
+    """Solves with every launch forced to its variant v give the same bits: both batch orders of the
+    FP32 FFT passes along each axis (runtime plans), 16 and 32 lines per work-group of the products."""
+    V = vpmlib
+    rng = np.random.default_rng(sum(nn))
+    nn = np.array(nn, np.int32)
+    rhs, sol = rng.standard_normal((2, nn[2], nn[1], nn[0], 3))
+    win = np.array([1, 1, 1, *nn], np.int32)
+    ref = None
+    for v in (0, 1):
+        with V.VPM(V.Params.make(0.125)) as c:
+            c.set_option("tune_variant", v)
+            c.set_precision(prec)
+            say("case: solve variants", nn.tolist(), "precision", prec, "variant", v)
+            got = c.stage_solve(np.zeros(6), np.array([0.05, 0.04, 0.06]), nn, 3, win, rhs, sol=sol)
+            rep = c.tuning_report()
+        assert "forced" in rep and ("matrix products" in rep if prec == 0 else "pass FP32 L=" in rep)
+        assert ref is None or np.array_equal(got, ref)
+        ref = got

@@ -1842,7 +1842,7 @@ static int fold_correct(Ctx *c, const DstArgs &a, int ncomp, bool f32, const GVi
     VPMX_TRY(dgemm_batched(c, true, mx, my, mx, Sx, mx, 0, T, my, fz, Z, mx, fz, np));
     // one thread per kx: rows of up to 320 (the one-wave kernels' limit is below that)
     if (a.px > 320) return fail(c, VPMX_ERR_UNSUP, "Poisson: forward-pass reuse needs rows of at most 320 points");
-    // small grids (the coarse problem): short spans, so the grid still fills the device
+    // few rows a plane: short spans, so the launch still fills the device
     const int span = my <= 96 ? 8 : FC_SPAN;
     const dim3 g((unsigned)((my + span - 1) / span), (unsigned)(mz * ncomp));
     const dim3 blk((unsigned)((a.px + 63) / 64 * 64));

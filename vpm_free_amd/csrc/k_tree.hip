@@ -510,6 +510,7 @@ int boundary_sums_tree(Ctx *c, const Grid &g, int64_t nb, const double *sig, con
     const int ntile = p->tiles.off[6];
     const int64_t nt = (int64_t)ntile * 64 * TR_T;
     int st = VPMX_OK;
+    // (384 bytes a target, 200 MB for the faces of a 289^3 block; a plan has 24 trees or more)
     double *part = (double *)ensure(c, c->tree_part, sizeof(double) * 3 * TR_PARTS * (size_t)nt, &st);
     if (st) return st;
     const unsigned blocks = (unsigned)((ntile + TR_WAVES - 1) / TR_WAVES);
