@@ -7,7 +7,7 @@
 #include <sys/syscall.h>
 #include <unistd.h>
 
-enum { MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH, NKIND };
+enum { MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH, RECORD, NKIND };
 static long calls[NKIND], done[NKIND], fail_at[NKIND], held_host, held_dev;
 static __thread int last_error;
 
@@ -78,7 +78,7 @@ int hipGraphExecDestroy(void *g) { return 0; }
 int hipEventCreate(void **e) { return enter(EVENT) ? 2 : get(e, 8, &held_dev); }
 int hipEventCreateWithFlags(void **e, unsigned f) { return enter(EVENT) ? 2 : get(e, 8, &held_dev); }
 int hipEventDestroy(void *e) { return put(e, &held_dev); }
-int hipEventRecord(void *e, void *s) { return 0; }
+int hipEventRecord(void *e, void *s) { return enter(RECORD) ? 2 : 0; }
 int hipEventSynchronize(void *e) { return 0; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { *ms = 1.0f; return 0; }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *f, int t, size_t l) { *n = 1; return 0; }

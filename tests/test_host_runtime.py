@@ -15,7 +15,7 @@ F = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
 for f in (F.fake_calls, F.fake_done, F.fake_held, F.fake_thread_copies):
     f.restype = ctypes.c_long
 F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
-MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH = range(6)
+MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH, RECORD = range(7)
 sys.path.insert(0, %r)
 from vpm_free_amd import vpm as V
 rng = np.random.default_rng(1)
@@ -204,4 +204,21 @@ with V.VPM(V.Params.make(h)) as c:
                 c.vpm(x, q, up, gp, 2, 3, 2, 1)
             except V.VpmError as e:
                 assert "prime factor" in str(e) or "too long" in str(e), (axis, cells, str(e))
+""")
+
+
+def test_stage_interval_after_the_first_fill(run):
+    """The stretching stage of a first mode-4 call begins after the fill of its new velocity grid: an
+    event of its own, where later calls (no fill) share the projection's last one."""
+    run("""
+x, q = np.array([[0.0, 0, 0], [1, 2, 3]]), np.ones((2, 4))
+up, gp = np.zeros_like(x), np.zeros_like(x)
+with V.VPM(V.Params.make(0.125)) as c:
+    c.vpm(x, q, up, gp, 2, 3, 0, 0)
+    n = []
+    for call in range(3):
+        was = F.fake_done(RECORD)
+        c.vpm(x, q, up, gp, 2, 3, 4, 1)
+        n.append(F.fake_done(RECORD) - was)
+assert n[0] == n[1] + 1 and n[1] == n[2], n
 """)

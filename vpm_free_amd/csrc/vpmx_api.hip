@@ -552,7 +552,7 @@ static int run_vpm(Ctx *c, int whattodo, const double *xp, const double *qp, dou
         double *str = (double *)ensure(c, c->str, sizeof(double) * 3 * (size_t)GG, &st); if (st) return st;
         if (fresh || whattodo == 5) VPMX_TRY(fill(c, vel, 3 * GG, 0.0));  // velvr*_pm = 0
         GView rg = global_rhs(c);
-        mark(c, ST_FD, 0, whattodo == 4);
+        mark(c, ST_FD, 0, whattodo == 4 && !fresh);
         if (whattodo == 4) VPMX_TRY(stretch_kernel(c, gn, G.dpm, rg, view(vel, gn), view(str, gn)));
         else VPMX_TRY(diffuse_kernel(c, gn, G.dpm, ni, rg, view(str, gn)));
         mark(c, ST_FD, 1);
