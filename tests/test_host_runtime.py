@@ -185,6 +185,24 @@ for prec in (0, 1):
 """)
 
 
+def test_solve_uploads_the_tables_it_reads(run):
+    """A first solve uploads, per axis, the eigenvalues and the sine matrix of the products, or the
+    twiddles and sines of an FFT line; nothing for a second one."""
+    run("""
+def uploads(c, nn):
+    nn = np.array(nn, np.int32)
+    a = np.zeros((nn[2], nn[1], nn[0], 3))
+    was = F.fake_done(MEMCPY)
+    c.stage_solve(np.zeros(6), np.full(3, 0.1), nn, 3, np.array([1, 1, 1, *nn], np.int32), a, None, True)
+    return F.fake_done(MEMCPY) - was
+with V.VPM(V.Params.make(0.125)) as c:
+    assert uploads(c, (13, 15, 17)) == 6
+    assert uploads(c, (13, 15, 17)) == 0
+    assert uploads(c, (13, 401, 17)) == 3  # 399 points: eigenvalues, twiddles, sines
+    assert uploads(c, (13, 401, 17)) == 0
+""")
+
+
 def test_every_block_length_in_the_mixed_form(run):
     """Evaluations in the mixed form (its inner-box solves return in FP64) of boxes with one axis of up
     to 330 nodes."""

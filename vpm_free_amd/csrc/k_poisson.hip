@@ -1232,6 +1232,7 @@ struct FftPlan {
     double2 *tw = nullptr;
 };
 
+// The stages of length L (refused when a factor is too large); plan_table() before a pass reads tw.
 static int get_plan(Ctx *c, int L, FftPlan **out) {
     auto it = c->fft_plans.find(L);
     if (it != c->fft_plans.end()) { *out = (FftPlan *)it->second; return VPMX_OK; }
@@ -1253,21 +1254,33 @@ static int get_plan(Ctx *c, int L, FftPlan **out) {
             return fail(c, VPMX_ERR_UNSUP, "DST length 2(m+1)=" + std::to_string(L) + " has a prime factor " +
                                                std::to_string(R) + " > 64");
         }
+    c->fft_plans[L] = p;
+    *out = p;
+    return VPMX_OK;
+}
+// The twiddle table, uploaded when the first FFT pass of that length needs it (most lengths take
+// matrix products and never do).
+static int plan_table(Ctx *c, FftPlan *p) {
+    if (p->tw) return VPMX_OK;
+    const int L = p->L;
     std::vector<double2> h(L);
     for (int t = 0; t < L; t++) {
         long double ang = 2.0L * 3.141592653589793238462643383279502884L * (long double)t / (long double)L;
         h[t] = make_double2((double)cosl(ang), (double)(-sinl(ang)));
     }
-    VPMX_HIP(c, hipMalloc(&p->tw, sizeof(double2) * L));
-    VPMX_HIP(c, hipMemcpy(p->tw, h.data(), sizeof(double2) * L, hipMemcpyHostToDevice));
-    c->fft_plans[L] = p;
-    *out = p;
+    double2 *d = nullptr;
+    VPMX_HIP(c, hipMalloc(&d, sizeof(double2) * L));
+    const hipError_t e = hipMemcpy(d, h.data(), sizeof(double2) * L, hipMemcpyHostToDevice);
+    if (e != hipSuccess) (void)hipFree(d);
+    VPMX_HIP(c, e);
+    p->tw = d;
     return VPMX_OK;
 }
 
 int fft_shape(Ctx *c, int L, FftShape *out) {
     FftPlan *p = nullptr;
     VPMX_TRY(get_plan(c, L, &p));
+    VPMX_TRY(plan_table(c, p));
     out->L = p->L;
     out->nstages = p->nstages;
     for (int s = 0; s < p->nstages; s++) out->radix[s] = p->radix[s];
@@ -1440,7 +1453,6 @@ static int launch_pass3(Ctx *c, DstArgs a, int ncomp, int rc) {
 struct AxisPlan {
     int m;
     FftPlan *full, *half;
-    const double *sn;
 };
 
 template <int MODE, class T>
@@ -1636,9 +1648,11 @@ static int launch_wave(Ctx *c, DstArgs a, int ncomp, int rc, const FftPlan *fp) 
 
 // The mixed z pass (k_dst_zmix) on the FP32 work array a.w, FP64 results into wo.
 static int launch_zmix(Ctx *c, DstArgs a, int ncomp, const AxisPlan &X, double *wo) {
-    const FftPlan *f32 = X.full, *f64 = X.half;
-    setup_axis(a, (FftPlan *)f32, X.m);
-    a.sn = X.sn;
+    FftPlan *f32 = X.full, *f64 = X.half;
+    VPMX_TRY(plan_table(c, f32));
+    VPMX_TRY(plan_table(c, f64));
+    setup_axis(a, f32, X.m);
+    VPMX_TRY(sine_table(c, f64->L, &a.sn));
     a.wo = wo;
     a.npairs = 8;
     a.ncomp = ncomp;
@@ -1711,22 +1725,25 @@ static int wave_class(const AxisPlan &P) {
 
 template <int MODE>
 static int run_pass(Ctx *c, DstArgs a, int ncomp, const AxisPlan &P, bool f32) {
-    if (f32) {
+    auto full = [&]() -> int {
+        VPMX_TRY(plan_table(c, P.full));
         setup_axis(a, P.full, P.m);
+        return VPMX_OK;
+    };
+    if (f32) {
+        VPMX_TRY(full());
         return launch_wave<MODE, float>(c, a, ncomp, wave_class(P), P.full);
     }
-    if (c->dst_kernel == 4 && P.half->L == FFT64_LENGTH) {
-        setup_axis(a, P.half, P.m);
-        a.sn = P.sn;
-        return launch_wave<MODE, double>(c, a, ncomp, 0, P.half);
+    setup_axis(a, P.half, P.m);
+    const int rc = radix_class(a);
+    if (c->dst_kernel >= 3 && rc) {
+        VPMX_TRY(plan_table(c, P.half));
+        a.tw = P.half->tw;
+        VPMX_TRY(sine_table(c, P.half->L, &a.sn));
+        if (c->dst_kernel == 4 && P.half->L == FFT64_LENGTH) return launch_wave<MODE, double>(c, a, ncomp, 0, P.half);
+        return launch_pass3<MODE>(c, a, ncomp, rc);
     }
-    if (c->dst_kernel >= 3) {
-        setup_axis(a, P.half, P.m);
-        a.sn = P.sn;
-        const int rc = radix_class(a);
-        if (rc) return launch_pass3<MODE>(c, a, ncomp, rc);
-    }
-    setup_axis(a, P.full, P.m);
+    VPMX_TRY(full());
     return launch_pass<MODE>(c, a, ncomp);
 }
 
@@ -2364,7 +2381,6 @@ int poisson_dirichlet(Ctx *c, int ncomp, const int wn[3], const double h[3], GVi
         ax[d].m = m[d];
         VPMX_TRY(get_plan(c, 2 * (m[d] + 1), &ax[d].full));
         VPMX_TRY(get_plan(c, m[d] + 1, &ax[d].half));
-        VPMX_TRY(sine_table(c, m[d] + 1, &ax[d].sn));
     }
     DstArgs a{};
     a.mx = m[0]; a.my = m[1]; a.mz = m[2];
