@@ -7,8 +7,11 @@
 //     asynchronous copy per array;
 //   * larger ones are cut into chunks that several threads move through pinned slots, each with a
 //     copy in flight while it touches the other slot's host side (the page faults of a fresh
-//     result array spread over the threads too).  The slots and the threads' streams are one set
-//     per device, used by one transfer at a time;
+//     result array spread over the threads too).  The slots and the streams are one set per device,
+//     used by one transfer at a time.  Two streams carry what eight do (16 MB in: 330 us on 2, 4 or
+//     8, 380 on one), and each stream's first copies cost 5 ms: a process' first 84 MB in and 156 MB
+//     out take 22 and 4 ms, with eight streams 26 and 4 and five transfers of 7 instead of 2 ms after
+//     them, by the runtime 16 and 16;
 //   * where no pinned memory is to be had, the runtime copies.
 // Particles in (MB: us) by the runtime / the pinned buffer / chunks: 0.11: 57 / 25 / 43; 1.9: 85 /
 // 72 / 108; 3.8: 146 / 120 / 168; 7.7: 254 / 233 / 303; 214: 7814 / 9742 / 4290.  Out: 0.2: 128 / 50 / 98;
@@ -34,7 +37,7 @@ namespace vpmx {
 namespace {
 
 constexpr size_t SMALL_COPY = 4 << 20, CHUNK = 2 << 20, PER_THREAD = 4 << 20;
-constexpr int MAX_THREADS = 8;
+constexpr int MAX_THREADS = 8, STREAMS = 2;
 
 // The pinned slots (two per thread) and streams of one device.
 struct Slots {
@@ -42,7 +45,7 @@ struct Slots {
     int device = 0;
     int ready = 0;  // threads whose slots are set up
     char *mem[MAX_THREADS] = {};
-    hipStream_t stream[MAX_THREADS] = {};
+    hipStream_t stream[STREAMS] = {};  // thread t's: t mod STREAMS
     hipEvent_t done[MAX_THREADS][2] = {};
     // at least n threads' slots; the number there are (fewer when memory is short; what a thread
     // got before the call that failed stays for the next attempt)
@@ -61,9 +64,9 @@ private:
             if (hipHostMalloc(&p, 2 * CHUNK, hipHostMallocDefault) != hipSuccess) return false;
             mem[t] = (char *)p;
         }
-        if (!stream[t]) {
+        if (!stream[t % STREAMS]) {
             if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return false;
-            stream[t] = s;
+            stream[t % STREAMS] = s;
         }
         for (hipEvent_t &d : done[t])
             if (!d) {
@@ -74,10 +77,10 @@ private:
     }
 };
 
-// The device's slots, shared by its contexts and kept until the process ends (32 MB pinned and eight
-// streams a device at most): to set them up and run their first copies takes 8 ms, 40 ms in a new
-// process, and to take them down 3 ms, as much as they save on a transfer of 200 MB, which a program
-// that opens a context per evaluation would pay each time.
+// The device's slots, shared by its contexts and kept until the process ends (at most 32 MB pinned and
+// the two streams): a set's memory, streams and first copies take 8 ms, and 3 ms go into taking it
+// down, as much as it saves on a transfer of 200 MB, which a program that opens a context per
+// evaluation would pay each time.
 Slots &slots_of(int device) {
     static std::mutex m;
     static auto *all = new std::map<int, std::unique_ptr<Slots>>;  // (outlives the runtime's own shutdown)
@@ -92,6 +95,7 @@ Slots &slots_of(int device) {
 
 // Moves chunks (taken off `next`) through thread t's two slots.
 hipError_t move_chunks(Slots &S, int t, bool in, const std::vector<Copy> &ch, std::atomic<size_t> &next) {
+    const hipStream_t stream = S.stream[t % STREAMS];
     hipError_t e = hipSetDevice(S.device);
     const Copy *held[2] = {nullptr, nullptr};  // a slot's copy in flight
     // the slot's copy done: out, its bytes go to the caller
@@ -108,13 +112,13 @@ hipError_t move_chunks(Slots &S, int t, bool in, const std::vector<Copy> &ch, st
         char *slot = S.mem[t] + k * CHUNK;
         if (in) std::memcpy(slot, ch[i].src, ch[i].bytes);
         e = hipMemcpyAsync(in ? ch[i].dst : slot, in ? slot : ch[i].src, ch[i].bytes,
-                           in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, S.stream[t]);
-        if (e == hipSuccess) e = hipEventRecord(S.done[t][k], S.stream[t]);
+                           in ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, stream);
+        if (e == hipSuccess) e = hipEventRecord(S.done[t][k], stream);
         held[k] = &ch[i];
     }
     settle(k);
     settle(k ^ 1);
-    const hipError_t last = hipStreamSynchronize(S.stream[t]);
+    const hipError_t last = hipStreamSynchronize(stream);
     return e != hipSuccess ? e : last;
 }
 
