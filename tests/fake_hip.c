@@ -4,10 +4,8 @@
 #include <stddef.h>
 #include <stdlib.h>
 #include <string.h>
-#include <sys/syscall.h>
-#include <unistd.h>
 
-enum { MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH, RECORD, NKIND };
+enum { MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH, RECORD, ASYNC, NKIND };
 static long calls[NKIND], done[NKIND], fail_at[NKIND], held_host, held_dev;
 static __thread int last_error;
 
@@ -50,11 +48,9 @@ int hipMemcpy(void *d, const void *s, size_t n, int k) {
     memcpy(d, s, n);
     return 0;
 }
-static long on_threads;
-long fake_thread_copies(void) { return __sync_fetch_and_add(&on_threads, 0); } /* issued off the main thread */
 int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st) {
     if (!d || !s) return last_error = 1;
-    if (syscall(SYS_gettid) != getpid()) __sync_add_and_fetch(&on_threads, 1);
+    if (enter(ASYNC)) return 2;
     memcpy(d, s, n);
     return 0;
 }

@@ -1,5 +1,6 @@
 """Copies between the caller's arrays and the device: one pass through the pinned buffer up to
-4 MiB, chunks of 2 MiB on one to several threads above it.  56 bytes a particle go in."""
+4 MiB; above it chunks of 2 MiB on one to several threads, into the device from 16 MiB and the
+runtime's copies up to there.  56 bytes a particle go in, 104 come out."""
 import ctypes as C
 import threading
 
@@ -8,9 +9,9 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# one particle; the last size of the small path and the first of the chunked one; chunk ends inside
-# and between the arrays; every thread busy
-SIZES = [1, 74898, 74899, 87381, 87382, 1200001]
+# one particle; the last sizes of the small path and the first past it, out and in; chunk ends inside
+# and between the arrays; the first size in chunks both ways; every thread busy
+SIZES = [1, 40329, 40330, 74898, 74899, 87381, 87382, 299593, 299594, 1200001]
 
 
 def pinned(a):

@@ -12,10 +12,10 @@ PRELUDE = """
 import ctypes, sys
 import numpy as np
 F = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
-for f in (F.fake_calls, F.fake_done, F.fake_held, F.fake_thread_copies):
+for f in (F.fake_calls, F.fake_done, F.fake_held):
     f.restype = ctypes.c_long
 F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
-MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH, RECORD = range(7)
+MALLOC, MEMCPY, HOSTMALLOC, STREAM, EVENT, LAUNCH, RECORD, ASYNC = range(8)
 sys.path.insert(0, %r)
 from vpm_free_amd import vpm as V
 rng = np.random.default_rng(1)
@@ -138,20 +138,35 @@ assert F.fake_held(1) == 0
 """)
 
 
+def test_large_transfers_go_in_chunks(run):
+    """Into the device 16 MiB and more, out of it more than 4 MiB; the others are a copy per array."""
+    run(TRANSFERS + """
+def copies(f, *a):
+    was = F.fake_done(ASYNC)
+    f(*a)
+    return F.fake_done(ASYNC) - was
+with V.VPM(V.Params.make(0.125)) as c:
+    # 56 bytes a particle go in (24 and 32 in two arrays), 104 come out (24, 32, 24 and 24 in four)
+    chunks = lambda n, arrays: sum(-(-n * b // (2 << 20)) for b in arrays)
+    for n, large_in, large_out in ((40329, 0, 0), (40330, 0, 1), (70000, 0, 1), (200000, 0, 1), (299593, 0, 1), (299594, 1, 1)):
+        assert copies(c.upload, *cloud(n)) == (chunks(n, (24, 32)) if large_in else 2), n
+        assert copies(c.download) == (chunks(n, (24, 32, 24, 24)) if large_out else 4), n
+""")
+
+
 def test_results_that_share_memory(run):
-    """Two result arrays in one buffer: the later one's values stay, as with one copy after the other,
-    and no threads move them."""
+    """Two result arrays in one buffer: the later one's values stay, with one copy after the other."""
     run(TRANSFERS + """
 P = ctypes.POINTER(ctypes.c_double)
 for n in (SMALL, LARGE):
     with V.VPM(V.Params.make(0.125)) as c:
         x, q = cloud(n)
         c.upload(x, q)
-        was = F.fake_thread_copies()
+        was = F.fake_done(ASYNC)
         buf = np.full(5 * n, 7.0)  # positions from 0, strengths from n
         xp, qp = buf.ctypes.data, buf.ctypes.data + 8 * n
         r = c._lib.vpmx_particles_download(c._h, ctypes.cast(xp, P), ctypes.cast(qp, P), None, None)
-        assert r == 0 and F.fake_thread_copies() == was
+        assert r == 0 and F.fake_done(ASYNC) == was + 2
         assert np.array_equal(buf[n:], q.ravel()) and np.array_equal(buf[:n], x.ravel()[:n]), n
 """)
 

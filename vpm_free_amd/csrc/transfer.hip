@@ -5,7 +5,11 @@
 // call each waits for the host.  Here
 //   * up to SMALL_COPY bytes pass through the context's pinned buffer: one memcpy and one
 //     asynchronous copy per array;
-//   * larger ones are cut into chunks that several threads move through pinned slots, each with a
+//   * into the device, from there to CHUNKED_IN bytes the runtime's copies are the fastest (MB: us,
+//     arrays used before / fresh ones; runtime, chunks): 4.5: 154 / 187, 179 / 214; 6: 195 / 241, 270 /
+//     326; 8: 251 / 304, 304 / 367; 12: 344 / 424, 386 / 415; 16: 450 / 568, 454 / 491; 24: 669 / 877,
+//     613 / 636; 48: 1634 / 1663, 1114 / 1182;
+//   * larger ones, and what comes out of the device, are cut into chunks that several threads move through pinned slots, each with a
 //     copy in flight while it touches the other slot's host side (the page faults of a fresh
 //     result array spread over the threads too).  The slots and the streams are one set per device,
 //     used by one transfer at a time.  Two streams carry what eight do (16 MB in: 330 us on 2, 4 or
@@ -36,7 +40,7 @@ namespace vpmx {
 
 namespace {
 
-constexpr size_t SMALL_COPY = 4 << 20, CHUNK = 2 << 20, PER_THREAD = 4 << 20;
+constexpr size_t SMALL_COPY = 4 << 20, CHUNKED_IN = 16 << 20, CHUNK = 2 << 20, PER_THREAD = 4 << 20;
 constexpr int MAX_THREADS = 8, STREAMS = 2;
 
 // The pinned slots (two per thread) and streams of one device.
@@ -78,9 +82,9 @@ private:
 };
 
 // The device's slots, shared by its contexts and kept until the process ends (at most 32 MB pinned and
-// the two streams): a set's memory, streams and first copies take 8 ms, and 3 ms go into taking it
-// down, as much as it saves on a transfer of 200 MB, which a program that opens a context per
-// evaluation would pay each time.
+// the two streams): memory, streams and first copies took 8 ms and taking them down 3 ms when a set had
+// eight streams, more than a transfer of 200 MB saves, and a program that opens a context per
+// evaluation paid it each time.
 Slots &slots_of(int device) {
     static std::mutex m;
     static auto *all = new std::map<int, std::unique_ptr<Slots>>;  // (outlives the runtime's own shutdown)
@@ -229,7 +233,7 @@ int copy_in(Ctx *c, const Copy *q, int n) {
     const size_t total = total_bytes(q, n);
     if (!total) return VPMX_OK;
     if (missing(q, n)) return fail(c, VPMX_ERR_HIP, "copy: invalid argument (a null array)");
-    if (any_direct(true, q, n)) return copy_direct(c, true, q, n);
+    if ((total > SMALL_COPY && total < CHUNKED_IN) || any_direct(true, q, n)) return copy_direct(c, true, q, n);
     if (total > SMALL_COPY) return copy_large(c, true, q, n, total);
     char *b = nullptr;
     VPMX_TRY(small_buffer(c, total, &b));
