@@ -86,15 +86,15 @@ LARGE, SMALL = 700000, 500  # 39 MB in chunks, 28 kB through the pinned buffer
 
 
 def test_transfer_slots_serve_every_context(run):
-    """Contexts one after another: the pinned slots and the two streams of large transfers are set up
-    once."""
+    """Contexts one after another: the pinned slots and the streams, four at most, of large transfers
+    are set up once."""
     run(TRANSFERS + """
 for turn in range(4):
     with V.VPM(V.Params.make(0.125)) as c:
         base = F.fake_done(STREAM), F.fake_done(HOSTMALLOC)
         round_trip(c, LARGE)
         new = F.fake_done(STREAM) - base[0], F.fake_done(HOSTMALLOC) - base[1]
-        assert (new[0] == 2 and 0 < new[1] <= 8) if turn == 0 else new == (0, 0), (turn, new)
+        assert (0 < new[0] <= 4 and 0 < new[1] <= 8) if turn == 0 else new == (0, 0), (turn, new)
 assert F.fake_held(1) <= 8
 """)
 

@@ -12,10 +12,11 @@
 //   * larger ones, and what comes out of the device, are cut into chunks that several threads move through pinned slots, each with a
 //     copy in flight while it touches the other slot's host side (the page faults of a fresh
 //     result array spread over the threads too).  The slots and the streams are one set per device,
-//     used by one transfer at a time.  Two streams carry what eight do (16 MB in: 330 us on 2, 4 or
-//     8, 380 on one), and each stream's first copies cost 5 ms: a process' first 84 MB in and 156 MB
-//     out take 22 and 4 ms, with eight streams 26 and 4 and five transfers of 7 instead of 2 ms after
-//     them, by the runtime 16 and 16;
+//     used by one transfer at a time.  A stream's first copies cost about 5 ms each (a process' first
+//     84 MB in take 25 ms, 16 by the runtime, whose first 156 MB out take 16 against 4 here; the next
+//     one or two in 7 instead of 2, with eight streams the next five), and two streams are slower
+//     (18 MB out: 570 us, 480 with one per thread): four, which serve eight threads as well (84 MB in
+//     1.9 ms, 397 MB out 9.7 ms, as with eight);
 //   * where no pinned memory is to be had, the runtime copies.
 // Particles in (MB: us) by the runtime / the pinned buffer / chunks: 0.11: 57 / 25 / 43; 1.9: 85 /
 // 72 / 108; 3.8: 146 / 120 / 168; 7.7: 254 / 233 / 303; 214: 7814 / 9742 / 4290.  Out: 0.2: 128 / 50 / 98;
@@ -41,7 +42,7 @@ namespace vpmx {
 namespace {
 
 constexpr size_t SMALL_COPY = 4 << 20, CHUNKED_IN = 16 << 20, CHUNK = 2 << 20, PER_THREAD = 4 << 20;
-constexpr int MAX_THREADS = 8, STREAMS = 2;
+constexpr int MAX_THREADS = 8, STREAMS = 4;
 
 // The pinned slots (two per thread) and streams of one device.
 struct Slots {
@@ -82,7 +83,7 @@ private:
 };
 
 // The device's slots, shared by its contexts and kept until the process ends (at most 32 MB pinned and
-// the two streams): memory, streams and first copies took 8 ms and taking them down 3 ms when a set had
+// the streams): memory, streams and first copies took 8 ms and taking them down 3 ms when a set had
 // eight streams, more than a transfer of 200 MB saves, and a program that opens a context per
 // evaluation paid it each time.
 Slots &slots_of(int device) {
