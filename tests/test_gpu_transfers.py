@@ -1,5 +1,5 @@
 """Copies between the caller's arrays and the device: one pass through the pinned buffer up to
-4 MiB; above it chunks of 2 MiB on one to several threads, into the device from 16 MiB and the
+4 MiB; above it chunks of 2 MiB on one to several threads, into the device from 8 MiB and the
 runtime's copies up to there.  56 bytes a particle go in, 104 come out."""
 import ctypes as C
 import threading
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 # one particle; the last sizes of the small path and the first past it, out and in; chunk ends inside
 # and between the arrays; the first size in chunks both ways; every thread busy
-SIZES = [1, 40329, 40330, 74898, 74899, 87381, 87382, 299593, 299594, 1200001]
+SIZES = [1, 40329, 40330, 74898, 74899, 87381, 87382, 149796, 149797, 1200001]
 
 
 def pinned(a):

@@ -139,7 +139,7 @@ assert F.fake_held(1) == 0
 
 
 def test_large_transfers_go_in_chunks(run):
-    """Into the device 16 MiB and more, out of it more than 4 MiB; the others are a copy per array."""
+    """Into the device 8 MiB and more, out of it more than 4 MiB; the others are a copy per array."""
     run(TRANSFERS + """
 def copies(f, *a):
     was = F.fake_done(ASYNC)
@@ -148,7 +148,7 @@ def copies(f, *a):
 with V.VPM(V.Params.make(0.125)) as c:
     # 56 bytes a particle go in (24 and 32 in two arrays), 104 come out (24, 32, 24 and 24 in four)
     chunks = lambda n, arrays: sum(-(-n * b // (2 << 20)) for b in arrays)
-    for n, large_in, large_out in ((40329, 0, 0), (40330, 0, 1), (70000, 0, 1), (200000, 0, 1), (299593, 0, 1), (299594, 1, 1)):
+    for n, large_in, large_out in ((40329, 0, 0), (40330, 0, 1), (70000, 0, 1), (149796, 0, 1), (149797, 1, 1), (300000, 1, 1)):
         assert copies(c.upload, *cloud(n)) == (chunks(n, (24, 32)) if large_in else 2), n
         assert copies(c.download) == (chunks(n, (24, 32, 24, 24)) if large_out else 4), n
 """)

@@ -107,8 +107,8 @@ int stretch_kernel(Ctx *c, const int n[3], const double h[3], GView rhs, GView v
 // -- the same values bit for bit, without writing the velocity grid and reading it back.  The
 // tile shape is a tuner choice (the halo's share against the x extent of the rows).  kc is 32
 // where that gives every CU two work-groups, and is halved down to 4 until it does: each plane
-// is one dependent step of some 2 us (a 41^3 grid in one chunk: 75 us on 11 work-groups), and
-// the three planes formed twice per chunk cost little there.
+// is one dependent step of some 2 us (49^3 nodes in chunks of 32: 75 us on 28 work-groups, of 4:
+// 17), and the three planes formed twice per chunk cost little there.
 constexpr int CS_KC = 32, CS_KC_MIN = 4;
 // Tiles go out XCD by XCD in contiguous slices of each round of R work-groups (xcd_slice; R
 // about the work-groups resident at once), so the tiles that share halo columns, and the

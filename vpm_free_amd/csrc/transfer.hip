@@ -5,13 +5,14 @@
 // call each waits for the host.  Here
 //   * up to SMALL_COPY bytes pass through the context's pinned buffer: one memcpy and one
 //     asynchronous copy per array;
-//   * into the device, from there to CHUNKED_IN bytes the runtime's copies are the fastest (MB: us,
-//     arrays used before / fresh ones; runtime, chunks): 4.5: 154 / 187, 179 / 214; 6: 195 / 241, 270 /
-//     326; 8: 251 / 304, 304 / 367; 12: 344 / 424, 386 / 415; 16: 450 / 568, 454 / 491; 24: 669 / 877,
-//     613 / 636; 48: 1634 / 1663, 1114 / 1182;
-//   * larger ones, and what comes out of the device, are cut into chunks that several threads move through pinned slots, each with a
-//     copy in flight while it touches the other slot's host side (the page faults of a fresh
-//     result array spread over the threads too).  The slots and the streams are one set per device,
+//   * into the device, from there to CHUNKED_IN bytes, where one thread would move the chunks, the
+//     runtime's copies are the fastest (MB: us, arrays used before / fresh ones; runtime, chunks): 4.5:
+//     154 / 187, 179 / 214; 6: 195 / 241, 270 / 326; 8: 251 / 304, 304 / 367; 10: 297 / 365, 293 / 319;
+//     12: 344 / 424, 386 / 415; 16: 450 / 568, 454 / 491; 24: 669 / 877, 613 / 636; 48: 1634 / 1663, 1114
+//     / 1182 (a call with 12 MB from arrays used in turn: 3.57 ms by the runtime, 3.50 in chunks);
+//   * larger ones, and what comes out of the device, are cut into chunks that several threads move
+//     through pinned slots, each with a copy in flight while it touches the other slot's host side
+//     (the page faults of a fresh result array spread over the threads too).  The slots and the streams are one set per device,
 //     used by one transfer at a time.  A stream's first copies cost about 5 ms each (a process' first
 //     84 MB in take 25 ms, 16 by the runtime, whose first 156 MB out take 16 against 4 here; the next
 //     one or two in 7 instead of 2, with eight streams the next five), and two streams are slower
@@ -41,7 +42,7 @@ namespace vpmx {
 
 namespace {
 
-constexpr size_t SMALL_COPY = 4 << 20, CHUNKED_IN = 16 << 20, CHUNK = 2 << 20, PER_THREAD = 4 << 20;
+constexpr size_t SMALL_COPY = 4 << 20, CHUNK = 2 << 20, PER_THREAD = 4 << 20, CHUNKED_IN = 2 * PER_THREAD;
 constexpr int MAX_THREADS = 8, STREAMS = 4;
 
 // The pinned slots (two per thread) and streams of one device.
